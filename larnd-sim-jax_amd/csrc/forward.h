@@ -11,20 +11,28 @@ namespace lsim {
 // bounds test (windows up to 3 * 63 - 2 = 187 samples).
 constexpr int kWinPad = 3 * kWave;
 constexpr int kXcd = 8;  // XCDs of an MI355X (workgroup i runs on XCD i % 8)
+constexpr int kNextPad = 32;  // one 128-byte line per band's slot counter (take_row)
 
-// Per-segment record of the window-store paths (sorted order, 32 bytes = one scalar load): window
-// start, charge, fractional tick, the interior-window flag, and byte offsets from which the
-// padded raw-window row of any neighbour offset follows with a few scalar operations.  For a
-// sub-bin position u and a pixel offset a != 0, offset_bin(u, a) = nsb a + nsb/2 - 1 - u (a > 0)
-// or u - nsb/2 + nsb |a| (a < 0): affine in u, so the row is a per-cell constant plus +-U.
-struct __align__(32) PairRec {
+// Raw-response windows as the stripe accumulation reads them: row (cx, cy) of `stripe_stride(L)` floats
+// holds kStripeLead zeros and then the L samples, and zeros follow up to the stride; the next row's
+// leading zeros serve as this row's tail.  The last of the leading zeros (sample -1) is kStripeMark:
+// the window's tick of the boundary correction, whose value depends on the segment and is put in
+// its place by the reader.  One more row, of zeros, follows the table.
+constexpr int kStripeLead = kWave;
+constexpr uint32_t kStripeMark = 0x7fa5c3e1u;
+__host__ __device__ inline int stripe_stride(int L) { return kStripeLead + (L > 2 * kWave ? L : 2 * kWave); }
+__host__ __device__ inline int64_t stripe_floats(int lx, int ly, int L) {
+  return ((int64_t)lx * ly + 1) * stripe_stride(L) + kWave;
+}
+
+// Per-segment record of the window paths (sorted order): window start, charge, fractional tick and
+// sub-bin position.
+struct __align__(16) PairRec {
   int S;          // first output tick of the (1-f) window: nt - L - k0
   float ne, f;
   int flags;      // bit 0: 2 <= S and S + L <= nout (interior window); bits 8-15: u; bits 16-23: v
-  int U, V;       // u * ly * kWinPad * 4 and v * kWinPad * 4
-  int U0, V0;     // offset_bin(u, 0) * ly * kWinPad * 4 and offset_bin(v, 0) * kWinPad * 4
 };
-static_assert(sizeof(PairRec) == 32, "PairRec layout");
+static_assert(sizeof(PairRec) == 16, "PairRec layout");
 
 // ------------------------------------------------------------------------------------------
 // small utility kernels
@@ -89,10 +97,10 @@ __global__ void k_cell_keys(Dev d, SegIn in, const uint32_t* __restrict__ vals, 
 // 2. records in cell order, cell ranges, pixel rows
 // ------------------------------------------------------------------------------------------
 
-// Boundary corrections of every (row offset, segment) pair of record R, written where the record
-// is built: dtot[ab][i] = n_e (D.x - f D.y) of the neighbour stripe (raw response, unless the offset
-// is (0, 0)) plus, for |a|, |b| <= 1, the sum over the diffusion bins landing on that row of
-// n_bin (D.x - f D.y) of the idx template (sim_jax.py:227-261), D = (C[nt-L] - C[k0],
+// Boundary corrections of every (row offset, segment) pair of record R per unit charge, written where
+// the record is built: dtot[ab][i] = D.x - f D.y of the neighbour stripe (raw response, unless the
+// offset is (0, 0)) plus, for |a|, |b| <= 1, the sum over the diffusion bins landing on that row of
+// w_bin (D.x - f D.y) of the idx template (sim_jax.py:227-261), D = (C[nt-L] - C[k0],
 // C[k0+1] - C[k0]), ab = (a + n)(2n + 1) + (b + n).  The D tables are tick-major, so all of one
 // segment's entries lie in the tick-k0 plane; the waveform kernels then read dtot[ab][cell range]
 // contiguously.
@@ -149,7 +157,7 @@ __device__ __forceinline__ void seg_corrections(const Dev& d, const float2* __re
       const int ab = ab0 + u;
       const int a = ab / W - d.ne, b = ab % W - d.ne;
       const bool on = ab < WW && (a != 0 || b != 0) && a >= -d.nn && a <= d.nn && b >= -d.nn && b <= d.nn;
-      dl[u] = on ? R.ne * (D[u].x - f * D[u].y) : 0.f;
+      dl[u] = on ? D[u].x - f * D[u].y : 0.f;
     }
 #pragma unroll
     for (int u = 0; u < kCorrBatch; ++u) {
@@ -173,7 +181,7 @@ __device__ __forceinline__ void seg_corrections(const Dev& d, const float2* __re
   for (int k = 0; k < NB; ++k) {
     const int vx = ux + k - SYM;
     const int dx = vx < 0 ? -1 : (vx >= nsb ? 1 : 0);
-    const float wxs = R.ne * R.wx[k];
+    const float wxs = R.wx[k];
     const int cx = offset_bin(vx - dx * nsb, 0, nsb);
     float2 D[NB];
     float c[NB];
@@ -233,10 +241,6 @@ __device__ __forceinline__ void record(const Dev& d, const SegIn& in, int64_t sr
   P.ne = r.ne;
   P.f = r.f;
   P.flags = ((P.S >= 2 && P.S + d.L <= d.nout) ? 1 : 0) | (ux << 8) | (uy << 16);
-  P.U = ux * d.ly * kWinPad * 4;
-  P.V = uy * kWinPad * 4;
-  P.U0 = offset_bin(ux, 0, d.nsb) * d.ly * kWinPad * 4;
-  P.V0 = offset_bin(uy, 0, d.nsb) * kWinPad * 4;
   prs[i] = P;
 }
 
@@ -304,8 +308,10 @@ __global__ void k_copy_count(const int* __restrict__ src, int64_t* __restrict__ 
 struct Tables {
   const float3* TM3;  // [nm][cm][cm][kWinPad] padded (T_{m-1}, T_m, T_{m+1}) windows of the diffusion bins
   const float* TM;    // [nm][cm][cm][L]   main-bin template windows
+  const float* TMW;   // [cm][cm][nm][bin_stride(L)] the same, two zeros before each window (and after the last)
   const float* TN;    // [lx][ly][L]       raw response window (neighbours)
   const float* TNP;   // [lx][ly][kWinPad] the same, padded
+  const float* TNQ;   // the same as stripe_floats() values (kStripeMark in each row's sample -1)
   const float2* DM;   // [nt][nm][cm][cm]  (C[nt-L]-C[k], C[min(k+1,nt-1)]-C[k]) of template m (tick-major)
   const float2* DN;   // [nt][lx][ly]      same for the raw response
   const double* CTM;  // [nm][cm][cm][L+1] window prefix sums (adjoint)
@@ -346,99 +352,73 @@ __device__ __forceinline__ T wave_sum(T v) {
   return v;
 }
 
-__device__ __forceinline__ int wave_min_i(int v) {
-#pragma unroll
-  for (int m = kWave / 2; m >= 1; m >>= 1) {
-    int u = __shfl_xor(v, m, kWave);
-    v = u < v ? u : v;
-  }
-  return v;
-}
-
 // Self-trigger of one row (fee_jax.py:168-279, noise off), then digitisation (fee_jax.py:55-71).
 // The float64 cumulative charge Q stays in registers: thread t holds ticks t * TPER + u in q[u]
 // (as finish_row leaves them) and takes the tick after its last one from the next lane (DPP, or
-// LDS across waves once, then updated by the same resets).  Q0 (LDS, written only with a tape)
-// is the unreset copy.  The passes' decisions go to LDS from the threads that own the ticks;
-// wave 0 then writes the outputs and the tape with one lane per pass (and one lane per tape point
-// for the clamp masks).
+// LDS across waves once, then updated by the same resets).  Q0 (LDS) is the unreset copy: what pass k
+// needs of a single tick (the window's end, the reset point) every thread takes from there and
+// puts through the k resets itself, so a pass has one barrier, for its crossing, and none for its
+// charges (two barriers, and 64-bit maxima by lane shuffles where ballots do, took 4.0 of the 30 ms of
+// a 160k-row launch; 2.1 with ballots).  Wave 0 then writes the outputs and the tape with one lane per
+// pass (and one lane per tape point for the clamp masks).
 template <int NT>
 __device__ void fee_row(const Dev& d, double (&q)[kMaxOut / NT], const double* Q0, int r, int plane,
-                        const RowOut& out, int* sh_int) {
+                        const RowOut& out, int (*sh_int)[NT / kWave]) {
   constexpr int TPER = kMaxOut / NT;
   constexpr int NW = NT / kWave;
   __shared__ int s_pe[kMaxH], s_pg[kMaxH], s_pi[kMaxH];
   __shared__ double s_pa[kMaxH];
-  __shared__ double s_qmax[NW], s_first[NW];
-  __shared__ double s_qg, s_gnone;
+  __shared__ double s_reset[kMaxH];  // Q[g] of each pass (written before the next pass's barrier)
+  __shared__ double s_first[NW];
   const int t = threadIdx.x;
   const int nout = d.nout;
   const int lane = t & (kWave - 1), wid = t / kWave;
   const int H = d.H;
   const int o0 = t * TPER;
-  // Q[o] into v when this thread holds tick o (register indices fixed at compile time)
-  auto held = [&](int o, double& v) {
-    bool own = false;
-#pragma unroll
-    for (int u = 0; u < TPER; ++u)
-      if (o0 + u == o) {
-        v = q[u];
-        own = true;
-      }
-    return own;
-  };
   // reset index of a pass without a crossing (i* = nout - 2), and its window end
   int g_none = nout - 2 + 1 + d.interval + 1;
   if (g_none >= nout) g_none = nout - 1;
   int e_none = nout - 2 + 1 + d.interval;
   if (e_none >= nout) e_none = nout - 1;
   if (lane == 0) s_first[wid] = q[0];
-  {
-    double v;
-    if (held(g_none, v)) s_gnone = v;
-  }
-  __syncthreads();
+  __syncthreads();  // also: Q0 is complete
   double nx = __shfl_down(q[0], 1, kWave);  // Q[o0 + TPER]
   if (lane == kWave - 1) nx = wid + 1 < NW ? s_first[wid + 1] : 0.0;
-  const double q_gnone = s_gnone;
+  const double q_gnone = Q0[g_none];
+  auto reset_by = [](double v, double c) {
+    const double x = v - c;
+    return x < 0 ? 0.0 : x;
+  };
+  // A wave's first crossing: lanes hold ticks in order, so the first lane with one has it.  kAbove: no
+  // crossing, but some Q[1 .. nout-1] at or above thr; kBelow: none (what a crossing needs).
+  constexpr int kBelow = 0x7fffffff, kAbove = kBelow - 1;
   for (int k = 0; k < H; ++k) {
-    int cand = 0x7fffffff;
-    double qmax = -1.0e300;  // max of Q[1 .. nout-1], the values a crossing needs at or above thr
+    int cand = kBelow;
+    bool above = false;
 #pragma unroll
-    for (int u = 0; u < TPER; ++u) {
+    for (int u = TPER - 1; u >= 0; --u) {
       const int o = o0 + u;
-      if (o <= nout - 2) {
-        const double q1 = u + 1 < TPER ? q[u + 1] : nx;
-        if (q1 >= d.thr && q[u] <= d.thr && o < cand) cand = o;
-        qmax = q1 > qmax ? q1 : qmax;
-      }
+      const double q1 = u + 1 < TPER ? q[u + 1] : nx;
+      const bool up = o <= nout - 2 && q1 >= d.thr;
+      above = above || up;
+      if (up && q[u] <= d.thr) cand = o;
     }
-    cand = wave_min_i(cand);
-#pragma unroll
-    for (int m = kWave / 2; m >= 1; m >>= 1) {
-      const double v = __shfl_xor(qmax, m, kWave);
-      qmax = v > qmax ? v : qmax;
-    }
-    if (lane == 0) {
-      sh_int[wid] = cand;
-      s_qmax[wid] = qmax;
-    }
-    __syncthreads();
-    int istar = 0x7fffffff;
-    double bmax = -1.0e300;
-    for (int w = 0; w < NW; ++w) {
-      istar = sh_int[w] < istar ? sh_int[w] : istar;
-      bmax = s_qmax[w] > bmax ? s_qmax[w] : bmax;
-    }
-    if (bmax < d.thr && (k > 0 || q_gnone >= 0.0)) {
+    const uint64_t mc = __ballot(cand != kBelow), ma = __ballot(above);
+    const int first = __builtin_amdgcn_readlane(cand, mc ? __builtin_ctzll(mc) : 0);
+    if (lane == 0) sh_int[k & 1][wid] = mc ? first : (ma ? kAbove : kBelow);
+    __syncthreads();  // (pass k + 1 writes the other row, pass k + 2 after the next barrier)
+    int istar = kBelow;
+    for (int w = 0; w < NW; ++w) istar = sh_int[k & 1][w] < istar ? sh_int[k & 1][w] : istar;
+    if (istar == kBelow && (k > 0 || q_gnone >= 0.0)) {
       // Nothing reaches the threshold: no crossing in this pass, and none later either.  A reset
       // Q <- max(Q - Q[g], 0) with Q[g] >= 0 never raises a value above max(Q, 0) < thr.  After
       // the first pass Q >= 0 everywhere, so Q[g] >= 0; in the first pass (the raw cumulative
       // charge may be negative) it is checked.  Every remaining pass ends at i* = nout-2 (no hit)
       // with e and g at their clamps, exactly as running it would; Q is not read again (the tape
       // follows Q0).
-      double v;
-      if (held(e_none, v)) {
+      if (t == 0) {
+        double v = Q0[e_none];
+        for (int p = 0; p < k; ++p) v = reset_by(v, s_reset[p]);
         for (int kk = k; kk < H; ++kk) {
           s_pe[kk] = e_none;
           s_pg[kk] = g_none;
@@ -446,36 +426,32 @@ __device__ void fee_row(const Dev& d, double (&q)[kMaxOut / NT], const double* Q
           s_pa[kk] = v;
         }
       }
-      __syncthreads();
       break;
     }
-    if (istar == 0x7fffffff) istar = nout - 2;
+    if (istar >= kAbove) istar = nout - 2;
     int e = istar + 1 + d.interval;
     if (e >= nout) e = nout - 1;
     int g = istar + 1 + d.interval + 1;
     if (g >= nout) g = nout - 1;
-    {
-      double v;
-      if (held(e, v)) {
-        s_pe[k] = e;
-        s_pg[k] = g;
-        s_pi[k] = istar;
-        s_pa[k] = v;
-      }
-      if (held(g, v)) s_qg = v;
+    double Qg = Q0[g], Qe = Q0[e];
+    for (int p = 0; p < k; ++p) {
+      const double c = s_reset[p];
+      Qg = reset_by(Qg, c);
+      Qe = reset_by(Qe, c);
     }
-    __syncthreads();
-    const double Qg = s_qg;
+    if (t == 0) {
+      s_pe[k] = e;
+      s_pg[k] = g;
+      s_pi[k] = istar;
+      s_pa[k] = Qe;
+      s_reset[k] = Qg;
+    }
 #pragma unroll
-    for (int u = 0; u < TPER; ++u) {
-      if (o0 + u < nout) {
-        const double x = q[u] - Qg;
-        q[u] = x < 0 ? 0.0 : x;
-      }
-    }
-    const double x = nx - Qg;  // the next thread's first tick, reset as its owner resets it
-    nx = x < 0 ? 0.0 : x;
+    for (int u = 0; u < TPER; ++u)
+      if (o0 + u < nout) q[u] = reset_by(q[u], Qg);
+    nx = reset_by(nx, Qg);  // the next thread's first tick, reset as its owner resets it
   }
+  __syncthreads();
   if (t >= kWave) return;
   // lane k < H: pass k's hit
   bool hit = false;
@@ -519,7 +495,7 @@ __device__ void fee_row(const Dev& d, double (&q)[kMaxOut / NT], const double* Q
 }
 
 // Sum of the per-wave partial rows, waveform store, float64 cumulative charge: thread t holds
-// Q[t * TPER + u] in q[u] (consecutive ticks per thread); with a tape Q0 receives a copy in LDS.
+// Q[t * TPER + u] in q[u] (consecutive ticks per thread); Q0 receives a copy in LDS.
 template <int NT>
 __device__ void finish_row(const Dev& d, const float* acc, int nwaves, int rstride, double (&q)[kMaxOut / NT],
                            double* Q0, int r, const RowOut& out, double* shd) {
@@ -550,76 +526,25 @@ __device__ void finish_row(const Dev& d, const float* acc, int nwaves, int rstri
 #pragma unroll
   for (int u = 0; u < TPER; ++u) q[u] = ex + loc[u];
   // the scan's barriers follow every read of the partial rows, which Q0 may now overwrite
-  if (out.tape) {
 #pragma unroll
-    for (int u = 0; u < TPER; ++u) {
-      const int o = t * TPER + u;
-      if (o < d.nout) Q0[o] = q[u];
-    }
+  for (int u = 0; u < TPER; ++u) {
+    const int o = t * TPER + u;
+    if (o < d.nout) Q0[o] = q[u];
   }
 }
 
 // Contributions of one segment to one pixel row.  The segment's stripes landing on the row share
 // one time window: V[j] = sum over stripes n_st * X_st[j], j < L, placed as (1-f) V at output
 // tick S+j and f V at S-1+j (S = nt - L - k0), plus the cumsum boundary correction Delta at
-// output ticks S-1 ((1-f) Delta) and S-2 (f Delta) (sim_jax.py:170-261).  Lane l of chunk c
-// owns output offset m = 63*c + l - 2 and holds V[m]; V[m+1] comes from lane l+1.  Window ticks
-// are kept for 1 <= o <= nout-1, corrections for 0 <= o <= nout-2 (the reference's garbage
-// column takes the rest).  Every per-pair quantity is wave uniform (scalar registers).
+// output ticks S-1 ((1-f) Delta) and S-2 (f Delta) (sim_jax.py:170-261).  Window ticks are kept for
+// 1 <= o <= nout-1, corrections for 0 <= o <= nout-2 (the reference's garbage column takes the
+// rest).
+//
+// kChunk: window samples per load of the adjoint's wave-wide reads (lane 63 supplies lane 62's next one).
 constexpr int kChunk = kWave - 1;
-// Slack after each wave's partial row for the interior store: a window at S (2 <= S, S + L <= nout)
-// is stored as three chunks of 63 lanes from index S - 2, so it writes up to S + 3 * 63 - 3 <=
-// nout - L + 186.
-__host__ __device__ inline int row_pad(int L) { return L < 3 * kChunk - 2 ? 3 * kChunk - 2 - L : 0; }
-
-// lane i receives lane i+1's value (lane 63 receives 0): DPP wavefront shift, no LDS traffic
-__device__ __forceinline__ float lane_next(float v) {
-  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x130 /* wave_shl:1 */, 0xf, 0xf, false));
-}
-
-// General store of one chunk with every bound checked (segments whose window reaches the ends).
-__device__ __forceinline__ void scatter_chunk(float* accw, int lane, int m, float v, float vn, float omf, float f,
-                                              float delta, int S, int L, int nout) {
-  const int o = S + m;
-  if (lane < kChunk && m < L && o >= 0 && o < nout) {
-    float val = 0.f;
-    if (o >= 1) val = omf * v + f * vn;
-    if (o <= nout - 2) {
-      if (m == -1) val += omf * delta;
-      if (m == -2) val += f * delta;
-    }
-    accw[o] += val;
-  }
-}
-
-// Store of a whole window held as three chunks (v0, v1, v2) of up to 63 outputs each, V = v
-// scaled by the charge: ne_omf = scale*(1-f), ne_f = scale*f.  `interior` windows (the caller
-// passes 2 <= S and S + L <= nout) need no per-lane tick checks: output m of chunk c goes to
-// accw[S + m] with m = 63 c + lane - 2.
-__device__ __forceinline__ void store_window(float* accw, int lane, float v0, float v1, float v2, float scale, float omf,
-                                             float f, float delta, int S, int L, int nout, bool interior) {
-  const float n0 = lane_next(v0), n1 = lane_next(v1), n2 = lane_next(v2);
-  if (interior) {
-    // all three chunks in one go (disjoint addresses); lanes past the window add +0 to the
-    // row or to the row_pad slack after it, so no per-chunk branch is needed
-    const float so = scale * omf, sf = scale * f;
-    float* p = accw + (S - 2) + lane;
-    float c0 = so * v0 + sf * n0;
-    c0 += (lane == 0) ? f * delta : ((lane == 1) ? omf * delta : 0.f);
-    const float c1 = (lane + kChunk - 2 < L) ? so * v1 + sf * n1 : 0.f;
-    const float c2 = (lane + 2 * kChunk - 2 < L) ? so * v2 + sf * n2 : 0.f;
-    if (lane < kChunk) {
-      const float a0 = p[0], a1 = p[kChunk], a2 = p[2 * kChunk];
-      p[0] = a0 + c0;
-      p[kChunk] = a1 + c1;
-      p[2 * kChunk] = a2 + c2;
-    }
-  } else {
-    scatter_chunk(accw, lane, lane - 2, scale * v0, scale * n0, omf, f, delta, S, L, nout);
-    scatter_chunk(accw, lane, lane - 2 + kChunk, scale * v1, scale * n1, omf, f, delta, S, L, nout);
-    scatter_chunk(accw, lane, lane - 2 + 2 * kChunk, scale * v2, scale * n2, omf, f, delta, S, L, nout);
-  }
-}
+// Slack after each wave's partial row: an interior window (2 <= S, S + L <= nout) is stored three ticks
+// per lane from S - 2 while 3 lane < L + 2, so it writes up to S + L + 1.
+__host__ __device__ inline int row_pad(int) { return 4; }
 
 // lane i receives lane i+1's value, lane 63 receives 0 (DPP wave shift; bound_ctrl supplies the
 // zero, so no register needs clearing first)
@@ -627,39 +552,33 @@ __device__ __forceinline__ float lane_next0(float v) {
   return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0x130 /* wave_shl:1 */, 0xf, 0xf, true));
 }
 
-// Store of a neighbour-stripe window with the pair's factors precomputed: so = n_e (1-f),
-// sf = n_e f, fD = f Delta, omfD = (1-f) Delta.  v0..v2 come from a padded table row (zero past the
-// window), so interior stores need no mask beyond lane < 63.  base = this wave's partial row - 2.
-// m0, m1: 1 on lane 0 (resp. 1), else 0; fD m0 + omfD m1 is exactly the correction of the lane.
-__device__ __forceinline__ void store_stripe(float* base, int lane, float m0, float m1, float v0, float v1, float v2,
-                                             float so, float sf, float fD, float omfD, int S, int L, int nout,
-                                             bool interior) {
-  const float n0 = lane_next0(v0), n1 = lane_next0(v1), n2 = lane_next0(v2);
+// Store of a whole window V held three samples per lane: lane l holds V[3 l - 2 + k] in vk, zero outside
+// 0 <= m < L, for 3 l < L + 2.  Output m receives (1-f) V[m] + f V[m+1]; delta is the boundary correction.
+// `interior` windows (2 <= S and S + L <= nout) need no tick checks.
+__device__ __forceinline__ void store_window(float* accw, int lane, float v0, float v1, float v2, float omf, float f,
+                                             float delta, int S, int L, int nout, bool interior) {
+  const float nx = lane_next0(v0);
+  const int m = 3 * lane - 2;
+  float c0 = omf * v0 + f * v1, c1 = omf * v1 + f * v2, c2 = omf * v2 + f * nx;
   if (interior) {
-    float* p = base + S + lane;
-    float c0 = so * v0 + sf * n0;
-    c0 += fD * m0 + omfD * m1;
-    const float c1 = so * v1 + sf * n1;
-    const float c2 = so * v2 + sf * n2;
-    if (lane < kChunk) {
-      const float a0 = p[0], a1 = p[kChunk], a2 = p[2 * kChunk];
+    c0 += lane == 0 ? f * delta : 0.f;
+    c1 += lane == 0 ? omf * delta : 0.f;
+    if (m < L) {
+      float* p = accw + S + m;
+      const float a0 = p[0], a1 = p[1], a2 = p[2];
       p[0] = a0 + c0;
-      p[kChunk] = a1 + c1;
-      p[2 * kChunk] = a2 + c2;
+      p[1] = a1 + (m + 1 < L ? c1 : 0.f);
+      p[2] = a2 + (m + 2 < L ? c2 : 0.f);
     }
   } else {
-    float* accw = base + 2;
 #pragma unroll
-    for (int c = 0; c < 3; ++c) {
-      const float v = c == 0 ? v0 : (c == 1 ? v1 : v2), vn = c == 0 ? n0 : (c == 1 ? n1 : n2);
-      const int m = lane - 2 + c * kChunk;
-      const int o = S + m;
-      if (lane < kChunk && m < L && o >= 0 && o < nout) {
-        float val = 0.f;
-        if (o >= 1) val = so * v + sf * vn;
+    for (int k = 0; k < 3; ++k) {
+      const int o = S + m + k;
+      if (m + k < L && o >= 0 && o < nout) {
+        float val = o >= 1 ? (k == 0 ? c0 : (k == 1 ? c1 : c2)) : 0.f;
         if (o <= nout - 2) {
-          if (m == -1) val += omfD;
-          if (m == -2) val += fD;
+          if (m + k == -1) val += omf * delta;
+          if (m + k == -2) val += f * delta;
         }
         accw[o] += val;
       }
@@ -667,24 +586,105 @@ __device__ __forceinline__ void store_stripe(float* base, int lane, float m0, fl
   }
 }
 
-// Window values of one pair (and, for the centre pairs, the pair's correction): the loads of a
-// group of pairs are issued before any of their stores, so a wave keeps several independent pairs
-// in flight.
-struct FarLoads {
-  float t0, t1, t2;
-  float D;  // boundary correction Delta of the pair (charge included)
+// 0x00020000: word 3 of a raw (stride 0) buffer descriptor on gfx9-family GPUs.
+constexpr int kBufDesc3 = 0x00020000;
+
+// ---- neighbour stripes of one row: pairs sorted by time chunk, accumulated chunk by chunk ----
+//
+// Output tick o of the row receives, from every pair, (1-f) n_e V[o - S] + f n_e V[o - S + 1], V the raw
+// window with the unit-charge boundary correction as its sample -1.  With
+//   A0[o] = sum so V[o - S],  A1[o] = sum sf V[o - S],  so = n_e (1-f), sf = n_e f,
+// the row is A0[o] + A1[o + 1], so a lane that owns tick o needs one sample of each pair: no
+// lane shift per pair and no read-modify-write of LDS per pair, which a wave that owns the pair needs.
+// Ticks are cut into chunks of 64 (position o + kTickOff, chunk position / 64); a pair whose first
+// position S - 1 lies in chunk b reaches chunks b .. b + 2, and b + 3 when it starts late enough in b
+// (r = position % 64 >= 192 - L).  The pairs of a batch are therefore counting-sorted in LDS by
+// 2 b + (reaches b + 3): those of chunk c are one contiguous run, the last part of it (b = c) holding
+// the samples -1.
+//
+// Per (pair, chunk): one 4-byte LDS read (lane l takes word l % 4 of the 16-byte entry; each word
+// reaches its use by a quad broadcast folded into the instruction), one 256-byte window load from L2 or
+// L1, an address add and two multiply-adds.
+constexpr int kTickOff = 3 * kWave;                         // S >= 1 - L > -kTickOff
+constexpr int kRowChunks = kMaxOut / kWave + 1;             // output chunks of the longest row, and tick nout of A1
+constexpr int kStripeKeys = 2 * (kRowChunks + 3);           // 2 b + late, b < kRowChunks + 3
+constexpr int kKeyOdd = kStripeKeys;                        // non-finite factors (handled tick by tick)
+constexpr int kKeyNone = kStripeKeys + 1;                   // not listed (no charge, or past the row)
+constexpr int kStripeRounds = 6;                            // pairs per lane and batch
+static_assert((kStripeKeys & 1) == 0 && kStripeKeys / 2 + 1 <= kWave, "one lane per pair of keys");
+
+struct __align__(16) StripeEnt {
+  int addr;       // byte offset into TNQ at position 0: 4 (row stride + kStripeLead - kTickOff - S)
+  float so, sf;   // n_e (1 - f), n_e f
+  float D;        // boundary correction per unit charge (kKeyOdd: S)
 };
 
-// Neighbour-stripe window loads through a buffer descriptor of the padded raw-window table: the
-// pair's byte offset goes in the scalar offset field and the lane's in the vector one, so there
-// is no per-pair address arithmetic.  0x00020000: word 3 of a raw (stride 0) buffer descriptor on
-// gfx9-family GPUs.
-constexpr int kBufDesc3 = 0x00020000;
-__device__ __forceinline__ void far_load_buf(__amdgpu_buffer_rsrc_t r, int lane4, int off, FarLoads& q) {
-  q.D = 0.f;
-  q.t0 = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, lane4, off, 0));
-  q.t1 = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, lane4 + 4 * kChunk, off, 0));
-  q.t2 = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, lane4 + 8 * kChunk, off, 0));
+template <int K>
+__device__ __forceinline__ int quad_word(int v) {  // word K of the lane's quad in every lane of it
+  return __builtin_amdgcn_mov_dpp(v, K * 0x55, 0xf, 0xf, true);
+}
+
+// N entries at ent (lane l's word): their shares of the lane's position (pos4 = 4 * position).  HEAD:
+// chunks that may hold a pair's sample -1.  n < N: the entries from n on repeat entry n - 1 with no
+// charge.  Four sums of each kind, so that a sum's float32 rounding is that of a chain a quarter as long (the
+// rows' error against float64 is that of per-wave partial rows: 7e-8 of their norm).
+constexpr int kStripeSums = 4;
+struct StripeSums {
+  float a0[kStripeSums] = {}, a1[kStripeSums] = {};
+};
+
+template <int N, bool HEAD>
+__device__ __forceinline__ void stripe_group(__amdgpu_buffer_rsrc_t tnq, const int* ent, int n, bool is_addr, int pos4,
+                                             StripeSums& A) {
+  int w[N];
+#pragma unroll
+  for (int g = 0; g < N; ++g) {
+    w[g] = ent[4 * (g < n ? g : n - 1)];
+    if (g >= n && !is_addr) w[g] = 0;
+  }
+  int v[N];
+#pragma unroll
+  for (int g = 0; g < N; ++g) v[g] = __builtin_amdgcn_raw_buffer_load_b32(tnq, pos4 + quad_word<0>(w[g]), 0, 0);
+#pragma unroll
+  for (int g = 0; g < N; ++g) {
+    if (HEAD) {
+      const int corr = quad_word<3>(w[g]);  // taken by every lane: a lane reads its quad, active or not
+      v[g] = v[g] == (int)kStripeMark ? corr : v[g];
+    }
+    float &a0 = A.a0[g % kStripeSums], &a1 = A.a1[g % kStripeSums];
+    a0 = __builtin_fmaf(__int_as_float(quad_word<1>(w[g])), __int_as_float(v[g]), a0);
+    a1 = __builtin_fmaf(__int_as_float(quad_word<2>(w[g])), __int_as_float(v[g]), a1);
+  }
+}
+
+template <bool HEAD>
+__device__ __forceinline__ void stripe_run(__amdgpu_buffer_rsrc_t tnq, const StripeEnt* list, int e, int e1, int lane,
+                                           int pos4, StripeSums& A) {
+  const int* ent = reinterpret_cast<const int*>(list) + (lane & 3);
+  const bool is_addr = (lane & 3) == 0;
+  for (; e1 - e >= 16; e += 16) stripe_group<16, HEAD>(tnq, ent + 4 * e, 16, is_addr, pos4, A);
+  if (e1 - e >= 8) {
+    stripe_group<8, HEAD>(tnq, ent + 4 * e, 8, is_addr, pos4, A);
+    e += 8;
+  }
+  if (e1 - e >= 4) {
+    stripe_group<4, HEAD>(tnq, ent + 4 * e, 4, is_addr, pos4, A);
+    e += 4;
+  }
+  if (e < e1) stripe_group<4, HEAD>(tnq, ent + 4 * e, e1 - e, is_addr, pos4, A);
+}
+
+// A pair with a non-finite factor at output tick o: what storing its whole padded window leaves there
+// (a non-finite charge times the padding's zeros is NaN from S - 2 to S + 186 of an interior window).
+__device__ __forceinline__ float odd_pair(const float* __restrict__ TNQ, const StripeEnt& E, int o, int L, int nout) {
+  const int S = __float_as_int(E.D), m = o - S;
+  const bool interior = S >= 2 && S + L <= nout;
+  if (m < -2 || m > (interior ? 3 * (kWave - 1) - 3 : L - 1)) return 0.f;
+  const float* T = TNQ + E.addr + kStripeLead;
+  const float v = m >= 0 && m < L ? T[m] : 0.f, vn = m + 1 >= 0 && m + 1 < L ? T[m + 1] : 0.f;
+  float val = interior || o >= 1 ? E.so * v + E.sf * vn : 0.f;
+  if (interior ? m <= kWave - 4 : (m < 0 && o <= nout - 2)) val += 0.f * (E.so + E.sf);
+  return val;
 }
 
 // Distinct LUT cells of a segment's diffusion bins that land on pixel offset a along one axis, with
@@ -732,46 +732,72 @@ __device__ __forceinline__ bool bins_reach(int u, int a, int nsb) {
   return a == 0 ? true : (a > 0 ? u + (NB - 1 - SYM) >= nsb : u - SYM < 0);
 }
 
-// Window of the diffusion bins of segment R that land on the pixel (a, b) from its main pixel
-// (|a|, |b| <= 1), charge included: V[j] = sum_bins n_bin * (lb T_idx + la T_{idx-1} +
-// lc T_{idx+1})[cx][cy][j] (sim_jax.py:186-194), at the padded positions lane + 63 k (the chunks of
-// store_window), each distinct LUT cell once.  Bin i of the segment lies floor((u + i - SYM) / nsb)
-// in {-1, 0, 1} pixels from the main pixel.
+// Window of one segment's diffusion bins that land on one pixel: V[m] = sum_bins n_bin * (la T_{idx-1} +
+// lb T_idx + lc T_{idx+1})[cx][cy][m] (sim_jax.py:186-194), three samples per lane as store_window takes
+// them, each distinct LUT cell once.  `st` holds the merged bins of the two axes, NB each: weights along
+// x (charge included) and y, byte offsets of the cells in TMW along x and y.  Lane i NB + j forms the
+// product of bin i along x and bin j along y; the wave then walks the non-zero ones, four at a time:
+// weight and offset by a lane read, nine multiply-adds, and the three templates' rows (neighbours in TMW)
+// by one 12-byte load per lane each.  TMW (1.5 MB for 100 templates of 150 samples) stays in each XCD's L2.
+// lane12: 12 * lane for the lanes that hold samples, past the table for the others (they read 0).
+__host__ __device__ inline int bin_stride(int L) { return L + 2; }
+__host__ __device__ inline int64_t bin_floats(int nm, int cm, int L) { return (int64_t)nm * cm * cm * bin_stride(L) + 4; }
+constexpr int kBinItems = 16;  // items whose merged bins a wave stages at a time
+
 template <int NB>
-__device__ __forceinline__ void pixel_bins(const Dev& d, const Tables& tb, const SegRec& R, int a, int b, int lane,
-                                           float& v0, float& v1, float& v2) {
-  const int nsb = d.nsb, cm = d.cm;
-  const int ux = R.uxy & 0xffff, uy = R.uxy >> 16;
-  bool okx[NB], oky[NB];
-  int cxs[NB], cys[NB];
-  float WX[NB], WY[NB];
-  axis_merge<NB>(ux, a, nsb, R.wx, R.ne, okx, cxs, WX);
-  axis_merge<NB>(uy, b, nsb, R.wy, 1.f, oky, cys, WY);
-  const float la = R.la, lb = R.lb, lc = R.lc;
-  const float3* T3 = tb.TM3 + (int64_t)R.idx * cm * cm * kWinPad + lane;
-  v0 = v1 = v2 = 0.f;
+__device__ __forceinline__ void bins_window(__amdgpu_buffer_rsrc_t tmw, const float* st, int base, int ws4, int lane,
+                                            int lane12, float la, float lb, float lc, float& v0, float& v1, float& v2) {
+  float c = 0.f;
+  int off = 0;
+  if (lane < NB * NB) {
+    const int i = lane / NB, j = lane - i * NB;
+    c = st[i] * st[NB + j];
+    off = base + __float_as_int(st[2 * NB + i]) + __float_as_int(st[3 * NB + j]);
+  }
+  float A[3] = {0.f, 0.f, 0.f}, B[3] = {0.f, 0.f, 0.f}, C[3] = {0.f, 0.f, 0.f};
+  for (uint64_t m = __ballot(c != 0.f); m != 0;) {
+    constexpr int G = 4;
+    float w[G];
+    typedef float f32x3 __attribute__((ext_vector_type(3)));
+    f32x3 qa[G], qb[G], qc[G];
+    int bit = 0;
 #pragma unroll
-  for (int i = 0; i < NB; ++i) {
-    if (!okx[i]) continue;
+    for (int g = 0; g < G; ++g) {
+      const bool on = m != 0;  // past the last one: its row again with no weight
+      bit = on ? __builtin_ctzll(m) : bit;
+      m &= m - 1;
+      const float wg = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(c), bit));
+      w[g] = on ? wg : 0.f;
+      const int o = __builtin_amdgcn_readlane(off, bit);
+      qa[g] = __builtin_bit_cast(f32x3, __builtin_amdgcn_raw_buffer_load_b96(tmw, lane12, o, 0));
+      qb[g] = __builtin_bit_cast(f32x3, __builtin_amdgcn_raw_buffer_load_b96(tmw, lane12, o + ws4, 0));
+      qc[g] = __builtin_bit_cast(f32x3, __builtin_amdgcn_raw_buffer_load_b96(tmw, lane12, o + 2 * ws4, 0));
+    }
 #pragma unroll
-    for (int jj = 0; jj < NB; ++jj) {
-      if (!oky[jj]) continue;
-      const float c = WX[i] * WY[jj];
-      const float3* tp = T3 + ((int64_t)cxs[i] * cm + cys[jj]) * kWinPad;
-      const float3 q0 = tp[0], q1 = tp[kChunk], q2 = tp[2 * kChunk];
-      v0 += c * (q0.y * lb + q0.x * la + q0.z * lc);
-      v1 += c * (q1.y * lb + q1.x * la + q1.z * lc);
-      v2 += c * (q2.y * lb + q2.x * la + q2.z * lc);
+    for (int g = 0; g < G; ++g) {
+#pragma unroll
+      for (int k = 0; k < 3; ++k) {
+        A[k] = __builtin_fmaf(w[g], qa[g][k], A[k]);
+        B[k] = __builtin_fmaf(w[g], qb[g][k], B[k]);
+        C[k] = __builtin_fmaf(w[g], qc[g][k], C[k]);
+      }
     }
   }
+  v0 = lb * B[0] + la * A[0] + lc * C[0];
+  v1 = lb * B[1] + la * A[1] + lc * C[1];
+  v2 = lb * B[2] + la * A[2] + lc * C[2];
 }
 
-// Dynamic LDS of the waveform kernel: the per-wave partial rows (reused afterwards for the unreset
-// float64 cumulative charge of the tape), then the neighbourhood's cell lists (ncell begins, ncell + 1
-// cumulative counts, ncell offsets).
+// Dynamic LDS of the waveform kernel: the per-wave partial rows (the stripe list lies over rows 1 and up
+// first; afterwards the rows are reused for the unreset float64 cumulative charge of the tape), then
+// the neighbourhood's cell lists (ncell begins, ncell + 1 cumulative counts, ncell offsets).
+__host__ __device__ inline int stripe_batch(int waves) { return kStripeRounds * kWave * waves; }
+__host__ __device__ inline size_t rows_list_off(int nout, int L) { return ((size_t)(nout + row_pad(L)) * 4 + 15) & ~(size_t)15; }
 __host__ __device__ inline size_t rows_acc_bytes(int waves, int nout, int L) {
   const size_t acc = (size_t)waves * (nout + row_pad(L)) * 4, q = (size_t)nout * 8;
-  return ((acc > q ? acc : q) + 15) & ~(size_t)15;
+  const size_t list = rows_list_off(nout, L) + (size_t)stripe_batch(waves) * sizeof(StripeEnt);
+  const size_t m = acc > q ? acc : q;
+  return ((m > list ? m : list) + 15) & ~(size_t)15;
 }
 inline size_t rows_lds_bytes(int waves, int nout, int L, int ncell) {
   return rows_acc_bytes(waves, nout, L) + (size_t)(3 * ncell + 1) * 4;
@@ -853,6 +879,86 @@ __device__ __forceinline__ void list_cells(const Dev& d, const int2* __restrict_
   __syncthreads();
 }
 
+// The same lists for the forward, by one wave (lane l of `lane`, which alone calls it): classes 0 (far), 1
+// (side) and 2 (centre), no condition on the segments.  The cells are walked in (class, i) order, lane l
+// taking cells 2 l and 2 l + 1 of each 128, so one wave scan of the counts numbers 128 cells; no scratch.
+// The block's other waves go on meanwhile; a barrier must follow.
+__device__ __forceinline__ void list_cells_fwd(const Dev& d, const int2* __restrict__ rng, int cell, int lane, int* c_beg,
+                                               int* c_cum, int* c_ab, int* ncls) {
+  const int n = d.ne, side = 2 * n + 1, ncell = side * side, nfar = ncell - 9;
+  const int px = cell % d.gx - d.halo;
+  const int py = (cell / d.gx) % d.gy - d.halo;
+  const int evp = cell / (d.gx * d.gy);
+  const int top = (n - 1) * side, mid = top + 3 * (side - 3);  // far cells before the rows a = -1 .. 1, and through them
+  int rank0 = 0, before0 = 0;
+  for (int i0 = 0; i0 < ncell; i0 += 2 * kWave) {
+    int cnt[2], beg[2], ab[2], cls[2];
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const int i = i0 + 2 * lane + h;
+      int a = 0, b = 0;
+      cls[h] = i < nfar ? 0 : (i < ncell - 1 ? 1 : 2);
+      if (i < top) {
+        a = i / side - n;
+        b = i % side - n;
+      } else if (i < mid) {
+        const int j = i - top, w = side - 3;
+        a = j / w - 1;
+        b = j % w - n;
+        if (b >= -1) b += 3;
+      } else if (i < nfar) {
+        const int j = i - mid;
+        a = j / side + 2;
+        b = j % side - n;
+      } else if (i < ncell - 1) {
+        const int j = i - nfar, k = j < 4 ? j : j + 1;  // 3 x 3 without its centre
+        a = k / 3 - 1;
+        b = k % 3 - 1;
+      }
+      const int qx = px - a, qy = py - b;
+      cnt[h] = beg[h] = 0;
+      ab[h] = ((a + 64) << 8) | (b + 64);
+      if (i < ncell && qx >= -d.halo && qx < d.nx + d.halo && qy >= -d.halo && qy < d.ny + d.halo) {
+        const int2 rg = rng[((int64_t)evp * d.gy + (qy + d.halo)) * d.gx + (qx + d.halo)];
+        beg[h] = rg.x;
+        cnt[h] = rg.y > rg.x ? rg.y - rg.x : 0;
+      }
+    }
+    // listed cells before this lane's, and their segments
+    const uint64_t m0 = __ballot(cnt[0] > 0), m1 = __ballot(cnt[1] > 0);
+    const uint64_t lt = (1ull << lane) - 1;
+    int inc = cnt[0] + cnt[1];
+#pragma unroll
+    for (int dd = 1; dd < kWave; dd <<= 1) {
+      const int u = __shfl_up(inc, dd, kWave);
+      if (lane >= dd) inc += u;
+    }
+    int rk = rank0 + __popcll(m0 & lt) + __popcll(m1 & lt), before = before0 + inc - cnt[0] - cnt[1];
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      if (cnt[h] == 0) continue;
+      c_beg[rk] = beg[h];
+      c_cum[rk] = before;
+      c_ab[rk] = ab[h];
+      ++rk;
+      before += cnt[h];
+    }
+    // listed cells of class <= c, c < 3
+    const uint64_t f0 = __ballot(cnt[0] > 0 && cls[0] == 0), f1 = __ballot(cnt[1] > 0 && cls[1] == 0);
+    const uint64_t s0 = __ballot(cnt[0] > 0 && cls[0] <= 1), s1 = __ballot(cnt[1] > 0 && cls[1] <= 1);
+    if (lane == 0) {
+      ncls[0] = (i0 ? ncls[0] : 0) + __popcll(f0) + __popcll(f1);
+      ncls[1] = (i0 ? ncls[1] : 0) + __popcll(s0) + __popcll(s1);
+    }
+    rank0 += __popcll(m0) + __popcll(m1);
+    before0 += __builtin_amdgcn_readlane(inc, kWave - 1);
+  }
+  if (lane == 0) {
+    ncls[2] = rank0;
+    c_cum[rank0] = before0;
+  }
+}
+
 // ------------------------------------------------------------------------------------------
 // work-balanced XCD bands of pixel rows for the row kernels
 // ------------------------------------------------------------------------------------------
@@ -930,10 +1036,12 @@ __global__ void k_row_work(Dev d, const int2* __restrict__ rng, const int* __res
 constexpr int kBandThreads = 1024;
 
 __global__ __launch_bounds__(kBandThreads) void k_bands(const int* __restrict__ work, const int* __restrict__ n_rows_dev,
-                                                      int64_t max_rows, int64_t slots, int* __restrict__ band) {
+                                                      int64_t max_rows, int64_t slots, int* __restrict__ band,
+                                                      int* __restrict__ next) {
   __shared__ int64_t part[kBandThreads];
   __shared__ int64_t cut[kXcd + 1];
   const int t = threadIdx.x;
+  if (t < kXcd) next[t * kNextPad] = 0;
   const int64_t P = *n_rows_dev < max_rows ? *n_rows_dev : max_rows;
   const int64_t per = (P + kBandThreads - 1) / kBandThreads;
   const int64_t r0 = (int64_t)t * per < P ? (int64_t)t * per : P;
@@ -976,36 +1084,75 @@ __global__ __launch_bounds__(kBandThreads) void k_bands(const int* __restrict__ 
   }
 }
 
-#ifndef LSIM_FAR_GROUP
-#define LSIM_FAR_GROUP 8
-#endif
-constexpr int kFarGroup = LSIM_FAR_GROUP;  // independent neighbour-only pairs in flight per wave
+// XCD-aware mapping of workgroups onto rows: workgroups are dispatched round-robin over the XCDs, so
+// workgroup i runs on XCD x = i % kXcd.  Band x (k_bands) holds contiguous slots of the tile-major
+// processing order at equal shares of the estimated work, so a band's records and tables stay in that
+// XCD's L2.  Workgroup i takes slot i / kXcd of band x among the band's first `fixed` slots (three
+// quarters of an equal share of the rows); the later workgroups take the next slot of band x that is left
+// and, with band x used up, one of another band: the work estimate is linear in the pairs, rows are not,
+// and an XCD that is done early would stand idle (on 60 events of 5k and 72k segments a quarter of the
+// CU time did: 25.0 -> 20.0 ms).  Taking every slot that way is slower for launches of 10k light rows (the
+// counters' atomics pass to the memory side: 0.32 -> 0.50 ms).  Which workgroup computes a row
+// changes nothing in the row.  Workgroups that find no slot exit at once.  A launch whose workgroups are
+// all resident together (max_rows <= kStaticRows) needs no balancing: every slot is taken by its index.
+constexpr int kStaticRows = 1024;
 
-// XCD-aware, work-balanced mapping of workgroups onto rows: workgroups are dispatched round-robin
-// over the XCDs, so workgroup i runs on XCD x = i % kXcd; it takes slot i / kXcd of band x (k_bands:
-// contiguous slots of the tile-major processing order, cut at equal shares of the estimated work,
-// so a band's records and tables stay in that XCD's L2 and every XCD finishes at about the same
-// time), and computes row order[slot].  The grid holds kXcd times the
-// longest band allowed (rows_grid); the workgroups past their band's end exit at once.
+__device__ __forceinline__ int take_row(const int* __restrict__ band, int* __restrict__ next,
+                                        const int* __restrict__ order, int P, int64_t max_rows, int* sh) {
+  const int x = (int)(blockIdx.x % kXcd);
+  const int j = (int)(blockIdx.x / kXcd), fixed = max_rows <= kStaticRows ? P : 3 * (P / kXcd) / 4;
+  if (j < fixed && j < band[x + 1] - band[x]) return band[x] + j < P ? order[band[x] + j] : -1;
+  if (max_rows <= kStaticRows) return -1;
+  if (threadIdx.x < kWave) {
+    // lane b < kXcd: band b.  The bands with slots left, this XCD's first; a band found used up on the
+    // way is not tried again.
+    const int b = threadIdx.x < kXcd ? threadIdx.x : 0;
+    const int len = band[b + 1] - band[b], b0 = band[b] + (len < fixed ? len : fixed), n = band[b + 1] - b0;
+    const bool left =
+        threadIdx.x < kXcd && __hip_atomic_load(next + b * kNextPad, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < n;
+    uint32_t m = (uint32_t)__ballot(left);
+    int r = -1;
+    while (m != 0 && r < 0) {
+      const uint32_t from_x = m >> x << x;
+      const int y = __builtin_ctz(from_x ? from_x : m);
+      m &= ~(1u << y);
+      int i = 0;
+      if (threadIdx.x == 0) i = atomicAdd(next + y * kNextPad, 1);
+      i = __builtin_amdgcn_readfirstlane(i);
+      const int y0 = __builtin_amdgcn_readlane(b0, y), ny = __builtin_amdgcn_readlane(n, y);
+      if (i < ny && y0 + i < P) r = order[y0 + i];
+    }
+    if (threadIdx.x == 0) *sh = r;
+  }
+  __syncthreads();
+  const int r = *sh;
+  __syncthreads();
+  return r;
+}
+
+// One workgroup per pixel row.  What bounds it (160k rows, 2e8 stripe pairs, 4 waves a row; parts by
+// leaving each out): the stripes' chunk sums 7 of 19 ms (one 4-byte-per-lane load per pair and chunk is near
+// the texture unit's 16 lanes a cycle), the bins' windows 5.5, their counting sort 2.5, the self-trigger 2;
+// occupancy is 4 workgroups a CU by LDS (40 KB).  One wave per pair with a read-modify-write of the row in
+// LDS, and the bins as unrolled scalar code, took 25 to 32 ms for the same rows.
 template <int NB, int WAVES>
-__global__ __launch_bounds__(WAVES * kWave) __attribute__((amdgpu_waves_per_eu(WAVES == 2 ? 5 : 1))) void k_rows_fwd(Dev d, Tables tb, const SegRec* __restrict__ rec,
+__global__ __launch_bounds__(WAVES * kWave) void k_rows_fwd(Dev d, Tables tb, const SegRec* __restrict__ rec,
                                                             const int2* __restrict__ rng, const int* __restrict__ row_cell,
                                                             const int* __restrict__ n_rows_dev, int64_t max_rows,
-                                                            const int* __restrict__ band, const int* __restrict__ order,
+                                                            const int* __restrict__ band, int* __restrict__ next,
+                                                            const int* __restrict__ order,
                                                             const float* __restrict__ dtot,
                                                             const PairRec* __restrict__ prs, int64_t nseg, RowOut out) {
   constexpr int NT = WAVES * kWave;
   extern __shared__ __align__(16) char smem[];
   __shared__ double shd[NT / kWave];
-  __shared__ int shi[NT / kWave];
+  __shared__ int shi[2][NT / kWave];
   __shared__ int ncls[3];  // far cells, + the centre cell, + the 8 side cells
 
   const int P0 = *n_rows_dev;
   const int P = P0 < max_rows ? P0 : (int)max_rows;
-  const int xcd = (int)(blockIdx.x % kXcd);
-  const int slot = band[xcd] + (int)(blockIdx.x / kXcd);
-  if (slot >= band[xcd + 1] || slot >= P) return;  // past the band (the bound on P is a guard only)
-  const int r = order[slot];
+  const int r = take_row(band, next, order, P, max_rows, ncls);
+  if (r < 0) return;
   const int nout = d.nout;
   float* acc = (float*)smem;
   // this row's neighbourhood cells: far cells first, then the 3x3 near cells, in (a, b) order
@@ -1025,156 +1172,238 @@ __global__ __launch_bounds__(WAVES * kWave) __attribute__((amdgpu_waves_per_eu(W
     const int py = (cell / d.gx) % d.gy - d.halo;
     out.pixel_ids[r] = ((int64_t)evp * d.ny + py) * d.nx + px;
   }
-  // far cells first, then the 8 side cells, then the centre cell (the partial rows are scratch)
-  list_cells<NT>(
-      d, rng, cell,
-      [](int a, int b) {
-        const bool near = a >= -1 && a <= 1 && b >= -1 && b <= 1;
-        return !near ? 0 : ((a == 0 && b == 0) ? 2 : 1);
-      },
-      [](int b, int e) { return e - b; }, reinterpret_cast<int*>(acc), c_beg, c_cum, c_ab, ncls);
-  {
-    // 16-byte stores (smem is 16-byte aligned), then the remainder
-    const int nz = WAVES * rstride, n4 = nz / 4;
-    for (int o = t; o < n4; o += NT) reinterpret_cast<float4*>(acc)[o] = make_float4(0.f, 0.f, 0.f, 0.f);
-    for (int o = 4 * n4 + t; o < nz; o += NT) acc[o] = 0.f;
-  }
+  if (wid == 0) list_cells_fwd(d, rng, cell, lane, c_beg, c_cum, c_ab, ncls);
+  __shared__ int s_hist[kStripeKeys + 2][WAVES];  // counts, then first places, of (key, wave)
+  __shared__ int s_start[kStripeKeys + 2];        // first place of each key
+  __shared__ float s_edge[kRowChunks + 1];        // A1 at each chunk's first tick (belongs to the tick before)
+  __shared__ int s_next;                          // next non-empty chunk to take
+  __shared__ float s_tick0[WAVES];                // what the waves' pairs leave at output tick 0
+  __shared__ float s_bins[WAVES][kBinItems][4 * NB];
+  for (int o = t; o < rstride; o += NT) acc[o] = 0.f;
+  if (t <= kRowChunks) s_edge[t] = 0.f;
   __syncthreads();
 
   float* accw = acc + wid * rstride;
   const int nsc = ncls[1], nct = ncls[2];  // far + side cells, all cells
-  // Neighbour stripes of the far and side pairs, flattened over those cells in blocks of 64: wave
-  // w takes blocks w, w + WAVES, ...  Lane l loads pair 64 b + l's record, boundary correction and
-  // row offset into registers (one memory round trip per block instead of one per pair group),
-  // then the wave walks the block kFarGroup pairs at a time, reading each pair's values from its
-  // lane.  A side pair's correction covers its diffusion bins too; the bins that land on a side
-  // row (segments near the pixel edge only) follow per block, picked out by a ballot.
+  const int nsb = d.nsb, L = d.L;
+  // Neighbour stripes of the far and side pairs, flattened over those cells, in batches of
+  // kStripeRounds * 64 pairs per wave.  Lane by lane: the pair's record and correction, its factors,
+  // window and sort key; the batch is counting-sorted (stable: by wave, round, lane) into the list, and
+  // the waves take its non-empty chunks in turn.  A side pair's correction covers its diffusion bins
+  // too (they follow below).
+  float tick0 = 0.f;
   {
-    const int nfar = c_cum[nsc];
-    const int W4 = kWinPad * 4, nsb = d.nsb, side = 2 * d.ne + 1;
-    const __amdgpu_buffer_rsrc_t tnp =
-        __builtin_amdgcn_make_buffer_rsrc((void*)tb.TNP, 0, d.lx * d.ly * kWinPad * 4, kBufDesc3);
-    // lane l's pair of the block at b0: its cell (a binary search of the cell list), record and
-    // correction.  The loads of the wave's next block are issued before this block's stores, so
-    // they arrive while the pairs are stored.
-    struct BlockIn {
-      PairRec P;
-      float D;
-      int sg, ab;
-    };
-    auto fetch = [&](int b0, BlockIn& B) {
-      const int p = b0 + lane;
-      if (p < nfar) {
-        int lo = 0, hi = nsc - 1;  // the cell holding p: last c with c_cum[c] <= p
-        while (lo < hi) {
-          const int mid = (lo + hi + 1) >> 1;
-          if (c_cum[mid] <= p) lo = mid;
-          else hi = mid - 1;
-        }
-        B.sg = c_beg[lo] + (p - c_cum[lo]);
-        B.ab = c_ab[lo];
-        const int a = (B.ab >> 8) - 64, b = (B.ab & 255) - 64;
-        B.P = prs[B.sg];
-        B.D = dtot[(int64_t)((a + d.ne) * side + (b + d.ne)) * nseg + B.sg];
-      }
-    };
-    BlockIn cur, nxt;
-    if (wid * kWave < nfar) fetch(wid * kWave, cur);
-    for (int b0 = wid * kWave; b0 < nfar; b0 += WAVES * kWave) {
-      if (b0 + WAVES * kWave < nfar) fetch(b0 + WAVES * kWave, nxt);
-      const int p = b0 + lane;
-      // padding lanes: an interior window at S = 2 with zero charge and correction (adds +0)
-      int rS = (2 << 1) | 1, roff = 0, rsg = 0, rab = 0;
-      float rso = 0.f, rsf = 0.f, rfD = 0.f, romfD = 0.f;
-      bool bins = false;
-      if (p < nfar) {
-        const int sg = cur.sg, ab = cur.ab;
-        const int a = (ab >> 8) - 64, b = (ab & 255) - 64;
-        // row offset = cell constant + ma U + za U0 + mb V + zb V0 (bytes)
-        int kc = 0, ma = 0, za = 0, mb = 0, zb = 0;
-        if (a > 0) { kc += (nsb * a + nsb / 2 - 1) * d.ly * W4; ma = -1; }
-        else if (a < 0) { kc += (nsb * -a - nsb / 2) * d.ly * W4; ma = 1; }
-        else za = 1;
-        if (b > 0) { kc += (nsb * b + nsb / 2 - 1) * W4; mb = -1; }
-        else if (b < 0) { kc += (nsb * -b - nsb / 2) * W4; mb = 1; }
-        else zb = 1;
-        const PairRec& P = cur.P;
-        const float D = cur.D;
-        // with no neighbour stripes (nn = 0) a side pixel gets its diffusion bins only
-        const float st = a >= -d.nn && a <= d.nn && b >= -d.nn && b <= d.nn ? 1.f : 0.f;
-        roff = kc + ma * P.U + za * P.U0 + mb * P.V + zb * P.V0;
-        rS = (P.S << 1) | (P.flags & 1);
-        const float omf = 1.f - P.f;
-        rso = st * (P.ne * omf);
-        rsf = st * (P.ne * P.f);
-        rfD = P.f * D;
-        romfD = omf * D;
-        rsg = sg;
-        rab = ab;
-        bins = a >= -1 && a <= 1 && b >= -1 && b <= 1 && P.ne != 0.f && bins_reach<NB>((P.flags >> 8) & 255, a, nsb) &&
-               bins_reach<NB>((P.flags >> 16) & 255, b, nsb);
-      }
-      const int n = __builtin_amdgcn_readfirstlane(nfar - b0 < kWave ? nfar - b0 : kWave);
-      float* base = accw - 2;
-      const float m0 = lane == 0 ? 1.f : 0.f, m1 = lane == 1 ? 1.f : 0.f;
-      // pairs i .. i + kFarGroup - 1 of the block: their factors from the owning lanes, their window
-      // loads issued (j < 64: i < n <= 64 and i is a multiple of kFarGroup)
-      struct FarGroup {
-        FarLoads q[kFarGroup];
-        int S[kFarGroup];
-        float so[kFarGroup], sf[kFarGroup], fD[kFarGroup], omfD[kFarGroup];
-      };
-      auto issue = [&](int i, FarGroup& G) {
+    const int nfar = c_cum[nsc], side = 2 * d.ne + 1;
+    const int stride = stripe_stride(L), nchunk = nout / kWave + 1;
+    StripeEnt* const list = reinterpret_cast<StripeEnt*>(smem + rows_list_off(nout, L));
+    const __amdgpu_buffer_rsrc_t tnq = __builtin_amdgcn_make_buffer_rsrc(
+        (void*)tb.TNQ, 0, (int)(uint32_t)(stripe_floats(d.lx, d.ly, L) * 4), kBufDesc3);
+    for (int b0 = 0; b0 < nfar; b0 += stripe_batch(WAVES)) {
+      for (int i = t; i < (kStripeKeys + 2) * WAVES; i += NT) (&s_hist[0][0])[i] = 0;
+      __syncthreads();  // also: the last batch's list has been read
+      StripeEnt E[kStripeRounds];
+      int key[kStripeRounds], place[kStripeRounds];
 #pragma unroll
-        for (int g = 0; g < kFarGroup; ++g) {
-          const int j = i + g;
-          G.S[g] = __builtin_amdgcn_readlane(rS, j);
-          G.so[g] = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(rso), j));
-          G.sf[g] = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(rsf), j));
-          G.fD[g] = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(rfD), j));
-          G.omfD[g] = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(romfD), j));
-          far_load_buf(tnp, lane * 4, __builtin_amdgcn_readlane(roff, j), G.q[g]);
+      for (int q = 0; q < kStripeRounds; ++q) {
+        const int p0 = b0 + (q * WAVES + wid) * kWave, p = p0 + lane;
+        key[q] = kKeyNone;
+        place[q] = 0;
+        if (p0 >= nfar) continue;
+        if (p < nfar) {
+          int lo = 0, hi = nsc - 1;  // the cell holding p: last c with c_cum[c] <= p
+          while (lo < hi) {
+            const int mid = (lo + hi + 1) >> 1;
+            if (c_cum[mid] <= p) lo = mid;
+            else hi = mid - 1;
+          }
+          const int sg = c_beg[lo] + (p - c_cum[lo]);
+          const int ab = c_ab[lo];
+          const int a = (ab >> 8) - 64, b = (ab & 255) - 64;
+          const PairRec P = prs[sg];
+          const float D = dtot[(int64_t)((a + d.ne) * side + (b + d.ne)) * nseg + sg];
+          E[q].D = D;
+          const float omf = 1.f - P.f;
+          E[q].so = P.ne * omf;
+          E[q].sf = P.ne * P.f;
+          if (P.S == 1) tick0 += E[q].so * D;  // the corrections at output tick 0
+          if (P.S == 2) tick0 += E[q].sf * D;
+          if (P.S == nout) E[q].so = 0.f;  // a correction at the last tick is dropped
+          // with no neighbour stripes (nn = 0) a side pixel gets its diffusion bins only: the zero row
+          const bool on = a >= -d.nn && a <= d.nn && b >= -d.nn && b <= d.nn;
+          const int row = on ? offset_bin((P.flags >> 8) & 255, a, nsb) * d.ly + offset_bin((P.flags >> 16) & 255, b, nsb)
+                             : d.lx * d.ly;
+          E[q].addr = (int)(4u * ((uint32_t)row * (uint32_t)stride + (uint32_t)(kStripeLead - kTickOff - P.S)));
+          const int pos = P.S - 1 + kTickOff;
+          key[q] = 2 * (pos / kWave) + ((pos & (kWave - 1)) >= kTickOff - L ? 1 : 0);
+          if (P.ne == 0.f || P.S > nout) key[q] = kKeyNone;
+          if (!(fabsf(E[q].so) + fabsf(E[q].sf) < __builtin_inff())) {
+            key[q] = kKeyOdd;
+            E[q].addr = row * stride;
+            E[q].D = __int_as_float(P.S);
+          }
         }
-      };
-      // unconditional stores: a branch on the charge would let the compiler sink a pair's loads
-      // into it and wait on them there instead of overlapping them with the other pairs'
-      auto drain = [&](const FarGroup& G) {
+        // place among the wave's pairs of the same key so far
+        uint64_t peers = ~0ull;
 #pragma unroll
-        for (int g = 0; g < kFarGroup; ++g)
-          store_stripe(base, lane, m0, m1, G.q[g].t0, G.q[g].t1, G.q[g].t2, G.so[g], G.sf[g], G.fD[g], G.omfD[g],
-                       G.S[g] >> 1, d.L, d.nout, (G.S[g] & 1) != 0);
-      };
-      // (issuing the next group's loads before this group's stores measured no faster on the
-      // MI355X: the loads are not what the waves wait on; 8-pair groups are 1 % faster than 4)
-      for (int i = 0; i < n; i += kFarGroup) {
-        FarGroup A;
-        issue(i, A);
-        drain(A);
+        for (int bt = 0; bt < 7; ++bt) {
+          const bool bit = (key[q] >> bt) & 1;
+          const uint64_t m = __ballot(bit);
+          peers &= bit ? m : ~m;
+        }
+        const int rank = __popcll(peers & ((1ull << lane) - 1));
+        const int before = s_hist[key[q]][wid];
+        __builtin_amdgcn_wave_barrier();  // wave-local LDS: program order
+        if (rank == 0) s_hist[key[q]][wid] = before + __popcll(peers);
+        __builtin_amdgcn_wave_barrier();
+        place[q] = before + rank;
       }
-      for (uint64_t m = __ballot(bins); m != 0; m &= m - 1) {
-        const int j = __builtin_ctzll(m);
-        const int ab = __builtin_amdgcn_readlane(rab, j);
-        const SegRec R = rec[__builtin_amdgcn_readlane(rsg, j)];
-        float v0, v1, v2;
-        pixel_bins<NB>(d, tb, R, (ab >> 8) - 64, (ab & 255) - 64, lane, v0, v1, v2);
-        const int S = d.nt - d.L - R.k0;
-        store_window(accw, lane, v0, v1, v2, 1.f, 1.f - R.f, R.f, 0.f, S, d.L, d.nout, S >= 2 && S + d.L <= d.nout);
+      __syncthreads();
+      if (wid == 0) {
+        if (lane == 0) s_next = 0;
+        // lane l: keys 2 l and 2 l + 1
+        int n[2] = {0, 0};
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+          if (2 * lane + h < kKeyNone)
+            for (int w = 0; w < WAVES; ++w) n[h] += s_hist[2 * lane + h][w];
+        int inc = n[0] + n[1];
+#pragma unroll
+        for (int dd = 1; dd < kWave; dd <<= 1) {
+          const int u = __shfl_up(inc, dd, kWave);
+          if (lane >= dd) inc += u;
+        }
+        int at = inc - n[0] - n[1];
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+          const int k = 2 * lane + h;
+          if (k <= kKeyNone) s_start[k] = at;
+          if (k < kKeyNone)
+            for (int w = 0; w < WAVES; ++w) {
+              const int c = s_hist[k][w];
+              s_hist[k][w] = at;
+              at += c;
+            }
+        }
       }
-      cur = nxt;
+      __syncthreads();
+#pragma unroll
+      for (int q = 0; q < kStripeRounds; ++q)
+        if (key[q] < kKeyNone) list[s_hist[key[q]][wid] + place[q]] = E[q];
+      __syncthreads();
+      // lane k: does output chunk k hold anything?  The waves take the non-empty ones as they come free
+      // (whichever wave takes a chunk adds the same pairs in the same order).
+      const int kk = lane < nchunk ? lane : 0;
+      uint64_t todo = __ballot(lane < nchunk && s_start[2 * kk + 8] > s_start[2 * kk + 1]);
+      for (int turn = 0;;) {
+        int mine = 0;
+        if (lane == 0) mine = atomicAdd(&s_next, 1);
+        mine = __builtin_amdgcn_readfirstlane(mine);
+        for (; turn < mine && todo != 0; ++turn) todo &= todo - 1;
+        if (todo == 0) break;
+        const int k = __builtin_ctzll(todo);
+        const int e0 = __builtin_amdgcn_readfirstlane(s_start[2 * k + 1]);  // chunk k + 3: keys 2 k + 1 .. 2 k + 7
+        const int e1 = __builtin_amdgcn_readfirstlane(s_start[2 * k + 6]);
+        const int e2 = __builtin_amdgcn_readfirstlane(s_start[2 * k + 8]);
+        const int pos4 = 4 * (k * kWave + kTickOff + lane);
+        StripeSums A;
+        stripe_run<false>(tnq, list, e0, e1, lane, pos4, A);
+        stripe_run<true>(tnq, list, e1, e2, lane, pos4, A);
+        const float a0 = (A.a0[0] + A.a0[1]) + (A.a0[2] + A.a0[3]), a1 = (A.a1[0] + A.a1[1]) + (A.a1[2] + A.a1[3]);
+        const int o = k * kWave + lane;
+        if (lane == 0) s_edge[k] += a1;
+        const float v = a0 + lane_next0(a1);
+        if (o < nout) acc[o] += v;
+      }
+      // pairs with non-finite factors, tick by tick (each tick has one owner in this loop)
+      const int x0 = s_start[kKeyOdd], x1 = s_start[kKeyNone];
+      if (x0 < x1) {
+        __syncthreads();
+        for (int x = x0; x < x1; ++x)
+          for (int o = t; o < nout; o += NT) {
+            const float v = odd_pair(tb.TNQ, list[x], o, L, nout);
+            if (o == 0) tick0 += v;
+            else acc[o] += v;
+          }
+      }
     }
+    tick0 = wave_sum(tick0);
+    if (lane == 0) s_tick0[wid] = tick0;
+    __syncthreads();
+    // chunk edges, tick 0 and the other waves' rows
+    if (t >= 1 && t < nchunk && t * kWave - 1 < nout) acc[t * kWave - 1] += s_edge[t];
+    if (t == 0) {
+      float v = 0.f;
+      for (int w = 0; w < WAVES; ++w) v += s_tick0[w];
+      acc[0] = v;
+    }
+    for (int o = rstride + t; o < WAVES * rstride; o += NT) acc[o] = 0.f;
+    __syncthreads();
   }
-  // the centre cell: the window of each segment's bins on this pixel, from the interpolated
-  // templates of its distinct LUT cells, one segment per wave at a time
-  const float* dtc = dtot + (int64_t)(d.ne * (2 * d.ne + 1) + d.ne) * nseg;
-  for (int c = nsc; c < nct; ++c) {
-    const int beg = __builtin_amdgcn_readfirstlane(c_beg[c]);
-    const int cnt = __builtin_amdgcn_readfirstlane(c_cum[c + 1] - c_cum[c]);
-    for (int k = wid; k < cnt; k += WAVES) {
-      const int sg = beg + k;
-      float v0, v1, v2;
-      pixel_bins<NB>(d, tb, rec[sg], 0, 0, lane, v0, v1, v2);
-      const PairRec P = prs[sg];
-      store_window(accw, lane, v0, v1, v2, 1.f, 1.f - P.f, P.f, dtc[sg], P.S, d.L, d.nout, (P.flags & 1) != 0);
+  // Diffusion bins that land on this pixel: from every segment of the centre cell, and from those of the
+  // side cells near their pixel's edge.  Each wave takes every WAVES-th pair (the centre cell's pairs are most
+  // of the work), 64 at a time.  Lane by lane: does any bin land here, and the bins merged per LUT cell
+  // along each axis, staged in LDS for the wave, which then computes and stores one pair's window after
+  // the other.
+  {
+    const int p0 = c_cum[ncls[0]], p1 = c_cum[nct];
+    const int cm = d.cm, ws4 = 4 * bin_stride(L);
+    const float* dtc = dtot + (int64_t)(d.ne * (2 * d.ne + 1) + d.ne) * nseg;
+    const int lane12 = 3 * lane < L + 2 ? 12 * lane : 0x7ffffff0;
+    const __amdgpu_buffer_rsrc_t tmw = __builtin_amdgcn_make_buffer_rsrc(
+        (void*)tb.TMW, 0, (int)(uint32_t)(bin_floats(d.nm, cm, L) * 4), kBufDesc3);
+    for (int b0 = p0; b0 < p1; b0 += WAVES * kWave) {
+      const int p = b0 + lane * WAVES + wid;
+      bool on = false;
+      PairRec P;
+      int base = 0, cxs[NB], cys[NB];
+      float la = 0.f, lb = 0.f, lc = 0.f, delta = 0.f, WX[NB], WY[NB];
+      if (p < p1) {
+        int lo = ncls[0];  // at most 9 cells
+        while (c_cum[lo + 1] <= p) ++lo;
+        const int sg = c_beg[lo] + (p - c_cum[lo]);
+        const int ab = c_ab[lo];
+        const int a = (ab >> 8) - 64, b = (ab & 255) - 64;
+        P = prs[sg];
+        const int ux = (P.flags >> 8) & 255, uy = (P.flags >> 16) & 255;
+        on = P.ne != 0.f && bins_reach<NB>(ux, a, nsb) && bins_reach<NB>(uy, b, nsb);
+        if (on) {
+          const SegRec& R = rec[sg];
+          la = R.la;
+          lb = R.lb;
+          lc = R.lc;
+          base = (R.idx - 1) * ws4;
+          if (lo >= nsc) delta = P.ne * dtc[sg];  // (a side pair's correction went with its stripe)
+          bool ok[NB];
+          axis_merge<NB>(ux, a, nsb, R.wx, P.ne, ok, cxs, WX);
+          axis_merge<NB>(uy, b, nsb, R.wy, 1.f, ok, cys, WY);
+        }
+      }
+      for (uint64_t m = __ballot(on); m != 0;) {
+        const int rank = __popcll(m & ((1ull << lane) - 1));
+        if (((m >> lane) & 1) && rank < kBinItems) {
+          float* st = s_bins[wid][rank];
+#pragma unroll
+          for (int k = 0; k < NB; ++k) {
+            st[k] = WX[k];
+            st[NB + k] = WY[k];
+            st[2 * NB + k] = __int_as_float(cxs[k] * cm * d.nm * ws4);
+            st[3 * NB + k] = __int_as_float(cys[k] * d.nm * ws4);
+          }
+        }
+        __builtin_amdgcn_wave_barrier();  // wave-local LDS: program order
+        for (int k = 0; k < kBinItems && m != 0; ++k) {
+          const int j = __builtin_ctzll(m);
+          m &= m - 1;
+          auto get = [&](float v) { return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), j)); };
+          const int S = __builtin_amdgcn_readlane(P.S, j);
+          const float f = get(P.f);
+          float v0, v1, v2;
+          bins_window<NB>(tmw, s_bins[wid][k], __builtin_amdgcn_readlane(base, j), ws4, lane, lane12, get(la), get(lb),
+                          get(lc), v0, v1, v2);
+          store_window(accw, lane, v0, v1, v2, 1.f - f, f, get(delta), S, L, nout, S >= 2 && S + L <= nout);
+        }
+        __builtin_amdgcn_wave_barrier();  // the stage is rewritten
+      }
     }
   }
   __syncthreads();
@@ -1192,7 +1421,7 @@ __global__ __launch_bounds__(NT) void k_fee_rows(Dev d, const float* __restrict_
   __shared__ __align__(16) char smem[kMaxOut * 8];
   __shared__ float accs[kMaxOut];
   __shared__ double shd[NT / kWave];
-  __shared__ int shi[NT / kWave];
+  __shared__ int shi[2][NT / kWave];
   const int64_t r = blockIdx.x;
   if (r >= n_rows) return;
   for (int o = threadIdx.x; o < kMaxOut; o += NT) accs[o] = o < d.nout ? wfs[r * d.nout + o] : 0.f;
@@ -1409,6 +1638,33 @@ __global__ __launch_bounds__(256) void k_lut_tables(Dev d, const float* __restri
       c += (double)win[j];
       CT[sbase * (L + 1) + j + 1] = c;
     }
+  }
+}
+
+// The raw-response windows TN as TNQ (stripe_floats values).
+__global__ void k_lut_tnq(Dev d, const float* __restrict__ TN, float* __restrict__ TNQ) {
+  const int stride = stripe_stride(d.L);
+  const int64_t ns = (int64_t)d.lx * d.ly, total = stripe_floats(d.lx, d.ly, d.L);
+  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < total; i += (int64_t)gridDim.x * blockDim.x) {
+    const int64_t row = i / stride;
+    const int m = (int)(i - row * stride) - kStripeLead;
+    float v = 0.f;
+    if (row <= ns && m == -1) v = __uint_as_float(kStripeMark);
+    if (row < ns && m >= 0 && m < d.L) v = TN[row * d.L + m];
+    TNQ[i] = v;
+  }
+}
+
+// The template windows TM regrouped as TMW, with the leading zeros of each row (and two values past the
+// last row).
+__global__ void k_lut_tmw(Dev d, const float* __restrict__ TM, float* __restrict__ TMW, int64_t total) {
+  const int ws = bin_stride(d.L);
+  const int64_t cc = (int64_t)d.cm * d.cm, rows = cc * d.nm;
+  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < total; i += (int64_t)gridDim.x * blockDim.x) {
+    const int64_t row = i / ws;
+    const int j = (int)(i - row * ws) - 2;
+    const int64_t m = row % d.nm, cell = row / d.nm;
+    TMW[i] = row < rows && j >= 0 ? TM[(m * cc + cell) * d.L + j] : 0.f;
   }
 }
 

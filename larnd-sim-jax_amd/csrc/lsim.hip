@@ -61,6 +61,8 @@ struct lsim_ctx {
   float* TM = nullptr;
   float* TN = nullptr;
   float* TNP = nullptr;
+  float* TNQ = nullptr;
+  float* TMW = nullptr;
   float2* DM = nullptr;
   float2* DN = nullptr;
   float2* DNS = nullptr;  // DN regrouped per (tick, sub-bin x, sub-bin y): one segment's neighbour entries contiguous
@@ -185,6 +187,7 @@ struct Ws {
   int* n_hits32;
   int* row_work;  // [n] estimated work of each pixel row in processing order (XCD band cuts)
   int* band;      // [kXcd + 1] first processing slot of each XCD's band
+  int* next;      // [kXcd][kNextPad] slots taken so far of those past each band's fixed part
   uint32_t *tk0, *tv0, *tk1, *tv1;  // [n + 1] tile sort ping-pong; the processing order lands in tv0 or tv1
   float* dtot;  // [(2 nn + 1)^2][n] boundary corrections of every (segment, row offset) pair
   size_t bytes;
@@ -212,6 +215,7 @@ Ws layout(void* base, int64_t n, int64_t n_cells) {
   w.n_hits32 = c.take<int>(4);
   w.row_work = c.take<int>(n);
   w.band = c.take<int>(kXcd + 1);
+  w.next = c.take<int>(kXcd * kNextPad);
   w.tk0 = c.take<uint32_t>(n + 1);
   w.tv0 = c.take<uint32_t>(n + 1);
   w.tk1 = c.take<uint32_t>(n + 1);
@@ -279,7 +283,7 @@ int launch_row_bands(const Dev& d, const Ws& w, int64_t max_rows, hipStream_t st
   hipLaunchKernelGGL(k_row_work, dim3(g), dim3(256), 0, st, d, w.rng, w.row_cell, row_order(w, d), w.n_rows, max_rows,
                      g_row_cost, w.row_work, w.hit_cnt);
   hipLaunchKernelGGL(k_bands, dim3(1), dim3(kBandThreads), 0, st, w.row_work, w.n_rows, max_rows, band_slots(max_rows),
-                     w.band);
+                     w.band, w.next);
   HIP_TRY(hipGetLastError());
   return LSIM_OK;
 }
@@ -288,9 +292,11 @@ template <int NB, int WAVES>
 void launch_rows_nb(const Dev& d, const Tables& tb, const Ws& w, int64_t n_seg, int64_t max_rows, const RowOut& ro,
                     hipStream_t st) {
   const size_t lds = rows_lds_bytes(WAVES, d.nout, d.L, (2 * d.ne + 1) * (2 * d.ne + 1));
-  const int64_t grid = kXcd * band_slots(max_rows);
+  // static rows: the longest band; else a workgroup per row and an eighth more, so that an XCD that is
+  // done early finds workgroups to go on with
+  const int64_t grid = max_rows <= kStaticRows ? kXcd * band_slots(max_rows) : max_rows + max_rows / 8;
   hipLaunchKernelGGL((k_rows_fwd<NB, WAVES>), dim3((unsigned)grid), dim3(WAVES * kWave), lds, st, d, tb, w.rec, w.rng,
-                     w.row_cell, w.n_rows, max_rows, w.band, row_order(w, d), w.dtot, w.prs, n_seg, ro);
+                     w.row_cell, w.n_rows, max_rows, w.band, w.next, row_order(w, d), w.dtot, w.prs, n_seg, ro);
 }
 
 template <int WAVES>
@@ -329,12 +335,14 @@ void free_tables(lsim_ctx* c) {
   (void)hipFree(c->TM);
   (void)hipFree(c->TN);
   (void)hipFree(c->TNP);
+  (void)hipFree(c->TNQ);
+  (void)hipFree(c->TMW);
   (void)hipFree(c->DM);
   (void)hipFree(c->DN);
   (void)hipFree(c->DNS);
   (void)hipFree(c->CTM);
   (void)hipFree(c->CTN);
-  c->TM = c->TN = c->TNP = nullptr;
+  c->TM = c->TN = c->TNP = c->TNQ = c->TMW = nullptr;
   c->TM3 = nullptr;
   c->DM = c->DN = c->DNS = nullptr;
   c->CTM = c->CTN = nullptr;
@@ -450,6 +458,8 @@ int lsim_lut_set(lsim_ctx* c, const float* raw, int32_t nx, int32_t ny, int32_t 
     const std::pair<void**, size_t> req[] = {
         {(void**)&c->TM3, ms * kWinPad * sizeof(float3)}, {(void**)&c->TM, ms * L * sizeof(float)},
         {(void**)&c->TN, ns * L * sizeof(float)},         {(void**)&c->TNP, ns * kWinPad * sizeof(float)},
+        {(void**)&c->TMW, (size_t)bin_floats(k.n_templates, c->cm, L) * sizeof(float)},
+        {(void**)&c->TNQ, (size_t)stripe_floats(nx, ny, L) * sizeof(float)},
         {(void**)&c->DM, ms * nt * sizeof(float2)},       {(void**)&c->DN, ns * nt * sizeof(float2)},
         {(void**)&c->DNS, nds * nt * sizeof(float2)},
         {(void**)&c->CTM, ms * (L + 1) * sizeof(double)}, {(void**)&c->CTN, ns * (L + 1) * sizeof(double)}};
@@ -465,6 +475,8 @@ int lsim_lut_set(lsim_ctx* c, const float* raw, int32_t nx, int32_t ny, int32_t 
   hipLaunchKernelGGL(k_lut_tables, dim3((unsigned)ms), dim3(256), 0, st, d, raw, 1, c->TM, (float*)nullptr, c->DM, c->CTM);
   hipLaunchKernelGGL(k_lut_tables, dim3((unsigned)ns), dim3(256), 0, st, d, raw, 0, c->TN, c->TNP, c->DN, c->CTN);
   hipLaunchKernelGGL(k_lut_tm3, dim3(1024), dim3(256), 0, st, d, c->TM, c->TM3);
+  hipLaunchKernelGGL(k_lut_tmw, dim3(1024), dim3(256), 0, st, d, c->TM, c->TMW, bin_floats(k.n_templates, c->cm, L));
+  hipLaunchKernelGGL(k_lut_tnq, dim3(1024), dim3(256), 0, st, d, c->TN, c->TNQ);
   hipLaunchKernelGGL(k_lut_dns, dim3(4096), dim3(256), 0, st, d, c->DN, c->DNS);
   const hipError_t e = hipGetLastError();
   if (e != hipSuccess) {
@@ -543,7 +555,7 @@ int lsim_forward_prepare(lsim_ctx* c, const lsim_params* p, const lsim_segments*
 
 static int forward_rows_impl(lsim_ctx* c, const Dev& d, const Ws& w, int64_t n_seg, int64_t max_rows,
                              const lsim_fwd_out* out, hipStream_t st) {
-  Tables tb{c->TM3, c->TM, c->TN, c->TNP, c->DM, c->DN, c->CTM, c->CTN};
+  Tables tb{c->TM3, c->TM, c->TMW, c->TN, c->TNP, c->TNQ, c->DM, c->DN, c->CTM, c->CTN};
   RowOut ro;
   ro.wfs = out->wfs;
   ro.adc = out->adc;
@@ -830,7 +842,7 @@ static int backward_impl(lsim_ctx* c, const lsim_params* p, const lsim_segments*
   double* dz = cv.take<double>(max_rows);
   double* partial = cv.take<double>(2 * max_rows * kNGrad);  // far pass rows, then near pass rows
   AdjRec* adj = cv.take<AdjRec>(n);
-  Tables tb{c->TM3, c->TM, c->TN, c->TNP, c->DM, c->DN, c->CTM, c->CTN};
+  Tables tb{c->TM3, c->TM, c->TMW, c->TN, c->TNP, c->TNQ, c->DM, c->DN, c->CTM, c->CTN};
   SegIn in = make_segin(seg);
   uint32_t *keys, *vals;
   sorted_buffers(w, d, keys, vals);
