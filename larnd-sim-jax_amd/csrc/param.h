@@ -107,50 +107,187 @@ __device__ __forceinline__ double emg_cdf_half(double X, double mu, double sigma
   return 0.5 * erf((X - mu) / (M_SQRT2 * sigma)) - pdf / lambd;
 }
 
-// One wave: sample k < T of one tail (decay `scale`) of a pair's current, loc = -t0 shifted,
-// integrated over the tick around sample time t_k: the integral runs between the boundaries
-// g_{k+1} = -t_k - dt/2 and g_k = -t_k + dt/2 (g_j = -t_j + dt/2 for j < T, g_T = -t_{T-1} - dt/2),
-// so lane j evaluates the tail's CDF (integrated_expon_diff, with diffusion) or its exponential
-// (integrated_expon) once at g_j and each value serves two samples (the next lane's by a shift).
-__device__ __forceinline__ double param_tail(double gj, double loc, double scale, double sigma, double dt, int T,
-                                             bool diffusion) {
-  if (diffusion) {
-    const double F = emg_cdf_half(gj, loc, sigma, 1.0 / scale);
-    const double Fn = __shfl_down(F, 1, kWave);
-    const double F1 = __shfl(F, 1, kWave), FT = __shfl(F, T - 1, kWave);  // lo of sample 0, up of T - 1
-    return (F - Fn) / (F1 - FT) / dt;
-  }
-  const double G = exp(fmin(0.0, (loc - gj) / scale));
-  const double Gn = __shfl_down(G, 1, kWave);
-  return (Gn - G + exp(fmin(0.0, (loc - dt / 2) / scale)) / T) / dt;
+// erfcx(x) = exp(x^2) erfc(x) of three non-negative arguments at once (they share the coefficients): the
+// method of Shepherd and Laframboise (Math. Comp. 36, 1981), (1 + 2 x) erfcx(x) as a polynomial in y =
+// (x - 3.75) / (x + 3.75).  The 25 coefficients are those of the truncated Chebyshev series computed in 60
+// digits; the relative error over 0 .. 1e6 is below 6e-16 in float64.  One reciprocal serves both quotients.
+constexpr int kErfcxN = 25;
+__device__ constexpr double kErfcx[kErfcxN] = {
+    1.2375126308378275,
+    -0.14024059858554697,
+    0.0035854154854644293,
+    0.0822767384901452,
+    -0.10880393014174886,
+    0.09230432116037748,
+    -0.05869339858963677,
+    0.028362277418956406,
+    -0.009746579558029276,
+    0.0017556258528952954,
+    0.0002937136655913448,
+    -0.0002901540805408417,
+    5.164909889268241e-05,
+    2.238423915508223e-05,
+    -1.1444146237700524e-05,
+    -9.73559896736775e-07,
+    1.751637648849062e-06,
+    -5.7218230603224086e-08,
+    -2.5866850716155884e-07,
+    2.3263508708859124e-08,
+    3.8675334242222354e-08,
+    -3.744210080962018e-09,
+    -5.1739902140113095e-09,
+    3.1114333809799254e-10,
+    4.2514714447963895e-10,
+};
+
+__device__ __forceinline__ double rcp_nr(double d) {  // 1 / d, d normal and finite: two Newton steps
+  double r = __builtin_amdgcn_rcp(d);
+  r = __builtin_fma(r, __builtin_fma(-d, r, 1.0), r);
+  return __builtin_fma(r, __builtin_fma(-d, r, 1.0), r);
 }
 
-// Both tails of a pair's current (decays sb and sc) at sample k: param_tail of each, with the
-// Gaussian part 1/2 erf((g - mu) / (sqrt2 sigma)) of the two CDFs evaluated once (the same operations
-// as emg_cdf_half, so the values are the same).
-__device__ __forceinline__ void param_tails(double gj, double loc, double sb, double sc, double sigma, double dt, int T,
-                                            bool diffusion, double& tb, double& tc) {
+// Horner step r <- r y + c of three polynomials.  The coefficient is held back from the register
+// allocator until here: 38 of them live across the loop over pairs would fill vector registers, each of
+// which is then copied before the (destructive) multiply-add.  In a scalar register it is an operand.
+__device__ __forceinline__ void horner3(double (&r)[3], const double (&y)[3], double c) {
+  asm volatile("" : "+s"(c));
+#pragma unroll
+  for (int k = 0; k < 3; ++k) r[k] = __builtin_fma(r[k], y[k], c);
+}
+
+// exp of three arguments at most 700 (below -745 it is 0; larger ones are not used): 2^n times the Taylor
+// polynomial of degree 13 in x - n log 2, |.| <= log(2) / 2, whose remainder is below 5e-18.
+__device__ __forceinline__ void exp3(const double (&x)[3], double (&e)[3]) {
+  double n[3], y[3];
+#pragma unroll
+  for (int k = 0; k < 3; ++k) {
+    const double v = fmax(x[k], -800.0);
+    n[k] = __builtin_rint(v * 1.4426950408889634);
+    y[k] = __builtin_fma(n[k], -2.3190468138462996e-17, __builtin_fma(n[k], -0.6931471805599453, v));
+    e[k] = 1.0 / 6227020800.0;
+  }
+  constexpr double kInvFact[13] = {1.0, 1.0, 1.0 / 2, 1.0 / 6, 1.0 / 24, 1.0 / 120, 1.0 / 720, 1.0 / 5040, 1.0 / 40320,
+                                   1.0 / 362880, 1.0 / 3628800, 1.0 / 39916800, 1.0 / 479001600};
+#pragma unroll
+  for (int i = 12; i >= 0; --i) horner3(e, y, kInvFact[i]);
+#pragma unroll
+  for (int k = 0; k < 3; ++k) e[k] = __builtin_ldexp(e[k], (int)n[k]);
+}
+
+__device__ __forceinline__ void erfcx3(const double (&x)[3], double (&e)[3]) {
+  double y[3], w[3];
+#pragma unroll
+  for (int k = 0; k < 3; ++k) {
+    const double v = fmin(x[k], 1e100);  // (the product below stays finite; erfcx(1e100) counts as 0 anywhere)
+    const double p = v + 3.75, q = __builtin_fma(2.0, v, 1.0), r = rcp_nr(p * q);
+    y[k] = (v - 3.75) * (q * r);
+    w[k] = p * r;
+    e[k] = kErfcx[kErfcxN - 1];
+  }
+#pragma unroll
+  for (int i = kErfcxN - 2; i >= 0; --i) horner3(e, y, kErfcx[i]);
+#pragma unroll
+  for (int k = 0; k < 3; ++k) e[k] *= w[k];
+}
+
+// What the samples of one pair's current need of it; sample k < T of a tail integrates it over the tick
+// around sample time t_k, between the boundaries g_{k+1} = -t_k - dt/2 and g_k = -t_k + dt/2 (g_j = -t_j +
+// dt/2 for j < T, g_T = -t_{T-1} - dt/2), so lane j evaluates the tail's CDF (integrated_expon_diff, with
+// diffusion) or its exponential (integrated_expon) once at g_j and each value serves two samples (the next
+// lane's by a shift).  Prepared one pair per lane, 64 pairs at a time, and handed to the wave by lane reads.
+struct PairCur {
+  double a, ne, loc;  // mix of the tails, charge, location -t0
+  double qb, qc;      // the tails' shares of the charge over a tick: a ne / dt, (1 - a) ne / dt
+  double sb, sc;      // decays
+  double r;           // 1 / (sqrt2 sigma)
+  double lb, lc;      // 1 / decay
+  double Ab, Ac;      // E = A - lambda g
+  double L, Zb, Zc;   // u = g r - L, z = Z - g r
+  double sig;
+  int o;              // waveform tick of sample 0
+  int general;        // the closed form below does not cover it (sigma 0, a decay near 0, not finite)
+};
+
+__device__ __forceinline__ PairCur pair_current(double xd, double yd, double t0, double sig, double ne, double ts, double dt,
+                                                 int T) {
+  PairCur c;
+  // detsim_jax.py:542-545, 585-588
+  const double a = 1.060 - 0.909 * xd - 0.909 * yd + 5.856 * xd * yd + 0.207 * xd * xd + 0.207 * yd * yd;
+  c.sb = 0.679 - 1.083 * xd - 1.083 * yd + 8.772 * xd * yd - 5.521 * xd * xd - 5.521 * yd * yd;
+  c.sc = 2.644 - 9.174 * xd - 9.174 * yd + 13.483 * xd * yd + 45.887 * xd * xd + 45.887 * yd * yd;
+  const double ts0 = 2.948 - 2.705 * xd - 2.705 * yd + 4.825 * xd * yd + 20.814 * xd * xd + 20.814 * yd * yd;
+  c.a = fmin(a, 1.0);
+  // t0 split into whole ticks and the remainder (detsim_jax.py:629-633)
+  const int t0_tick = (int)(t0 / ts + 0.5);
+  c.loc = -((t0 - t0_tick * ts) + ts0);
+  c.o = t0_tick - T;
+  c.ne = ne;
+  c.qb = c.a * ne / dt;
+  c.qc = (1.0 - c.a) * ne / dt;
+  c.sig = sig;
+  c.r = 1.0 / (M_SQRT2 * sig);
+  c.lb = 1.0 / c.sb;
+  c.lc = 1.0 / c.sc;
+  const double ss = sig * sig;
+  c.Ab = c.lb * (c.loc + 0.5 * c.lb * ss);
+  c.Ac = c.lc * (c.loc + 0.5 * c.lc * ss);
+  c.L = c.loc * c.r;
+  c.Zb = (c.loc + c.lb * ss) * c.r;
+  c.Zc = (c.loc + c.lc * ss) * c.r;
+  c.general = !(fabs(c.lb) < 1e8 && fabs(c.lc) < 1e8 && c.r < 1e100 && fabs(c.loc) < 1e100) ? 1 : 0;
+  return c;
+}
+
+__device__ __forceinline__ double lane_next_d(double v) {  // lane i receives lane i + 1's value
+  const int lo = __builtin_amdgcn_mov_dpp(__double2loint(v), 0x130 /* wave_shl:1 */, 0xf, 0xf, true);
+  const int hi = __builtin_amdgcn_mov_dpp(__double2hiint(v), 0x130, 0xf, 0xf, true);
+  return __hiloint2double(hi, lo);
+}
+
+// Sample k of the current times the charge of the pair that lane l prepared (k its lane's; lanes past T are
+// not samples).  The exponentially modified Gaussian's CDF minus 1/2 is F = erf(u)/2 - Y/2, u = (g - mu) r,
+// Y = exp(E) erfc(z); as E - z^2 = -u^2, Y = exp(-u^2) erfcx(z) for z >= 0 and 2 exp(E) - exp(-u^2)
+// erfcx(-z) below, and erf(u) = +-(1 - exp(-u^2) erfcx(|u|)): three exponentials and three erfcx for both
+// tails, each three sharing their coefficients.  What bounds it is the issue of these: about 200 float64 and 90
+// other vector instructions a pair, 84 % of the cycles (erf, two erfc and two exponentials, each with its own
+// quotient, took 760; 50k-segment event, 4.1 M pairs, 81 pixels an electron: the whole call 5.59 -> 3.62 ms).
+// Two pairs at a time did not pay: their lane reads run out of scalar registers.
+// Lanes whose exponential leaves (or nears) the float64 range take emg_cdf_half itself, so that what
+// overflows there overflows here, to the same infinities and NaNs.
+__device__ __forceinline__ double pair_sample(const PairCur& mine, int l, double gj, double dt, int T, bool diffusion) {
   if (!diffusion) {
-    tb = param_tail(gj, loc, sb, sigma, dt, T, false);
-    tc = param_tail(gj, loc, sc, sigma, dt, T, false);
-    return;
+    const double a = readlane_d(mine.a, l), loc = readlane_d(mine.loc, l);
+    const double sb = readlane_d(mine.sb, l), sc = readlane_d(mine.sc, l);
+    const double Gb = exp(fmin(0.0, (loc - gj) / sb)), Gc = exp(fmin(0.0, (loc - gj) / sc));
+    const double tb = (lane_next_d(Gb) - Gb + exp(fmin(0.0, (loc - dt / 2) / sb)) / T) / dt;
+    const double tc = (lane_next_d(Gc) - Gc + exp(fmin(0.0, (loc - dt / 2) / sc)) / T) / dt;
+    return (a * tb + (1 - a) * tc) * readlane_d(mine.ne, l);
   }
-  const double half = 0.5 * erf((gj - loc) / (M_SQRT2 * sigma));
-  double F[2];
-#pragma unroll
-  for (int k = 0; k < 2; ++k) {
-    const double lambd = 1.0 / (k == 0 ? sb : sc);
-    const double coeff = lambd / 2;
-    const double ex = coeff * (2 * loc + lambd * sigma * sigma - 2 * gj);
-    const double pdf = coeff * exp(ex) * erfc((loc + lambd * sigma * sigma - gj) / (M_SQRT2 * sigma));
-    F[k] = half - pdf / lambd;
+  const double gr = gj * readlane_d(mine.r, l);
+  const double u = gr - readlane_d(mine.L, l), zb = readlane_d(mine.Zb, l) - gr, zc = readlane_d(mine.Zc, l) - gr;
+  const double x[3] = {-u * u, __builtin_fma(-gj, readlane_d(mine.lb, l), readlane_d(mine.Ab, l)),
+                       __builtin_fma(-gj, readlane_d(mine.lc, l), readlane_d(mine.Ac, l))};
+  double e[3], ex[3];
+  exp3(x, ex);
+  const double z[3] = {fabs(u), fabs(zb), fabs(zc)};
+  erfcx3(z, e);
+  const double half = copysign(__builtin_fma(-ex[0], e[0], 1.0), u);
+  double Yb = ex[0] * e[1], Yc = ex[0] * e[2];
+  Yb = zb < 0 ? __builtin_fma(2.0, ex[1], -Yb) : Yb;
+  Yc = zc < 0 ? __builtin_fma(2.0, ex[2], -Yc) : Yc;
+  double Fb = half - Yb, Fc = half - Yc;  // 2 F
+  const bool general = __builtin_amdgcn_readlane(mine.general, l) || !(fmax(x[1], x[2]) <= 690.0);
+  if (__builtin_amdgcn_ballot_w64(general)) {  // (wave uniform: the lane reads need every lane's registers)
+    const double loc = readlane_d(mine.loc, l), sig = readlane_d(mine.sig, l);
+    const double lb = 1.0 / readlane_d(mine.sb, l), lc = 1.0 / readlane_d(mine.sc, l);
+    const double Gb = 2.0 * emg_cdf_half(gj, loc, sig, lb), Gc = 2.0 * emg_cdf_half(gj, loc, sig, lc);
+    Fb = general ? Gb : Fb;
+    Fc = general ? Gc : Fc;
   }
-#pragma unroll
-  for (int k = 0; k < 2; ++k) {
-    const double Fn = __shfl_down(F[k], 1, kWave);
-    const double F1 = __shfl(F[k], 1, kWave), FT = __shfl(F[k], T - 1, kWave);
-    (k == 0 ? tb : tc) = (F[k] - Fn) / (F1 - FT) / dt;
-  }
+  const double db = readlane_d(Fb, 1) - readlane_d(Fb, T - 1), dc = readlane_d(Fc, 1) - readlane_d(Fc, T - 1);
+  double ib = rcp_nr(db), ic = rcp_nr(dc);
+  if (__builtin_amdgcn_readfirstlane(!(fmin(db, dc) > 1e-280))) ib = 1.0 / db, ic = 1.0 / dc;
+  return (Fb - lane_next_d(Fb)) * ib * readlane_d(mine.qb, l) + (Fc - lane_next_d(Fc)) * ic * readlane_d(mine.qc, l);
 }
 
 // One workgroup per row (sorted unique pixel id upix[r]): the pairs order[offs[r] .. offs[r+1]) in
@@ -180,26 +317,20 @@ __global__ __launch_bounds__(kParamWaves* kWave) void k_param_rows(Dev d, ParamE
     const double tk = kk == T - 1 ? 5.0 : (double)kk * dt;  // linspace(0, 5, T)
     const double gj = lane < T ? -tk + dt / 2 : -5.0 - dt / 2;  // tick boundaries (lane T: the last)
     const int b0 = offs[r], b1 = offs[r + 1];
-    for (int i = b0 + wid; i < b1; i += kParamWaves) {
-      const int pr = order[i];
-      const int64_t el = pr / K;
-      const double xd = fabs(e.x[el] - cx), yd = fabs(e.y[el] - cy);
-      // detsim_jax.py:542-545, 585-588
-      double a = 1.060 - 0.909 * xd - 0.909 * yd + 5.856 * xd * yd + 0.207 * xd * xd + 0.207 * yd * yd;
-      const double b = 0.679 - 1.083 * xd - 1.083 * yd + 8.772 * xd * yd - 5.521 * xd * xd - 5.521 * yd * yd;
-      const double c = 2.644 - 9.174 * xd - 9.174 * yd + 13.483 * xd * yd + 45.887 * xd * xd + 45.887 * yd * yd;
-      const double ts0 = 2.948 - 2.705 * xd - 2.705 * yd + 4.825 * xd * yd + 20.814 * xd * xd + 20.814 * yd * yd;
-      a = fmin(a, 1.0);
-      // t0 split into whole ticks and the remainder (detsim_jax.py:629-633)
-      const double t0 = e.t0[el];
-      const int t0_tick = (int)(t0 / d.ts + 0.5);
-      const double st0 = (t0 - t0_tick * d.ts) + ts0;
-      const double sig = e.sig[el];
-      double tlb, tlc;
-      param_tails(gj, -st0, b, c, sig, dt, T, diffusion != 0, tlb, tlc);
-      const double cur = a * tlb + (1 - a) * tlc;
-      const int o = t0_tick - T + kk;
-      if (lane < T && o >= 0 && o < nout) acc[wid][o] += cur * e.ne[el];
+    // lane l prepares pair i0 + kParamWaves l + wid; the wave then takes them in order
+    for (int i0 = b0; i0 < b1; i0 += kParamWaves * kWave) {
+      const int i = i0 + lane * kParamWaves + wid;
+      PairCur mine = {};
+      if (i < b1) {
+        const int el = order[i] / K;
+        mine = pair_current(fabs(e.x[el] - cx), fabs(e.y[el] - cy), e.t0[el], e.sig[el], e.ne[el], d.ts, dt, T);
+      }
+      const int n = __builtin_amdgcn_readfirstlane((b1 - i0 - wid + kParamWaves - 1) / kParamWaves);
+      for (int l = 0; l < n && l < kWave; ++l) {
+        const int o = __builtin_amdgcn_readlane(mine.o, l) + kk;
+        const double cur = pair_sample(mine, l, gj, dt, T, diffusion != 0);
+        if (lane < T && o >= 0 && o < nout) acc[wid][o] += cur;
+      }
     }
   }
   __syncthreads();
@@ -294,7 +425,7 @@ __global__ void k_param_adj_electrons(Dev d, SegIn in, int mode, int diffusion, 
   }
 }
 
-// One tail of a pair's current at sample k (param_tail) and its partial derivatives in the
+// One tail of a pair's current at sample k and its partial derivatives in the
 // tail's location, decay constant and longitudinal spread.  With diffusion the tail is
 // (F_k - F_{k+1}) / (F_1 - F_{T-1}) / dt of H(g) = 1/2 erf(u) - P, u = (g - mu) / (sqrt2 sigma),
 // P = 1/2 exp(E) erfc(z), E = lambda (mu - g) + lambda^2 sigma^2 / 2,
