@@ -29,14 +29,17 @@ struct RbfAcc {
 template <int D>
 __device__ __forceinline__ void rbf_span(const float4& p, const float4* __restrict__ y, const float4* __restrict__ c,
                                          int ja, int jb, float inv_l2, RbfAcc& a) {
+  // (constant address space: the loads of a wave-uniform index stay scalar behind a barrier too)
+  using Const4 = const __attribute__((address_space(4))) float __attribute__((ext_vector_type(4)));
+  const Const4* yq = (const Const4*)(uintptr_t)y;
+  const Const4* cq = (const Const4*)(uintptr_t)c;
   // the lanes walking a span share its run position: keep it (and so the loop) wave-uniform
   int run = __builtin_amdgcn_readfirstlane(a.run);
   while (ja < jb) {
     const int n = jb - ja < kRbfRun - run ? jb - ja : kRbfRun - run;
 #pragma unroll 4
     for (int u = 0; u < n; ++u) {
-      const float4 q = y[ja + u];
-      const float4 w = c[ja + u];
+      const auto q = yq[ja + u], w = cq[ja + u];
       const float dx = p.x - q.x, dy = p.y - q.y, dz = p.z - q.z;
       float d2 = dx * dx + dy * dy + dz * dz;
       if (D == 4) {
@@ -135,14 +138,25 @@ __device__ __forceinline__ float wave_max_f(float v) {
   return __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(v)));
 }
 
+// A workgroup holds 64 queries, the same in each of its kRbfWaves waves, which share their candidates: thread
+// t finds the span of column b0 + t, a scan of the spans' lengths joins them into one list, and wave w walks
+// the w-th part of it.  One wave to 64 queries left most of the chip idle and waited for the wave with the
+// longest list (both sums of a 20k-segment fit step: 1188 -> 188 us); a fixed split keeps the order of the sums.
+// A pair costs 11 float32 instructions and an exponential, which now bound it; y and c come by scalar loads.
+constexpr int kRbfWaves = 8;
+constexpr int kRbfCols = kRbfWaves * kWave;
+
 template <int D>
-__global__ __launch_bounds__(256) void k_rbf_grid(const float4* __restrict__ x, const int32_t* __restrict__ ev, int64_t nx,
-                                                  const float4* __restrict__ y, const float4* __restrict__ c,
-                                                  const int64_t* __restrict__ ykey, int32_t ny,
-                                                  const float* __restrict__ grid, float inv, float rc,
-                                                  double* __restrict__ out) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  const int lane = threadIdx.x & (kWave - 1);
+__global__ __launch_bounds__(kRbfCols) void k_rbf_grid(const float4* __restrict__ x, const int32_t* __restrict__ ev,
+                                                       int64_t nx, const float4* __restrict__ y,
+                                                       const float4* __restrict__ c, const int64_t* __restrict__ ykey,
+                                                       int32_t ny, const float* __restrict__ grid, float inv, float rc,
+                                                       double* __restrict__ out) {
+  __shared__ int s_start[kRbfCols], s_end[kRbfCols];  // a column's candidates; their end in the joined list
+  __shared__ int s_tot[kRbfWaves];
+  __shared__ double s_sum[kRbfWaves][4][kWave];
+  const int t = threadIdx.x, lane = t & (kWave - 1), wid = __builtin_amdgcn_readfirstlane(t / kWave);
+  const int64_t i = (int64_t)blockIdx.x * kWave + lane;
   const bool valid = i < nx;
   const float4 p = valid ? x[i] : make_float4(0.f, 0.f, 0.f, 0.f);
   const int my_ev = valid ? ev[i] : 0;
@@ -151,7 +165,7 @@ __global__ __launch_bounds__(256) void k_rbf_grid(const float4* __restrict__ x, 
   const float inf = __builtin_inff();
   RbfAcc a = {0.0, 0.0, 0.0, 0.0, 0.f, 0.f, 0.f, 0.f, 0};
   bool pending = valid;
-  for (uint64_t pm = __ballot(pending); pm != 0; pm = __ballot(pending)) {
+  for (uint64_t pm = __ballot(pending); pm != 0; pm = __ballot(pending)) {  // (alike in every wave)
     const int e = __builtin_amdgcn_readlane(my_ev, __builtin_ctzll(pm));
     const bool mine = pending && my_ev == e;
     const float bx0 = wave_min_f(mine ? p.x : inf), bx1 = wave_max_f(mine ? p.x : -inf);
@@ -160,10 +174,10 @@ __global__ __launch_bounds__(256) void k_rbf_grid(const float4* __restrict__ x, 
     const int cxa = rbf_cell(bx0 - rc, lox, hx, Gx), cxb = rbf_cell(bx1 + rc, lox, hx, Gx);
     const int cya = rbf_cell(by0 - rc, loy, hy, Gy), cyb = rbf_cell(by1 + rc, loy, hy, Gy);
     const int ncy = cyb - cya + 1, ncol = cxb < cxa || cyb < cya ? 0 : (cxb - cxa + 1) * ncy;
-    for (int b0 = 0; b0 < ncol; b0 += kWave) {
-      // lane l finds the candidate span of column b0 + l
+    for (int b0 = 0; b0 < ncol; b0 += kRbfCols) {
+      // this thread's column, and where its candidates end in its wave's part of the list
       int j0 = 0, j1 = 0;
-      const int col = b0 + lane;
+      const int col = b0 + t;
       if (col < ncol) {
         const int cx = cxa + col / ncy, cy = cya + col % ncy;
         const float gx = rbf_gap(cx, bx0, bx1, lox, hx, Gx), gy = rbf_gap(cy, by0, by1, loy, hy, Gy);
@@ -176,15 +190,51 @@ __global__ __launch_bounds__(256) void k_rbf_grid(const float4* __restrict__ x, 
           j1 = rbf_lower_bound(ykey, ny, kb + czb + 1);
         }
       }
-      const int nc = ncol - b0 < kWave ? ncol - b0 : kWave;
-      for (int cc = 0; cc < nc; ++cc) {
-        const int ja = __builtin_amdgcn_readlane(j0, cc), jb = __builtin_amdgcn_readlane(j1, cc);
-        if (mine) rbf_span<D>(p, y, c, ja, jb, inv * kLog2e, a);
+      int n = j1 - j0;
+#pragma unroll
+      for (int m = 1; m < kWave; m <<= 1) {
+        const int v = __shfl_up(n, m, kWave);
+        if (lane >= m) n += v;
+      }
+      __syncthreads();  // (the list of the round before has been walked)
+      s_start[t] = j0;
+      s_end[t] = n;
+      if (lane == kWave - 1) s_tot[wid] = n;
+      __syncthreads();
+      int tot = 0;
+      for (int w = 0; w < kRbfWaves; ++w) tot += __builtin_amdgcn_readfirstlane(s_tot[w]);
+      // positions la .. lb - 1 of the joined list are this wave's
+      const int la = (int)((int64_t)tot * wid / kRbfWaves), lb = (int)((int64_t)tot * (wid + 1) / kRbfWaves);
+      for (int w = 0, wa = 0, we = 0; w < kRbfWaves && wa < lb; ++w, wa = we) {
+        we = wa + __builtin_amdgcn_readfirstlane(s_tot[w]);
+        if (we <= la) continue;  // (none of this wave's among these 64 columns)
+        const int q1 = s_end[w * kWave + lane], qs = s_start[w * kWave + lane];
+        const int up = __shfl_up(q1, 1, kWave);
+        const int q0 = lane == 0 ? 0 : up;
+        const int k0 = max(la - wa, q0), k1 = min(lb - wa, q1);  // this column's part of this wave's list
+        const int ja = qs + (k0 - q0), jb = qs + (k1 - q0);
+        for (uint64_t m = __ballot(k0 < k1); m != 0; m &= m - 1) {
+          const int cc = __builtin_ctzll(m);
+          const int ua = __builtin_amdgcn_readlane(ja, cc), ub = __builtin_amdgcn_readlane(jb, cc);
+          if (mine) rbf_span<D>(p, y, c, ua, ub, inv * kLog2e, a);
+        }
       }
     }
     pending = pending && !mine;
   }
-  if (valid) rbf_store(a, out + i * 4);
+  s_sum[wid][0][lane] = a.s0 + (double)a.f0;
+  s_sum[wid][1][lane] = a.s1 + (double)a.f1;
+  s_sum[wid][2][lane] = a.s2 + (double)a.f2;
+  s_sum[wid][3][lane] = a.s3 + (double)a.f3;
+  __syncthreads();
+  // thread t < 256: column t % 4 of query t / 4
+  const int64_t o = (int64_t)blockIdx.x * kWave + t / 4;
+  if (t < 4 * kWave && o < nx) {
+    double v = 0.0;
+#pragma unroll
+    for (int w = 0; w < kRbfWaves; ++w) v += s_sum[w][t % 4][t / 4];
+    out[o * 4 + t % 4] = v;
+  }
 }
 
 // Event-blocked nearest neighbour for the chamfer loss (losses_jax.py:195-229

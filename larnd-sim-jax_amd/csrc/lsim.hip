@@ -1053,12 +1053,12 @@ int lsim_rbf_sums_grid(const float* x, const int32_t* x_event, int64_t nx, const
   if (!x || !x_event || !grid || !out || (ny > 0 && (!y || !c || !y_key))) return fail(LSIM_E_ARG, "NULL argument");
   const float inv = 1.f / (2.f * sigma * sigma);
   const float rc = lsim_rbf_cull_radius(sigma);
-  const dim3 g((unsigned)((nx + 255) / 256));
+  const dim3 g((unsigned)((nx + kWave - 1) / kWave));
   if (dims == 3)
-    hipLaunchKernelGGL(k_rbf_grid<3>, g, dim3(256), 0, (hipStream_t)stream, (const float4*)x, x_event, nx,
+    hipLaunchKernelGGL(k_rbf_grid<3>, g, dim3(kRbfCols), 0, (hipStream_t)stream, (const float4*)x, x_event, nx,
                        (const float4*)y, (const float4*)c, y_key, (int32_t)ny, grid, inv, rc, out);
   else
-    hipLaunchKernelGGL(k_rbf_grid<4>, g, dim3(256), 0, (hipStream_t)stream, (const float4*)x, x_event, nx,
+    hipLaunchKernelGGL(k_rbf_grid<4>, g, dim3(kRbfCols), 0, (hipStream_t)stream, (const float4*)x, x_event, nx,
                        (const float4*)y, (const float4*)c, y_key, (int32_t)ny, grid, inv, rc, out);
   HIP_TRY(hipGetLastError());
   return LSIM_OK;
