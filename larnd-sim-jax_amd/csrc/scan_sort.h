@@ -147,108 +147,265 @@ inline hipError_t exclusive_scan(const T* in, T* out, int64_t n, T* tmp, TT* tot
 }
 
 // ------------------------------------------------------------------------------------------
-// stable LSD radix sort, 8-bit digits, tiles of 2048 items (256 threads x 8 rounds)
+// stable LSD radix sort, 8-bit digits
 // ------------------------------------------------------------------------------------------
+//
+// Every wave owns 64 R consecutive items and ranks them by itself (ballots give the peers of a digit, a
+// per-wave counter in LDS carries over its R rounds), so a tile costs a fixed few barriers whatever R is.
+// Three sizes, each bound by the latency of its steps rather than by the 16 bytes an item moves per pass:
+//   n <= 4096            all passes in one workgroup with the items in LDS: one launch instead of 3 a pass
+//                        (1k segments: FIGA);
+//   n <= 256 tiles of 8  two launches a pass, R = 1 .. 8 such that there are at most 256 tiles (many small
+//                        tiles in flight); a tile sums the histograms of those before it as it starts
+//                        (256 KB from L2 at most), which saves the scan's one to three launches
+//                        (200k segments: FIGB);
+//   above                histogram, device-wide scan, scatter (that sum would grow as the square of n).
 
 constexpr int kSortThreads = 256;
-constexpr int kSortRounds = 8;
+constexpr int kSortWaves = kSortThreads / kWave;
+constexpr int kSortRounds = 8;  // the most
 constexpr int kSortTile = kSortThreads * kSortRounds;
 constexpr int kRadix = 256;
+constexpr int kSortSumTiles = 256;
+constexpr int kSumBatch = 32;
+constexpr int kSmallThreads = 1024;
+constexpr int kSmallRounds = 4;
+constexpr int kSmallMax = kSmallThreads * kSmallRounds;
 
-__global__ __launch_bounds__(kSortThreads) void k_radix_hist(const uint32_t* __restrict__ keys, int64_t n, int shift,
-                                                             int ntiles, int* __restrict__ hist) {
-  __shared__ int h[kRadix];
-  h[threadIdx.x] = 0;
-  __syncthreads();
-  const int64_t base = (int64_t)blockIdx.x * kSortTile;
-  for (int r = 0; r < kSortRounds; ++r) {
-    const int64_t i = base + r * kSortThreads + threadIdx.x;
-    if (i < n) atomicAdd(&h[(keys[i] >> shift) & (kRadix - 1)], 1);
-  }
-  __syncthreads();
-  hist[(int64_t)threadIdx.x * ntiles + blockIdx.x] = h[threadIdx.x];
-}
+__device__ __forceinline__ int radix_digit(uint32_t key, int shift) { return (key >> shift) & (kRadix - 1); }
 
-// Scatter with stable ranks: items are ranked in index order (round by round, lane order within
-// a round), so equal digits keep their input order.
-__global__ __launch_bounds__(kSortThreads) void k_radix_scatter(const uint32_t* __restrict__ kin,
-                                                                const uint32_t* __restrict__ vin,
-                                                                uint32_t* __restrict__ kout,
-                                                                uint32_t* __restrict__ vout, int64_t n, int shift,
-                                                                int ntiles, const int* __restrict__ offs) {
-  constexpr int NW = kSortThreads / kWave;
-  __shared__ int base[kRadix];
-  __shared__ int wcnt[NW][kRadix];
-  const int lane = threadIdx.x & (kWave - 1), wid = threadIdx.x / kWave;
-  base[threadIdx.x] = offs[(int64_t)threadIdx.x * ntiles + blockIdx.x];
+// Ranks of a wave's items (item r of lane l is the (64 r + l)-th) among its items of the same digit;
+// cnt[digit] (this wave's, zero before) ends as the digit's count.
+template <int R>
+__device__ __forceinline__ void radix_rank(const uint32_t (&key)[R], const bool (&valid)[R], int shift, int* cnt,
+                                           int (&rank)[R]) {
+  const int lane = threadIdx.x & (kWave - 1);
   const uint64_t lt = (lane == 0) ? 0ull : ((~0ull) >> (64 - lane));
-  const int64_t tile0 = (int64_t)blockIdx.x * kSortTile;
-  for (int r = 0; r < kSortRounds; ++r) {
 #pragma unroll
-    for (int w = 0; w < NW; ++w) wcnt[w][threadIdx.x] = 0;
-    __syncthreads();
-    const int64_t i = tile0 + r * kSortThreads + threadIdx.x;
-    const bool valid = i < n;
-    uint32_t key = 0, val = 0;
-    int dg = 0;
-    if (valid) {
-      key = kin[i];
-      val = vin[i];
-      dg = (key >> shift) & (kRadix - 1);
-    }
-    uint64_t peers = __ballot(valid);
+  for (int r = 0; r < R; ++r) {
+    const int dg = radix_digit(key[r], shift);
+    uint64_t peers = __ballot(valid[r]);
 #pragma unroll
     for (int b = 0; b < 8; ++b) {
       const bool bit = (dg >> b) & 1;
       const uint64_t bb = __ballot(bit);
       peers &= bit ? bb : ~bb;
     }
-    const int rank_w = __popcll(peers & lt);
-    if (valid && rank_w == 0) wcnt[wid][dg] = __popcll(peers);
-    __syncthreads();
-    if (valid) {
-      int pos = base[dg] + rank_w;
-      for (int w = 0; w < wid; ++w) pos += wcnt[w][dg];
-      kout[pos] = key;
-      vout[pos] = val;
-    }
-    __syncthreads();
-    int add = 0;
-#pragma unroll
-    for (int w = 0; w < NW; ++w) add += wcnt[w][threadIdx.x];
-    base[threadIdx.x] += add;
-    __syncthreads();
+    const int below = __popcll(peers & lt);
+    const int before = valid[r] ? cnt[dg] : 0;
+    __builtin_amdgcn_wave_barrier();
+    if (valid[r] && below == 0) cnt[dg] = before + __popcll(peers);
+    __builtin_amdgcn_wave_barrier();
+    rank[r] = before + below;
   }
 }
 
-inline int sort_tiles(int64_t n) { return (int)((n + kSortTile - 1) / kSortTile); }
+// hist[digit * dstride + tile * tstride] = the tile's count of the digit
+template <int R>
+__global__ __launch_bounds__(kSortThreads) void k_radix_hist(const uint32_t* __restrict__ keys, int64_t n, int shift,
+                                                             int64_t dstride, int64_t tstride, int* __restrict__ hist) {
+  __shared__ int h[kRadix];
+  h[threadIdx.x] = 0;
+  __syncthreads();
+  const int64_t base = (int64_t)blockIdx.x * (kSortThreads * R);
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    const int64_t i = base + r * kSortThreads + threadIdx.x;
+    if (i < n) atomicAdd(&h[radix_digit(keys[i], shift)], 1);
+  }
+  __syncthreads();
+  hist[threadIdx.x * dstride + blockIdx.x * tstride] = h[threadIdx.x];
+}
 
-// Bytes of scratch the sort needs for n items (histogram + scan tiles).
+// SUM: `hist` holds the tiles' histograms ([tile][digit]) and this tile derives its digits' first
+// positions from them; otherwise the scanned ones ([digit][tile]).
+template <int R, bool SUM>
+__global__ __launch_bounds__(kSortThreads) void k_radix_scatter(const uint32_t* __restrict__ kin,
+                                                                const uint32_t* __restrict__ vin,
+                                                                uint32_t* __restrict__ kout,
+                                                                uint32_t* __restrict__ vout, int64_t n, int shift,
+                                                                int ntiles, const int* __restrict__ hist) {
+  __shared__ int cnt[kSortWaves][kRadix];
+  __shared__ int s_scan[kSortWaves];
+  const int t = threadIdx.x, lane = t & (kWave - 1), wid = t / kWave;
+  const int64_t i0 = (int64_t)blockIdx.x * (kSortThreads * R) + wid * (kWave * R) + lane;
+  uint32_t key[R], val[R];
+  bool valid[R];
+  int rank[R];
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    valid[r] = i0 + r * kWave < n;
+    key[r] = valid[r] ? kin[i0 + r * kWave] : 0;
+    val[r] = valid[r] ? vin[i0 + r * kWave] : 0;
+  }
+#pragma unroll
+  for (int w = 0; w < kSortWaves; ++w) cnt[w][t] = 0;
+  __syncthreads();
+  radix_rank<R>(key, valid, shift, cnt[wid], rank);
+  int base;
+  if (SUM) {
+    int before = 0, total = 0;
+    const int me = blockIdx.x;
+    for (int t0 = 0; t0 < ntiles; t0 += kSumBatch) {  // (a batch's loads in flight together)
+      int v[kSumBatch];
+#pragma unroll
+      for (int k = 0; k < kSumBatch; ++k) v[k] = hist[min(t0 + k, ntiles - 1) * kRadix + t];
+#pragma unroll
+      for (int k = 0; k < kSumBatch; ++k) {
+        total += t0 + k < ntiles ? v[k] : 0;
+        before += t0 + k < me ? v[k] : 0;
+      }
+    }
+    int tot;
+    base = block_exclusive_scan<int>(total, s_scan, tot) + before;
+  } else {
+    base = hist[(int64_t)t * ntiles + blockIdx.x];
+  }
+  __syncthreads();
+  // (thread t: the first positions of digit t in each wave)
+#pragma unroll
+  for (int w = 0; w < kSortWaves; ++w) {
+    const int c = cnt[w][t];
+    cnt[w][t] = base;
+    base += c;
+  }
+  __syncthreads();
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    if (valid[r]) {
+      const int pos = cnt[wid][radix_digit(key[r], shift)] + rank[r];
+      kout[pos] = key[r];
+      vout[pos] = val[r];
+    }
+  }
+}
+
+// All passes over n <= kSmallMax items in one workgroup.
+__global__ __launch_bounds__(kSmallThreads) void k_radix_small(const uint32_t* kin, const uint32_t* vin,
+                                                               uint32_t* kout, uint32_t* vout,  // may equal kin, vin
+                                                               int n, int bits) {
+  constexpr int NW = kSmallThreads / kWave, R = kSmallRounds;
+  __shared__ uint32_t s_key[kSmallMax], s_val[kSmallMax];
+  __shared__ int cnt[NW][kRadix];
+  __shared__ int s_scan[NW];
+  const int t = threadIdx.x, lane = t & (kWave - 1), wid = t / kWave;
+  const int i0 = wid * (kWave * R) + lane;
+  uint32_t key[R], val[R];
+  bool valid[R];
+  int rank[R];
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    valid[r] = i0 + r * kWave < n;
+    key[r] = valid[r] ? kin[i0 + r * kWave] : 0;
+    val[r] = valid[r] ? vin[i0 + r * kWave] : 0;
+  }
+  for (int shift = 0; shift < bits; shift += 8) {
+#pragma unroll
+    for (int k = 0; k < NW * kRadix / kSmallThreads; ++k) (&cnt[0][0])[k * kSmallThreads + t] = 0;
+    __syncthreads();  // (and the pass before has been read back)
+    radix_rank<R>(key, valid, shift, cnt[wid], rank);
+    __syncthreads();
+    int total = 0;
+    if (t < kRadix) {
+#pragma unroll
+      for (int w = 0; w < NW; ++w) total += cnt[w][t];
+    }
+    int tot;
+    int base = block_exclusive_scan<int>(total, s_scan, tot);
+    if (t < kRadix) {
+#pragma unroll
+      for (int w = 0; w < NW; ++w) {
+        const int c = cnt[w][t];
+        cnt[w][t] = base;
+        base += c;
+      }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      if (valid[r]) {
+        const int pos = cnt[wid][radix_digit(key[r], shift)] + rank[r];
+        s_key[pos] = key[r];
+        s_val[pos] = val[r];
+      }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      if (valid[r]) {
+        key[r] = s_key[i0 + r * kWave];
+        val[r] = s_val[i0 + r * kWave];
+      }
+    }
+  }
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    if (valid[r]) {
+      kout[i0 + r * kWave] = key[r];
+      vout[i0 + r * kWave] = val[r];
+    }
+  }
+}
+
+inline int sort_tiles(int64_t n, int rounds) { return (int)((n + (int64_t)kSortThreads * rounds - 1) / (kSortThreads * rounds)); }
+
+// Rounds of a tile for n items: the fewest that leave no more than kSortSumTiles tiles.
+inline int sort_rounds(int64_t n) {
+  int r = 1;
+  while (r < kSortRounds && sort_tiles(n, r) > kSortSumTiles) r *= 2;
+  return r;
+}
+
+// Bytes of scratch the sort of up to n items needs (histogram + scan tiles).
 inline size_t radix_sort_scratch(int64_t n) {
-  const int64_t nt = sort_tiles(n);
+  int64_t nt = sort_tiles(n, sort_rounds(n));
+  const int64_t fine = (n + kSortThreads - 1) / kSortThreads;  // (fewer items may have more, smaller tiles)
+  if (nt < kSortSumTiles) nt = fine < kSortSumTiles ? fine : kSortSumTiles;
   const int64_t hist = nt * kRadix;
   return (size_t)(hist + scan_tiles(hist) + 4) * sizeof(int);
 }
 
-// Sort (keys, vals) by the low `bits` bits of the key.  Ping-pongs between (k0, v0) and
-// (k1, v1); returns the buffer index (0 or 1) holding the result.
+template <int R>
+inline hipError_t radix_pass(const uint32_t* ki, const uint32_t* vi, uint32_t* ko, uint32_t* vo, int64_t n, int shift,
+                             int* hist, hipStream_t st) {
+  const int nt = sort_tiles(n, R);
+  if (nt <= kSortSumTiles) {
+    hipLaunchKernelGGL(k_radix_hist<R>, dim3(nt), dim3(kSortThreads), 0, st, ki, n, shift, (int64_t)1, (int64_t)kRadix, hist);
+    hipLaunchKernelGGL((k_radix_scatter<R, true>), dim3(nt), dim3(kSortThreads), 0, st, ki, vi, ko, vo, n, shift, nt, hist);
+    return hipSuccess;
+  }
+  hipLaunchKernelGGL(k_radix_hist<R>, dim3(nt), dim3(kSortThreads), 0, st, ki, n, shift, (int64_t)nt, (int64_t)1, hist);
+  const hipError_t err = exclusive_scan<int, int>(hist, hist, (int64_t)nt * kRadix, hist + (int64_t)nt * kRadix, (int*)nullptr, st);
+  if (err != hipSuccess) return err;
+  hipLaunchKernelGGL((k_radix_scatter<R, false>), dim3(nt), dim3(kSortThreads), 0, st, ki, vi, ko, vo, n, shift, nt, hist);
+  return hipSuccess;
+}
+
+// Sort (keys, vals) by the low `bits` bits of the key.  Ping-pongs between (k0, v0) and (k1, v1); returns
+// the buffer index (0 or 1) holding the result: the parity of the passes, whatever n is.
 inline int radix_sort_pairs(uint32_t* k0, uint32_t* v0, uint32_t* k1, uint32_t* v1, int64_t n, int bits, void* scratch,
                             hipStream_t st, hipError_t* err) {
-  const int nt = sort_tiles(n);
   int* hist = (int*)scratch;
-  int* tmp = hist + (int64_t)nt * kRadix;
   int cur = 0;
   *err = hipSuccess;
   if (n == 0) return 0;
+  if (n <= kSmallMax) {
+    const int odd = ((bits + 7) / 8) & 1;
+    hipLaunchKernelGGL(k_radix_small, dim3(1), dim3(kSmallThreads), 0, st, k0, v0, odd ? k1 : k0, odd ? v1 : v0, (int)n, bits);
+    *err = hipGetLastError();
+    return odd;
+  }
+  const int R = sort_rounds(n);
   for (int shift = 0; shift < bits; shift += 8) {
     uint32_t* ki = cur ? k1 : k0;
     uint32_t* vi = cur ? v1 : v0;
     uint32_t* ko = cur ? k0 : k1;
     uint32_t* vo = cur ? v0 : v1;
-    hipLaunchKernelGGL(k_radix_hist, dim3(nt), dim3(kSortThreads), 0, st, ki, n, shift, nt, hist);
-    *err = exclusive_scan<int, int>(hist, hist, (int64_t)nt * kRadix, tmp, (int*)nullptr, st);
+    *err = R == 1   ? radix_pass<1>(ki, vi, ko, vo, n, shift, hist, st)
+           : R == 2 ? radix_pass<2>(ki, vi, ko, vo, n, shift, hist, st)
+           : R == 4 ? radix_pass<4>(ki, vi, ko, vo, n, shift, hist, st)
+                    : radix_pass<8>(ki, vi, ko, vo, n, shift, hist, st);
     if (*err != hipSuccess) return cur;
-    hipLaunchKernelGGL(k_radix_scatter, dim3(nt), dim3(kSortThreads), 0, st, ki, vi, ko, vo, n, shift, nt, hist);
     cur ^= 1;
   }
   *err = hipGetLastError();
