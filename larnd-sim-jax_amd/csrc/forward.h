@@ -116,11 +116,14 @@ __global__ void k_cell_keys(Dev d, SegIn in, const uint32_t* __restrict__ vals, 
 constexpr int kCorrBatch = 9;
 constexpr int kRecThreads = 256;
 
+//
+// part < 0: all of a segment's corrections.  Otherwise a share of them: part p < parts - 1 batch p without
+// the entries of |a|, |b| <= 1, part parts - 1 those and the diffusion bins.
 template <int NB>
 __device__ __forceinline__ void seg_corrections(const Dev& d, const float2* __restrict__ DNS, const float2* __restrict__ DM,
                                                 const SegRec& R, bool live, int ux, int uy, int64_t i, int64_t n,
                                                 float2* __restrict__ stage, int* __restrict__ base,
-                                                float* __restrict__ dtot) {
+                                                float* __restrict__ dtot, int part, int parts) {
   constexpr int SYM = (NB - 1) / 2;
   const int W = 2 * d.ne + 1, WW = W * W, nsb = d.nsb, cm = d.cm;
   const int lane = threadIdx.x & (kWave - 1);
@@ -130,7 +133,11 @@ __device__ __forceinline__ void seg_corrections(const Dev& d, const float2* __re
   __builtin_amdgcn_wave_barrier();
   float dn[9];  // entries (a, b) in [-1, 1]^2, index (a + 1) * 3 + (b + 1)
   // stripe terms of every entry
-  for (int ab0 = 0; ab0 < WW; ab0 += kCorrBatch) {
+  const bool near = part < 0 || part == parts - 1, far = part < 0 || !near;
+  // (the near entries lie between (-1, -1) and (1, 1))
+  const int first = part < 0 ? 0 : (near ? (d.ne - 1) * W + d.ne - 1 : part * kCorrBatch);
+  const int last = part < 0 ? WW : (near ? (d.ne + 1) * W + d.ne + 2 : first + 1);
+  for (int ab0 = first; ab0 < last; ab0 += kCorrBatch) {
 #pragma unroll
     for (int m = 0; m < kCorrBatch; ++m) {
       const int e = lane + kWave * m;
@@ -169,12 +176,12 @@ __device__ __forceinline__ void seg_corrections(const Dev& d, const float2* __re
 #pragma unroll
         for (int e = 0; e < 9; ++e)
           if (e == (a + 1) * 3 + (b + 1)) dn[e] = delta;
-      } else {
+      } else if (far) {
         dtot[(int64_t)ab * n + i] = delta;
       }
     }
   }
-  if (!live) return;
+  if (!live || !near) return;
   const float2* DMk = DM + ((int64_t)R.k0 * d.nm + R.idx) * cm * cm;
   // diffusion bins of the idx template, one x-bin row of loads at a time
 #pragma unroll
@@ -210,14 +217,12 @@ __device__ __forceinline__ void seg_corrections(const Dev& d, const float2* __re
   }
 }
 
-// The record of the segment with input index src at sorted position i, and its pair record.
+// The record of the segment with input index src at sorted position i, and its pair record; whole = false
+// leaves out what only the diffusion bins need (their weights) and writes neither.
 __device__ __forceinline__ void record(const Dev& d, const SegIn& in, int64_t src, int64_t i, SegRec& r, int& ux, int& uy,
-                                       SegRec* __restrict__ rec, PairRec* __restrict__ prs) {
+                                       SegRec* __restrict__ rec, PairRec* __restrict__ prs, bool whole) {
   Phys ph;
   seg_physics(d, in, src, ph);
-  double wx[kMaxNb], wy[kMaxNb];
-  tran_weights(d, ph.x0, ph.st, wx, nullptr);
-  tran_weights(d, ph.y0, ph.st, wy, nullptr);
   r.bx = ph.bx;
   r.by = ph.by;
   r.k0 = ph.k0;
@@ -227,14 +232,18 @@ __device__ __forceinline__ void record(const Dev& d, const SegIn& in, int64_t sr
   r.la = (float)ph.la;
   r.lb = (float)ph.lb;
   r.lc = (float)ph.lc;
+  ux = pymod_i(ph.bx, d.nsb);
+  uy = pymod_i(ph.by, d.nsb);
+  r.uxy = ux | (uy << 16);
+  if (!whole) return;
+  double wx[kMaxNb], wy[kMaxNb];
+  tran_weights(d, ph.x0, ph.st, wx, nullptr);
+  tran_weights(d, ph.y0, ph.st, wy, nullptr);
 #pragma unroll
   for (int k = 0; k < kMaxNb; ++k) {
     r.wx[k] = k < d.nb ? (float)wx[k] : 0.f;
     r.wy[k] = k < d.nb ? (float)wy[k] : 0.f;
   }
-  ux = pymod_i(ph.bx, d.nsb);
-  uy = pymod_i(ph.by, d.nsb);
-  r.uxy = ux | (uy << 16);
   rec[i] = r;
   PairRec P;
   P.S = d.nt - d.L - ph.k0;
@@ -259,8 +268,18 @@ __global__ __launch_bounds__(kRecThreads) void k_records(Dev d, SegIn in, const 
   const bool live = i < n && keys[i] < (uint32_t)d.n_cells;
   SegRec r = {};
   int ux = 0, uy = 0;
-  if (live) record(d, in, vals[i], i, r, ux, uy, rec, prs);
-  seg_corrections<NB>(d, DNS, DM, r, live, ux, uy, i, n, stage[wid], sbase[wid], dtot);
+  const int parts = gridDim.y, part = parts == 1 ? -1 : (int)blockIdx.y;
+  if (live) record(d, in, vals[i], i, r, ux, uy, rec, prs, part < 0 || part == parts - 1);
+  seg_corrections<NB>(d, DNS, DM, r, live, ux, uy, i, n, stage[wid], sbase[wid], dtot, part, parts);
+}
+
+// Parts of k_records for n segments.  A segment's batches are a chain of loads of 3 to 5 us each; with few
+// segments waves of their own take it apart, at the price of the segment's physics in each (whole / parts:
+// 1k segments 48 / 30 us, 30k 65 / 47, 50k 82 / 61, 200k 103 / 153).
+constexpr int64_t kRecSplitMax = 65536;
+inline int rec_parts(const Dev& d, int64_t n) {
+  const int W = 2 * d.ne + 1;
+  return n <= kRecSplitMax ? (W * W + kCorrBatch - 1) / kCorrBatch + 1 : 1;
 }
 
 // Cell ranges [begin, end) in the sorted order and the "first segment of an on-plane cell" flag

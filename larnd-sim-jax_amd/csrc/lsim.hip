@@ -538,11 +538,11 @@ int lsim_forward_prepare(lsim_ctx* c, const lsim_params* p, const lsim_segments*
     uint32_t *keys, *vals;
     sorted_buffers(w, d, keys, vals);
     if (d.nb == 5) {
-      hipLaunchKernelGGL(k_records<5>, dim3(g), dim3(kRecThreads), 0, st, d, in, keys, vals, n, c->DNS, c->DM, w.rec, w.prs, w.dtot);
+      hipLaunchKernelGGL(k_records<5>, dim3(g, rec_parts(d, n)), dim3(kRecThreads), 0, st, d, in, keys, vals, n, c->DNS, c->DM, w.rec, w.prs, w.dtot);
     } else if (d.nb == 3) {
-      hipLaunchKernelGGL(k_records<3>, dim3(g), dim3(kRecThreads), 0, st, d, in, keys, vals, n, c->DNS, c->DM, w.rec, w.prs, w.dtot);
+      hipLaunchKernelGGL(k_records<3>, dim3(g, rec_parts(d, n)), dim3(kRecThreads), 0, st, d, in, keys, vals, n, c->DNS, c->DM, w.rec, w.prs, w.dtot);
     } else {
-      hipLaunchKernelGGL(k_records<1>, dim3(g), dim3(kRecThreads), 0, st, d, in, keys, vals, n, c->DNS, c->DM, w.rec, w.prs, w.dtot);
+      hipLaunchKernelGGL(k_records<1>, dim3(g, rec_parts(d, n)), dim3(kRecThreads), 0, st, d, in, keys, vals, n, c->DNS, c->DM, w.rec, w.prs, w.dtot);
     }
     hipLaunchKernelGGL(k_cells, dim3(g), dim3(256), 0, st, d, keys, n, w.rng, w.flag);
     HIP_TRY((exclusive_scan<int, int>(w.flag, w.ridx, n, w.scan_tmp, w.n_rows, st)));
