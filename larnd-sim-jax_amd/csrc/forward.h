@@ -304,19 +304,24 @@ __global__ void k_cells(Dev d, const uint32_t* __restrict__ keys, int64_t n, int
 }
 
 __global__ void k_rows_map(Dev d, const uint32_t* __restrict__ keys, const int* __restrict__ flag, const int* __restrict__ ridx,
-                           int64_t n, int* __restrict__ row_cell, int* __restrict__ cell_row) {
+                           int64_t n, int* __restrict__ row_cell, const int* __restrict__ n_rows,
+                           int64_t* __restrict__ n_rows_out) {
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i == 0 && n_rows_out) *n_rows_out = (int64_t)*n_rows;
   if (i >= n || !flag[i]) return;
-  const int r = ridx[i];
-  const uint32_t k = keys[i];
-  row_cell[r] = (int)k;
-  cell_row[k] = r;
+  row_cell[ridx[i]] = (int)keys[i];
 }
 
-__global__ void k_copy_count(const int* __restrict__ src, int64_t* __restrict__ dst, int64_t max_rows, int* __restrict__ status) {
+// A count for the caller (dst and status may be NULL), with the row overflow flag if it exceeds max_rows >= 0.
+__device__ __forceinline__ void copy_count(const int* __restrict__ src, int64_t* __restrict__ dst, int64_t max_rows,
+                                           int* __restrict__ status) {
   const int64_t v = (int64_t)*src;
   if (dst) *dst = v;
   if (status && max_rows >= 0 && v > max_rows) atomicOr(status, LSIM_STATUS_ROWS_OVERFLOW);
+}
+
+__global__ void k_copy_count(const int* __restrict__ src, int64_t* __restrict__ dst, int64_t max_rows, int* __restrict__ status) {
+  copy_count(src, dst, max_rows, status);
 }
 
 // ------------------------------------------------------------------------------------------
@@ -1001,8 +1006,10 @@ inline int64_t row_tiles(const Dev& d, int tile) {
 
 // Sort keys of the rows: the tile id, or `past` for the rows P..max_rows-1 (after every tile).
 __global__ void k_tile_keys(Dev d, int tile, const int* __restrict__ row_cell, const int* __restrict__ n_rows_dev,
-                            int64_t max_rows, uint32_t past, uint32_t* __restrict__ keys, uint32_t* __restrict__ vals) {
+                            int64_t max_rows, uint32_t past, uint32_t* __restrict__ keys, uint32_t* __restrict__ vals,
+                            int64_t* __restrict__ n_rows_out, int* __restrict__ status) {
   const int64_t r = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (r == 0) copy_count(n_rows_dev, n_rows_out, max_rows, status);
   if (r >= max_rows) return;
   const int64_t P = *n_rows_dev < max_rows ? *n_rows_dev : max_rows;
   vals[r] = (uint32_t)r;
@@ -1019,31 +1026,35 @@ __global__ void k_tile_keys(Dev d, int tile, const int* __restrict__ row_cell, c
 // Estimated work of every row, in processing order (work[s] for the row order[s]): one thread per
 // slot.  Rows P..max_rows-1 hold no pixel (and keep their place in the order): their hit count is
 // zeroed here for the hit scan over max_rows (the row kernel never visits them).
+// kWorkLanes lanes a row: its (2 ne + 1)^2 cell ranges are a few loads in flight per lane, not a chain.
+constexpr int kWorkLanes = 16;
 __global__ void k_row_work(Dev d, const int2* __restrict__ rng, const int* __restrict__ row_cell,
                            const int* __restrict__ order, const int* __restrict__ n_rows_dev, int64_t max_rows,
                            int row_cost, int* __restrict__ work, int* __restrict__ hit_cnt) {
-  const int64_t s = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  const int64_t g = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  const int64_t s = g / kWorkLanes;
+  const int l = (int)(g & (kWorkLanes - 1));
   const int64_t P = *n_rows_dev < max_rows ? *n_rows_dev : max_rows;
   if (s >= P) {
-    if (s < max_rows) hit_cnt[s] = 0;
+    if (l == 0 && s < max_rows) hit_cnt[s] = 0;
     return;
   }
   const int cell = row_cell[order[s]];
   const int px = cell % d.gx - d.halo;
   const int py = (cell / d.gx) % d.gy - d.halo;
   const int evp = cell / (d.gx * d.gy);
-  int n = row_cost;
-  for (int a = -d.ne; a <= d.ne; ++a) {
-    const int qx = px - a;
-    if (qx < -d.halo || qx >= d.nx + d.halo) continue;
-    for (int b = -d.ne; b <= d.ne; ++b) {
-      const int qy = py - b;
-      if (qy < -d.halo || qy >= d.ny + d.halo) continue;
-      const int2 rg = rng[((int64_t)evp * d.gy + (qy + d.halo)) * d.gx + (qx + d.halo)];
-      n += rg.y - rg.x;
-    }
+  const int W = 2 * d.ne + 1;
+  int n = 0;
+#pragma unroll 6
+  for (int k = l; k < W * W; k += kWorkLanes) {
+    const int qx = px - (k / W - d.ne), qy = py - (k % W - d.ne);
+    const bool in = qx >= -d.halo && qx < d.nx + d.halo && qy >= -d.halo && qy < d.ny + d.halo;
+    const int2 rg = rng[in ? ((int64_t)evp * d.gy + (qy + d.halo)) * d.gx + (qx + d.halo) : 0];
+    n += in ? rg.y - rg.x : 0;
   }
-  work[s] = n;
+#pragma unroll
+  for (int m = kWorkLanes / 2; m >= 1; m >>= 1) n += __shfl_xor(n, m, kWorkLanes);
+  if (l == 0) work[s] = n + row_cost;
 }
 
 // Band starts band[0..kXcd] (band[kXcd] = P) at equal shares of the total work; one workgroup of

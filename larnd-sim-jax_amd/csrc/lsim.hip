@@ -176,7 +176,6 @@ struct Ws {
   SegRec* rec;
   PairRec* prs;  // [n] window-store records (sorted order)
   int2* rng;
-  int* cell_row;
   int* flag;
   int* ridx;
   int* row_cell;
@@ -184,7 +183,6 @@ struct Ws {
   int* hit_cnt;
   int* hit_off;
   int* scan_tmp;
-  int* n_hits32;
   int* row_work;  // [n] estimated work of each pixel row in processing order (XCD band cuts)
   int* band;      // [kXcd + 1] first processing slot of each XCD's band
   int* next;      // [kXcd][kNextPad] slots taken so far of those past each band's fixed part
@@ -204,7 +202,6 @@ Ws layout(void* base, int64_t n, int64_t n_cells) {
   w.rec = c.take<SegRec>(n);
   w.prs = c.take<PairRec>(n);
   w.rng = c.take<int2>(n_cells);
-  w.cell_row = c.take<int>(n_cells);
   w.flag = c.take<int>(n);
   w.ridx = c.take<int>(n);
   w.row_cell = c.take<int>(n);
@@ -212,7 +209,6 @@ Ws layout(void* base, int64_t n, int64_t n_cells) {
   w.hit_cnt = c.take<int>(n);
   w.hit_off = c.take<int>(n);
   w.scan_tmp = c.take<int>(scan_tiles(n) + 4);
-  w.n_hits32 = c.take<int>(4);
   w.row_work = c.take<int>(n);
   w.band = c.take<int>(kXcd + 1);
   w.next = c.take<int>(kXcd * kNextPad);
@@ -272,15 +268,15 @@ const int* row_order(const Ws& w, const Dev& d) {
 
 // Processing order, work estimate of every row and the XCD band cuts (k_tile_keys + sort,
 // k_row_work, k_bands) before the row kernel; also zeroes the hit counts of the rows past P.
-int launch_row_bands(const Dev& d, const Ws& w, int64_t max_rows, hipStream_t st) {
+int launch_row_bands(const Dev& d, const Ws& w, int64_t max_rows, int64_t* n_rows_out, int* status, hipStream_t st) {
   const int bits = tile_key_bits(d);
   const unsigned g = (unsigned)((max_rows + 255) / 256);
   hipLaunchKernelGGL(k_tile_keys, dim3(g), dim3(256), 0, st, d, g_row_tile, w.row_cell, w.n_rows, max_rows,
-                     (uint32_t)(((uint64_t)1 << bits) - 1), w.tk0, w.tv0);
+                     (uint32_t)(((uint64_t)1 << bits) - 1), w.tk0, w.tv0, n_rows_out, status);
   hipError_t err;
   radix_sort_pairs(w.tk0, w.tv0, w.tk1, w.tv1, max_rows, bits, w.sort_scratch, st, &err);
   HIP_TRY(err);
-  hipLaunchKernelGGL(k_row_work, dim3(g), dim3(256), 0, st, d, w.rng, w.row_cell, row_order(w, d), w.n_rows, max_rows,
+  hipLaunchKernelGGL(k_row_work, dim3((unsigned)((max_rows * kWorkLanes + 255) / 256)), dim3(256), 0, st, d, w.rng, w.row_cell, row_order(w, d), w.n_rows, max_rows,
                      g_row_cost, w.row_work, w.hit_cnt);
   hipLaunchKernelGGL(k_bands, dim3(1), dim3(kBandThreads), 0, st, w.row_work, w.n_rows, max_rows, band_slots(max_rows),
                      w.band, w.next);
@@ -520,8 +516,6 @@ int lsim_forward_prepare(lsim_ctx* c, const lsim_params* p, const lsim_segments*
   int* status = status_dev;
 
   fill<int2>(w.rng, d.n_cells, make_int2(0, 0), st);
-  fill<int>(w.cell_row, d.n_cells, -1, st);
-  fill<int>(w.n_rows, 1, 0, st);
   if (n > 0) {
     const unsigned g = (unsigned)((n + 255) / 256);
     hipLaunchKernelGGL(k_keys, dim3(g), dim3(256), 0, st, d, in, w.k0, w.v0, status);
@@ -546,9 +540,12 @@ int lsim_forward_prepare(lsim_ctx* c, const lsim_params* p, const lsim_segments*
     }
     hipLaunchKernelGGL(k_cells, dim3(g), dim3(256), 0, st, d, keys, n, w.rng, w.flag);
     HIP_TRY((exclusive_scan<int, int>(w.flag, w.ridx, n, w.scan_tmp, w.n_rows, st)));
-    hipLaunchKernelGGL(k_rows_map, dim3(g), dim3(256), 0, st, d, keys, w.flag, w.ridx, n, w.row_cell, w.cell_row);
+    hipLaunchKernelGGL(k_rows_map, dim3(g), dim3(256), 0, st, d, keys, w.flag, w.ridx, n, w.row_cell, w.n_rows,
+                       n_rows_dev);
+  } else {
+    fill<int>(w.n_rows, 1, 0, st);
+    if (n_rows_dev) fill<int64_t>(n_rows_dev, 1, 0, st);
   }
-  hipLaunchKernelGGL(k_copy_count, dim3(1), dim3(1), 0, st, w.n_rows, n_rows_dev, (int64_t)-1, (int*)nullptr);
   HIP_TRY(hipGetLastError());
   return LSIM_OK;
 }
@@ -563,9 +560,8 @@ static int forward_rows_impl(lsim_ctx* c, const Dev& d, const Ws& w, int64_t n_s
   ro.tape = (FeeTape*)out->tape;
   ro.hit_cnt = w.hit_cnt;
   ro.pixel_ids = out->pixel_ids;
-  hipLaunchKernelGGL(k_copy_count, dim3(1), dim3(1), 0, st, w.n_rows, out->n_rows, max_rows, out->status);
   if (max_rows > 0) {
-    const int rc = launch_row_bands(d, w, max_rows, st);
+    const int rc = launch_row_bands(d, w, max_rows, out->n_rows, out->status, st);
     if (rc) return rc;
     hipEvent_t stop_ev;
     timer_begin(st, &stop_ev);
@@ -577,7 +573,7 @@ static int forward_rows_impl(lsim_ctx* c, const Dev& d, const Ws& w, int64_t n_s
     }
     HIP_TRY(hipGetLastError());
     if (stop_ev) HIP_TRY(hipEventRecord(stop_ev, st));
-    HIP_TRY((exclusive_scan<int, int>(w.hit_cnt, w.hit_off, max_rows, w.scan_tmp, w.n_hits32, st)));
+    HIP_TRY((exclusive_scan<int, int64_t>(w.hit_cnt, w.hit_off, max_rows, w.scan_tmp, out->n_hits, st)));
     if (out->hit_adc) {
       HitOut h{out->hit_adc, out->hit_x, out->hit_y, out->hit_z, out->hit_tick, out->hit_prob, out->hit_event,
                out->hit_pixel, out->hit_index};
@@ -586,9 +582,9 @@ static int forward_rows_impl(lsim_ctx* c, const Dev& d, const Ws& w, int64_t n_s
                          out->ticks, w.hit_off, out->n_rows, max_rows, (int64_t)0, h);
     }
   } else {
-    fill<int>(w.n_hits32, 1, 0, st);
+    hipLaunchKernelGGL(k_copy_count, dim3(1), dim3(1), 0, st, w.n_rows, out->n_rows, max_rows, out->status);
+    if (out->n_hits) fill<int64_t>(out->n_hits, 1, 0, st);
   }
-  if (out->n_hits) hipLaunchKernelGGL(k_copy_count, dim3(1), dim3(1), 0, st, w.n_hits32, out->n_hits, (int64_t)-1, (int*)nullptr);
   HIP_TRY(hipGetLastError());
   return LSIM_OK;
 }
@@ -694,7 +690,6 @@ static int fee_forward_impl(lsim_ctx* c, const lsim_params* p, const float* wfs,
   int* cnt = cv.take<int>(n_rows);
   int* off = cv.take<int>(n_rows);
   int* tmp = cv.take<int>(scan_tiles(n_rows) + 4);
-  int* tot = cv.take<int>(4);
   RowOut ro;
   ro.wfs = nullptr;
   ro.adc = out->adc;
@@ -704,7 +699,7 @@ static int fee_forward_impl(lsim_ctx* c, const lsim_params* p, const float* wfs,
   ro.pixel_ids = nullptr;
   if (n_rows > 0) {
     hipLaunchKernelGGL((k_fee_rows<256>), dim3((unsigned)n_rows), dim3(256), 0, st, d, wfs, pixel_ids, n_rows, ro);
-    HIP_TRY((exclusive_scan<int, int>(cnt, off, n_rows, tmp, tot, st)));
+    HIP_TRY((exclusive_scan<int, int64_t>(cnt, off, n_rows, tmp, out->n_hits, st)));
     if (out->hit_adc) {
       HitOut h{out->hit_adc, out->hit_x, out->hit_y, out->hit_z, out->hit_tick, out->hit_prob, out->hit_event,
                out->hit_pixel, out->hit_index};
@@ -713,9 +708,8 @@ static int fee_forward_impl(lsim_ctx* c, const lsim_params* p, const float* wfs,
                          (const int64_t*)nullptr, n_rows, n_rows, h);
     }
   } else {
-    fill<int>(tot, 1, 0, st);
+    if (out->n_hits) fill<int64_t>(out->n_hits, 1, 0, st);
   }
-  if (out->n_hits) hipLaunchKernelGGL(k_copy_count, dim3(1), dim3(1), 0, st, tot, out->n_hits, (int64_t)-1, (int*)nullptr);
   HIP_TRY(hipGetLastError());
   return LSIM_OK;
 }
@@ -852,7 +846,7 @@ static int backward_impl(lsim_ctx* c, const lsim_params* p, const lsim_segments*
     // partials are reduced by row); the rows no workgroup takes keep zero partials
     const bool banded = max_rows >= kAdjBandRows;
     if (banded) {
-      const int rc2 = launch_row_bands(d, w, max_rows, st);
+      const int rc2 = launch_row_bands(d, w, max_rows, nullptr, nullptr, st);
       if (rc2) return rc2;
     }
     fill<double>(partial, 2 * max_rows * kNGrad, 0.0, st);
