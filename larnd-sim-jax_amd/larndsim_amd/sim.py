@@ -210,18 +210,25 @@ class Simulator:
         _lib.check(self.lib.lsim_forward_query(self._ctx, n, n_events, C.byref(sz), C.byref(bound)))
         return torch.empty(int(sz.value), dtype=torch.uint8, device=self.device), int(bound.value)
 
-    def alloc_out(self, max_rows, want_wfs=True, want_tape=False, want_hits=True):
+    def alloc_out(self, max_rows, want_wfs=True, want_tape=False, want_hits=True, rows=None):
+        """Output buffers for ``max_rows`` rows; ``rows`` = (pixel ids, waveforms) to use instead of new ones."""
         d, H = self.device, self.H
         R = max(int(max_rows), 1)
+        counts = torch.zeros(3, dtype=torch.int64, device=d)  # one fill for the three
+        ids, wfs = rows if rows is not None else (None, None)
+        if ids is None:
+            ids = torch.empty(R, dtype=torch.int64, device=d)
+        if wfs is None and want_wfs:
+            wfs = torch.empty((R, self.nout), dtype=torch.float32, device=d)
         o = dict(
-            n_rows=torch.zeros(1, dtype=torch.int64, device=d),
-            pixel_ids=torch.empty(R, dtype=torch.int64, device=d),
-            wfs=torch.empty((R, self.nout), dtype=torch.float32, device=d) if want_wfs else None,
+            n_rows=counts[:1],
+            pixel_ids=ids,
+            wfs=wfs,
             adc=torch.empty((R, H), dtype=torch.float32, device=d),
             ticks=torch.empty((R, H), dtype=torch.int32, device=d),
             tape=torch.empty(R * self.tape_bytes, dtype=torch.uint8, device=d) if want_tape else None,
-            n_hits=torch.zeros(1, dtype=torch.int64, device=d),
-            status=torch.zeros(1, dtype=torch.int32, device=d),
+            n_hits=counts[1:2],
+            status=counts[2:].view(torch.int32)[:1],
         )
         if want_hits:
             for k in ("hit_adc", "hit_x", "hit_y", "hit_z", "hit_tick", "hit_prob"):
@@ -270,6 +277,38 @@ class Simulator:
                                              ws.numel(), max_rows, C.byref(oc), st))
         return ForwardState(seg.n, n_events, t, seg, ws, int(max_rows), out, oc, params)
 
+    def forward_reference_rows(self, params, tracks, fields, n_events=None):
+        """``forward`` with the rows where the reference's layout has them (``reference_rows``): the
+        waveform kernel writes behind the leading rows instead of being copied there, and both row
+        counts come with one host read.  Returns (state, waveforms, pixel ids)."""
+        _check_noise(params)
+        t, seg = self.segments(tracks, fields)
+        if n_events is None:
+            n_events = infer_n_events(tracks, fields)
+        pc = params_struct(params)
+        ws, _ = self.workspace(seg.n, n_events)
+        counts = torch.zeros(3, dtype=torch.int64, device=self.device)  # rows, negative ids, status
+        n_rows, n_neg, status = counts[:1], counts[1:2], counts[2:].view(torch.int32)[:1]
+        _lib.check(self.lib.lsim_forward_prepare(self._ctx, C.byref(pc), C.byref(seg), n_events, C.c_void_p(ws.data_ptr()),
+                                                 ws.numel(), C.c_void_p(n_rows.data_ptr()), C.c_void_p(status.data_ptr()),
+                                                 self._stream()))
+        neg_ids, _ = self.negative_rows(params, seg, n_neg)
+        P, k, _ = counts.tolist()
+        tgt = pad_size(P + k + 1, "unique_pixels", 0.2)
+        front = tgt - P
+        ids = torch.empty(tgt, dtype=torch.int64, device=self.device)
+        wfs = torch.empty((tgt, self.nout), dtype=torch.float32, device=self.device)
+        if k:
+            ids[:k] = neg_ids[:k]
+        ids[k:front] = -1
+        wfs[:front] = 0.0
+        out = self.alloc_out(P, rows=(ids[front:], wfs[front:]) if P else None)
+        out["status"] = status
+        oc = self.out_struct(out)
+        _lib.check(self.lib.lsim_forward_rows(self._ctx, C.byref(pc), seg.n, n_events, C.c_void_p(ws.data_ptr()), ws.numel(),
+                                              P, C.byref(oc), self._stream()))
+        return ForwardState(seg.n, n_events, t, seg, ws, P, out, oc, params), wfs, ids
+
     def backward(self, state: ForwardState, d_adc, d_z=None, d_wfs=None):
         """d loss / d (Ab, kb, eField, lifetime, vdrift, long_diff, tran_diff) as float64 (7,), from
         cotangents on the ADC grid, the hit z grid and (optionally) the waveforms (max_rows, nout)."""
@@ -301,15 +340,17 @@ class Simulator:
                                           self._stream()))
         return grad
 
-    def negative_rows(self, params, seg):
+    def negative_rows(self, params, seg, n=None):
         """Negative ids of the reference's pixel set, on the device: ``(ids, count)`` with the
         distinct negative main-pixel ids ascending in ``ids[:count]`` (padding segments' packed
-        event -1 ids, and -1 when a main pixel is off the plane).  Stream ordered, no host read."""
+        event -1 ids, and -1 when a main pixel is off the plane).  Stream ordered, no host read.
+        ``n``: the count's (1,) int64 tensor, if the caller has one."""
         sz, mx = C.c_size_t(), C.c_int64()
         _lib.check(self.lib.lsim_negative_rows_query(self._ctx, C.byref(sz), C.byref(mx)))
         ws = torch.empty(int(sz.value), dtype=torch.uint8, device=self.device)
         ids = torch.empty(max(int(mx.value), 1), dtype=torch.int64, device=self.device)
-        n = torch.zeros(1, dtype=torch.int64, device=self.device)
+        if n is None:
+            n = torch.zeros(1, dtype=torch.int64, device=self.device)
         _lib.check(self.lib.lsim_negative_rows(self._ctx, C.byref(params_struct(params)), C.byref(seg),
                                                C.c_void_p(ws.data_ptr()), ws.numel(), C.c_void_p(ids.data_ptr()),
                                                ids.numel(), C.c_void_p(n.data_ptr()), self._stream()))
@@ -395,12 +436,10 @@ def simulate_wfs(params, response_template, tracks, fields, pad=True):
     only the rows with ids >= 0 are returned.
     """
     sim = get_simulator(params, response_template)
-    st = sim.forward(params, tracks, fields, want_wfs=True)
-    wfs, pids = st.out["wfs"][: st.max_rows], st.out["pixel_ids"][: st.max_rows]
     if pad:
-        neg, n_neg = sim.negative_rows(params, st.seg)
-        wfs, pids = reference_rows(wfs, pids, neg, n_neg)
-    return wfs, pids
+        return sim.forward_reference_rows(params, tracks, fields)[1:]
+    st = sim.forward(params, tracks, fields, want_wfs=True)
+    return st.out["wfs"][: st.max_rows], st.out["pixel_ids"][: st.max_rows]
 
 
 def simulate_stochastic(params, wfs, unique_pixels, rngseed=0):

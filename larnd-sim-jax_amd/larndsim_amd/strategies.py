@@ -45,10 +45,8 @@ class HipLUTSimulation(SimulationStrategy):
             return dict(adcs=adcs, pixel_x=o["pixel_x"], pixel_y=o["pixel_y"], pixel_z=z, ticks=o["ticks"],
                         hit_prob=o["hit_prob"], event=o["event"], hit_pixels=o["hit_pixels"],
                         unique_pixels=ids, wfs=wfs)
-        st = sim.forward(params, tracks, fields, n_events=n_events, want_wfs=True)
-        neg = sim.negative_rows(params, st.seg)
+        st, wfs, ids = sim.forward_reference_rows(params, tracks, fields, n_events=n_events)
         h = hits_dict(st.out)
-        wfs, ids = reference_rows(st.out["wfs"][: st.max_rows], st.out["pixel_ids"][: st.max_rows], *neg)
         return dict(adcs=h["adcs"], pixel_x=h["pixel_x"], pixel_y=h["pixel_y"], pixel_z=h["pixel_z"], ticks=h["ticks"],
                     hit_prob=h["hit_prob"], event=h["event"], hit_pixels=h["hit_pixels"], unique_pixels=ids, wfs=wfs)
 
