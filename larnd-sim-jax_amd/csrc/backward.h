@@ -607,21 +607,24 @@ __global__ __launch_bounds__(WAVES * kWave) __attribute__((amdgpu_waves_per_eu(4
 //
 // G(o) = gw[r][o] + the self-trigger's step function: one value per output tick, so the window
 // sums are plain dot products, and they take the forward's access pattern with reads in place of
-// stores.  A whole wave works on one (segment, row) pair: lane l holds the padded window samples
-// p = l + 63 c (c < 3) of the pair (output tick o = S - 2 + p), G(o) comes from LDS and the next
-// sample (the f window) from lane l + 1 by a DPP shift; lane 63 only supplies that next sample.
+// stores.  A wave works on four windows at once, 16 lanes each: lane l of a group holds the padded window
+// samples p = 64 c + 4 l .. + 3 (c < 3; output tick o = S - 2 + p) by three 16-byte loads, G(o) comes from
+// LDS, and the f window's sum takes G(o - 1) instead of the next sample, so no lane needs another's.
 // The window sums of a pair enter the gradients linearly, so every lane scales its own share by
 // the pair's chain factors and adds it to its 7 partial gradients: no reduction per pair, one
 // per row at the end (fixed order: deterministic).
 //   Stripes (the raw-window stripe of every pixel offset but the centre, |a|, |b| <= nn): blocks
-//     of 64 pairs whose factors the lanes compute in parallel and stage in LDS; the wave then reads
-//     them back by broadcast, 4 pairs' window loads in flight at a time.  The boundary-correction
-//     terms (no window) are added by the lane that set the pair up.
+//     of 64 pairs whose factors the lanes compute in parallel and stage in LDS; each group of lanes then
+//     reads its pair's.  The boundary-correction terms (no window) are added by the lane that set the pair up.
 //   Diffusion bins landing on the row (the 3x3 cells; side rows only for segments near the pixel
-//     edge): one (segment, row) item per wave at a time, LUT cell by LUT cell from the interleaved
-//     template windows (T_{m-1}, T_m, T_{m+1}) of TM3: V = la T_{m-1} + lb T_m + lc T_{m+1} for
-//     n_e, f, sigma_T, and dV/dlambda = da (T_{m-1} - T_m) + dc (T_{m+1} - T_m) for lambda (the
-//     three Lagrange derivatives sum to zero, so the differences lose no precision).
+//     edge): one (segment, row) item per wave at a time.  A lane per bin merges the bins of one LUT cell,
+//     adds the cell's terms without a window and leaves weight and cell in LDS; four cells at a time take
+//     the sums of G with T_m and with the differences dm = T_{m-1} - T_m, dp = T_{m+1} - T_m from the
+//     interleaved template windows of TM3: V = (la + lb + lc) T_m + la dm + lc dp for n_e, f, sigma_T, and
+//     dV/dlambda = da dm + dc dp for lambda (the three Lagrange derivatives sum to zero).
+// A whole wave per window spent its time on what it did once a window or cell in every lane (25 float64
+// instructions a cell, 7 a stripe, 16-byte reads of the stage) and on 4-byte loads: 796 -> 570 us for the
+// 50k-segment step with a waveform loss; one group of four windows in flight is enough (two 588, four 686 us).
 
 constexpr int kGOff = 192;                       // LDS index of output tick 0
 constexpr int kGLen = kMaxOut + 2 * kGOff + 64;  // ticks -kGOff .. kMaxOut + kGOff + 63
@@ -635,6 +638,14 @@ struct __align__(16) DenseStripe {
   double fN[4], fF;
 };
 static_assert(sizeof(DenseStripe) == 64, "DenseStripe layout");
+
+// One merged LUT cell of a bins item: its weight and the weight's derivative in sigma_T.
+struct DenseCell {
+  double w, dw;
+  int cell, pad;
+};
+constexpr int kDensePairs = 1;  // groups of four pairs in flight
+typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 // G at a correction tick (those are kept for 0 <= o <= nout - 2); Gw holds 0 at tick 0 (a window
 // tick is kept from 1 on), G0 holds G(0).
@@ -661,6 +672,7 @@ __global__ __launch_bounds__(WAVES * kWave) void k_rows_adj_dense(Dev d, Tables 
   constexpr int SYM = (NB - 1) / 2;
   __shared__ float Gw[kGLen];
   __shared__ DenseStripe stage[WAVES][kWave];
+  __shared__ DenseCell s_cells[WAVES][NB * NB + 3];
   __shared__ int c_beg[kMaxCells], c_cum[kMaxCells + 1], c_ab[kMaxCells];
   __shared__ int ncls[3];
   __shared__ int cell_scratch[3 * kMaxCells];
@@ -723,7 +735,7 @@ __global__ __launch_bounds__(WAVES * kWave) void k_rows_adj_dense(Dev d, Tables 
   const int nstripe = c_cum[n_stripe_cells];
   const __amdgpu_buffer_rsrc_t tnp =
       __builtin_amdgcn_make_buffer_rsrc((void*)tb.TNP, 0, d.lx * d.ly * kWinPad * 4, kBufDesc3);
-  const float gmask = lane < kChunk ? 1.f : 0.f;  // lane 63 only supplies the next sample
+  const int sub = lane & 15, grp = lane >> 4;
   // ---- stripes ----
   for (int b0 = wid * kWave; b0 < nstripe; b0 += WAVES * kWave) {
     const int p = b0 + lane;
@@ -778,33 +790,37 @@ __global__ __launch_bounds__(WAVES * kWave) void k_rows_adj_dense(Dev d, Tables 
     stage[wid][lane] = z;
     __builtin_amdgcn_wave_barrier();
     const int n = __builtin_amdgcn_readfirstlane(nstripe - b0 < kWave ? nstripe - b0 : kWave);
-    for (int i = 0; i < n; i += 4) {
-      // pairs i .. i + 3 (entries past n are padding: factors 0, a window at S = 2)
-      DenseStripe q[4];
-      float x[4][3];
+    for (int i = 0; i < n; i += 4 * kDensePairs) {
+      // four pairs at a time, 16 lanes each (entries past n are padding: factors 0, a window at S = 2)
+      f32x4 x[kDensePairs][3];
+      int S[kDensePairs];
 #pragma unroll
-      for (int k = 0; k < 4; ++k) {
-        q[k] = stage[wid][i + k];
+      for (int h = 0; h < kDensePairs; ++h) {
+        const DenseStripe& q = stage[wid][i + 4 * h + grp];
+        S[h] = q.S;
+        const int off = q.off + sub * 16;
 #pragma unroll
         for (int c = 0; c < 3; ++c)
-          x[k][c] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(tnp, lane * 4 + c * 4 * kChunk + q[k].off, 0, 0));
+          x[h][c] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(tnp, off, c * 4 * kWave, 0));
       }
 #pragma unroll
-      for (int k = 0; k < 4; ++k) {
+      for (int h = 0; h < kDensePairs; ++h) {
+        const DenseStripe& q = stage[wid][i + 4 * h + grp];
         float u1 = 0.f, u0 = 0.f;
-        const float* gp = Gw + kGOff + q[k].S - 2 + lane;
 #pragma unroll
         for (int c = 0; c < 3; ++c) {
-          const float gv = gmask * gp[c * kChunk];
-          const float xn = lane_next0(x[k][c]);
-          u1 += gv * x[k][c];
-          u0 += gv * xn;
+          const float* gp = Gw + kGOff + S[h] - 2 + 4 * sub + kWave * c;
+#pragma unroll
+          for (int k = 0; k < 4; ++k) {
+            u1 = __builtin_fmaf(gp[k], x[h][c][k], u1);
+            u0 = __builtin_fmaf(gp[k - 1], x[h][c][k], u0);
+          }
         }
-        const double aa = (double)(q[k].c1 * u1 + q[k].c0 * u0), bb = (double)(q[k].ne * (u0 - u1));
-        g[0] += q[k].fN[0] * aa;
-        g[1] += q[k].fN[1] * aa;
-        g[2] += q[k].fN[2] * aa + q[k].fF * bb;
-        g[3] += q[k].fN[3] * aa;
+        const double aa = (double)(q.c1 * u1 + q.c0 * u0), bb = (double)(q.ne * (u0 - u1));
+        g[0] += q.fN[0] * aa;
+        g[1] += q.fN[1] * aa;
+        g[2] += q.fN[2] * aa + q.fF * bb;
+        g[3] += q.fN[3] * aa;
       }
     }
     __builtin_amdgcn_wave_barrier();  // the stage is rewritten by the next block
@@ -812,7 +828,6 @@ __global__ __launch_bounds__(WAVES * kWave) void k_rows_adj_dense(Dev d, Tables 
   // ---- diffusion bins of the 3x3 cells ----
   const int kb0 = c_cum[ncls[0]], kb1 = c_cum[ncls[2]];
   int cur = ncls[0];
-  const double lead = lane == 0 ? 1.0 : 0.0;  // terms without a window: once per item
   for (int k = kb0 + wid; k < kb1; k += WAVES) {
     while (k >= c_cum[cur + 1]) ++cur;
     const int s = __builtin_amdgcn_readfirstlane(c_beg[cur] + (k - c_cum[cur]));
@@ -828,71 +843,99 @@ __global__ __launch_bounds__(WAVES * kWave) void k_rows_adj_dense(Dev d, Tables 
     const double gc0 = g_corr(Gw, G0, S - 1, nout), gc1 = g_corr(Gw, G0, S - 2, nout);
     const double gc = (1.0 - f) * gc0 + f * gc1;
     const bool live = window_live(S, L, nout);
-    const float* gp = Gw + kGOff + (live ? S : 2) - 2 + lane;
-    float gv[3];
-#pragma unroll
-    for (int c = 0; c < 3; ++c) gv[c] = live ? gmask * gp[c * kChunk] : 0.f;
-    bool oky[NB];
-    int cyv[NB];
-    float WY[NB], DWY[NB];
-    axis_cells<NB>(uy, b, nsb, R.wy, A->dwy, oky, cyv, WY, DWY);
-    const float la = R.la, lb = R.lb, lc = R.lc;
-    const float da = (float)A->dl[0], dc = (float)A->dl[2];
+    // lane i NB + j: x-bin i, y-bin j.  Bins on one LUT cell are merged into the first of them, axis by axis.
     const int cm = d.cm;
+    const int bi = lane / NB, bj = lane - bi * NB;
+    int cx = 0, cy = 0;
+    float WX = 0.f, WY = 0.f, DWX = 0.f, DWY = 0.f;
+    bool mine = lane < NB * NB;
+#pragma unroll
+    for (int k = 0; k < NB; ++k) {
+      const int vx = ux + k - SYM, vy = uy + k - SYM;
+      const int dx = vx < 0 ? -1 : (vx >= nsb ? 1 : 0), dy = vy < 0 ? -1 : (vy >= nsb ? 1 : 0);
+      const int cxk = dx == a ? offset_bin(vx - dx * nsb, 0, nsb) : -1, cyk = dy == b ? offset_bin(vy - dy * nsb, 0, nsb) : -1;
+      cx = k == bi ? cxk : cx;
+      cy = k == bj ? cyk : cy;
+    }
+    mine = mine && cx >= 0 && cy >= 0;
+#pragma unroll
+    for (int k = 0; k < NB; ++k) {
+      const int vx = ux + k - SYM, vy = uy + k - SYM;
+      const int dx = vx < 0 ? -1 : (vx >= nsb ? 1 : 0), dy = vy < 0 ? -1 : (vy >= nsb ? 1 : 0);
+      const int cxk = dx == a ? offset_bin(vx - dx * nsb, 0, nsb) : -1, cyk = dy == b ? offset_bin(vy - dy * nsb, 0, nsb) : -1;
+      WX += cxk == cx ? R.wx[k] : 0.f;
+      DWX += cxk == cx ? A->dwx[k] : 0.f;
+      WY += cyk == cy ? R.wy[k] : 0.f;
+      DWY += cyk == cy ? A->dwy[k] : 0.f;
+      mine = mine && !(k < bi && cxk == cx) && !(k < bj && cyk == cy);
+    }
+    const double w = (double)WX * (double)WY, dw = (double)DWX * (double)WY + (double)WX * (double)DWY;
+    const int cell = mine ? (R.idx * cm + cx) * cm + cy : 0;
     double gN = 0.0, gF = 0.0, gS = 0.0, gL = 0.0;
+    // every cell's terms without a window, by its lane
+    if (mine) {
+      const float2 D = tb.DM[(int64_t)R.k0 * d.nm * cm * cm + cell];  // tick-major
+      const double corr = (double)D.x - f * (double)D.y, dy = (double)D.y;
+      gN = gc * corr * w;
+      gS = gc * corr * ne * dw;
+      gF = ne * w * ((gc1 - gc0) * corr - gc * dy);
+    }
+    const uint64_t m = __ballot(mine);
+    const int nc = __popcll(m);
+    if (live && nc > 0) {
+      // the cells in slots 0 .. nc - 1, up to a multiple of 4 filled with the first one at no weight
+      DenseCell* cells = s_cells[wid];
+      const int rank = __popcll(m & ((1ull << lane) - 1));
+      if (mine) cells[rank] = DenseCell{w, dw, cell, 0};
+      const int cell0 = __builtin_amdgcn_readlane(cell, __builtin_ctzll(m));
+      if (lane < 3) cells[nc + lane] = DenseCell{0.0, 0.0, cell0, 0};
+      __builtin_amdgcn_wave_barrier();
+      float gv[3][5];
 #pragma unroll
-    for (int i = 0; i < NB; ++i) {
-      const int vi = ux + i - SYM;
-      const int di = vi < 0 ? -1 : (vi >= nsb ? 1 : 0);
-      if (di != a) continue;
-      const int cx = offset_bin(vi - di * nsb, 0, nsb);
-      // x-bins on the same LUT cell are merged into the first of them
-      float WXi = 0.f, DWXi = 0.f;
-      bool first = true;
+      for (int c = 0; c < 3; ++c)
 #pragma unroll
-      for (int kk = 0; kk < NB; ++kk) {
-        const int v = ux + kk - SYM;
-        const int dv = v < 0 ? -1 : (v >= nsb ? 1 : 0);
-        if (dv != a || offset_bin(v - dv * nsb, 0, nsb) != cx) continue;
-        if (kk < i) first = false;
-        WXi += R.wx[kk];
-        DWXi += A->dwx[kk];
-      }
-      if (!first) continue;
-      // the y cells of this x cell: all window loads first, then the sums
-      float3 q[NB][3];
+        for (int k = 0; k < 5; ++k) gv[c][k] = Gw[kGOff + S - 3 + 4 * sub + kWave * c + k];
+      const float la = R.la, lc = R.lc, ls = R.la + R.lb + R.lc;
+      const float da = (float)A->dl[0], dc = (float)A->dl[2];
+      double U1 = 0.0, U0 = 0.0, D1 = 0.0, D0 = 0.0, L1 = 0.0, L0 = 0.0;
+      for (int k4 = 0; k4 < nc; k4 += 4) {
+        const DenseCell q = cells[k4 + grp];
+        const f32x4* T = (const f32x4*)(tb.TM3 + (int64_t)q.cell * kWinPad) + 3 * sub;
+        f32x4 v[3][3];
 #pragma unroll
-      for (int jj = 0; jj < NB; ++jj) {
-        const int cy = oky[jj] ? cyv[jj] : cyv[0];
-        const float3* T3 = tb.TM3 + (((int64_t)R.idx * cm + cx) * cm + cy) * kWinPad + lane;
+        for (int c = 0; c < 3; ++c)
 #pragma unroll
-        for (int c = 0; c < 3; ++c) q[jj][c] = T3[c * kChunk];
-      }
-#pragma unroll
-      for (int jj = 0; jj < NB; ++jj) {
-        if (!oky[jj]) continue;
-        const int64_t cell = ((int64_t)R.idx * cm + cx) * cm + cyv[jj];
-        float u1 = 0.f, u0 = 0.f, ul1 = 0.f, ul0 = 0.f;
+          for (int k = 0; k < 3; ++k) v[c][k] = T[c * (3 * kWave / 4) + k];
+        // sums of G and of G one tick on with T_m and its differences from T_{m-1}, T_{m+1}
+        float y1 = 0.f, y0 = 0.f, p1 = 0.f, p0 = 0.f, n1 = 0.f, n0 = 0.f;
 #pragma unroll
         for (int c = 0; c < 3; ++c) {
-          const float V = q[jj][c].y * lb + q[jj][c].x * la + q[jj][c].z * lc;
-          const float VL = da * (q[jj][c].x - q[jj][c].y) + dc * (q[jj][c].z - q[jj][c].y);
-          const float Vn = lane_next0(V), VLn = lane_next0(VL);
-          u1 += gv[c] * V;
-          u0 += gv[c] * Vn;
-          ul1 += gv[c] * VL;
-          ul0 += gv[c] * VLn;
+#pragma unroll
+          for (int k = 0; k < 4; ++k) {
+            const float tm = v[c][(3 * k) / 4][(3 * k) % 4], tc = v[c][(3 * k + 1) / 4][(3 * k + 1) % 4],
+                        tp = v[c][(3 * k + 2) / 4][(3 * k + 2) % 4];
+            const float dm = tm - tc, dp = tp - tc;
+            y1 = __builtin_fmaf(gv[c][k + 1], tc, y1);
+            y0 = __builtin_fmaf(gv[c][k], tc, y0);
+            p1 = __builtin_fmaf(gv[c][k + 1], dm, p1);
+            p0 = __builtin_fmaf(gv[c][k], dm, p0);
+            n1 = __builtin_fmaf(gv[c][k + 1], dp, n1);
+            n0 = __builtin_fmaf(gv[c][k], dp, n0);
+          }
         }
-        const float2 D = tb.DM[(int64_t)R.k0 * d.nm * cm * cm + cell];  // tick-major
-        const double corr = lead * ((double)D.x - f * (double)D.y), dy = lead * (double)D.y;
-        const double wxy = (double)WXi * (double)WY[jj];
-        const double dwxy = (double)DWXi * (double)WY[jj] + (double)WXi * (double)DWY[jj];
-        const double gn = (1.0 - f) * (double)u1 + f * (double)u0 + gc * corr;
-        gN += gn * wxy;
-        gS += gn * ne * dwxy;
-        gF += ne * wxy * ((double)u0 - (double)u1 + (gc1 - gc0) * corr - gc * dy);
-        gL += ne * wxy * ((1.0 - f) * (double)ul1 + f * (double)ul0);
+        const double u1 = (double)(ls * y1 + la * p1 + lc * n1), u0 = (double)(ls * y0 + la * p0 + lc * n0);
+        U1 += q.w * u1;
+        U0 += q.w * u0;
+        D1 += q.dw * u1;
+        D0 += q.dw * u0;
+        L1 += q.w * (double)(da * p1 + dc * n1);
+        L0 += q.w * (double)(da * p0 + dc * n0);
       }
+      __builtin_amdgcn_wave_barrier();  // the slots are rewritten by the next item
+      gN += (1.0 - f) * U1 + f * U0;
+      gS += ne * ((1.0 - f) * D1 + f * D0);
+      gF += ne * (U0 - U1);
+      gL += ne * ((1.0 - f) * L1 + f * L0);
     }
     add_chain(A, gN, gF, gS, gL, true, g);
   }
