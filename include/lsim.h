@@ -192,15 +192,9 @@ int lsim_timing_read(double *total_ms, int64_t *launches);
 /* Tuning: waves per pixel-row workgroup of the waveform kernel (1, 2, 4 or 8; default 4). */
 int lsim_set_row_waves(int waves);
 
-/* Tuning: the fixed cost of one pixel row in units of segment-row pairs (default 256), used to cut
- * the rows into per-XCD bands of equal estimated work for the waveform kernel.  Only
- * the schedule changes: results are the same for every value. */
+/* Settings of an earlier schedule (the cost of a row in pairs, the side of the cell tiles rows were taken
+ * by): checked and accepted, without effect.  Results never depended on them. */
 int lsim_set_row_cost(int pairs);
-
-/* Scheduling knob of the waveform kernel, no counterpart in the reference (like the two above): the
- * pixel rows are processed tile by tile, `cells` x `cells` pixel cells of one event plane per tile
- * (default 16; 1 = plain row order), so that the rows running together on one XCD share their
- * segments in its L2.  Changes only the order rows are computed in, never their values. */
 int lsim_set_row_tile(int cells);
 
 /* Backward workspace bytes for n_seg segments and max_rows rows. */

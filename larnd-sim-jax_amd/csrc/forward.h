@@ -6,12 +6,11 @@
 
 namespace lsim {
 
-// Window tables used by the waveform kernels are zero padded: P[p] = W[p - 2] for 2 <= p < L + 2
-// and 0 elsewhere, kWinPad entries per series, so chunk c of lane l reads P[63 c + l] with no
-// bounds test (windows up to 3 * 63 - 2 = 187 samples).
+// Window tables of the waveform adjoint are zero padded: P[p] = W[p - 2] for 2 <= p < L + 2 and 0
+// elsewhere, kWinPad entries per series, read without bounds tests (windows up to kMaxWindow samples).
 constexpr int kWinPad = 3 * kWave;
+constexpr int kMaxWindow = kWinPad - 5;
 constexpr int kXcd = 8;  // XCDs of an MI355X (workgroup i runs on XCD i % 8)
-constexpr int kNextPad = 32;  // one 128-byte line per band's slot counter (take_row)
 
 // Raw-response windows as the stripe accumulation reads them: row (cx, cy) of `stripe_stride(L)` floats
 // holds kStripeLead zeros and then the L samples, and zeros follow up to the stride; the next row's
@@ -349,6 +348,8 @@ struct RowOut {
   FeeTape* tape;       // [max_rows] or null
   int* hit_cnt;        // [max_rows]
   int64_t* pixel_ids;  // [max_rows]
+  int64_t* n_rows = nullptr;  // the row count and overflow flag for the caller (row kernel only)
+  int* status = nullptr;
 };
 
 // NaN passes through both clamps, as through jnp.maximum / jnp.minimum (a waveform poisoned by an
@@ -564,8 +565,6 @@ __device__ void finish_row(const Dev& d, const float* acc, int nwaves, int rstri
 // 1 <= o <= nout-1, corrections for 0 <= o <= nout-2 (the reference's garbage column takes the
 // rest).
 //
-// kChunk: window samples per load of the adjoint's wave-wide reads (lane 63 supplies lane 62's next one).
-constexpr int kChunk = kWave - 1;
 // Slack after each wave's partial row: an interior window (2 <= S, S + L <= nout) is stored three ticks
 // per lane from S - 2 while 3 lane < L + 2, so it writes up to S + L + 1.
 __host__ __device__ inline int row_pad(int) { return 4; }
@@ -984,180 +983,25 @@ __device__ __forceinline__ void list_cells_fwd(const Dev& d, const int2* __restr
 }
 
 // ------------------------------------------------------------------------------------------
-// work-balanced XCD bands of pixel rows for the row kernels
+// rows on the XCDs
 // ------------------------------------------------------------------------------------------
 //
-// Workgroup i of a launch runs on XCD i % kXcd, so each XCD is given one contiguous band of rows
-// (its records and tables stay in that XCD's L2).  Rows differ in cost (the segments in their
-// neighbourhood), and equal row counts per band leave some XCDs with up to 1.4x the mean work on
-// uneven batches.  The bands are therefore cut at equal shares of the estimated work: segments in
-// the row's (2e+1)^2 neighbourhood cells plus a fixed per-row cost (row set-up, sum, cumulative
-// charge and self-trigger) in the same units.
+// Workgroups are dispatched round-robin over the XCDs (workgroup i runs on XCD i % kXcd) and, within one, as
+// its CUs come free.  The row kernels hand the rows out in row order by runs of kRowRun: neighbours along a
+// pixel row, which share most of their segments, land in one L2, and every XCD gets its share of the dense
+// and of the empty parts of an event.  One contiguous band an XCD, cut at equal shares of the estimated work
+// in an order by cell tiles, with the last quarter of the rows handed out by counters, balanced worse: 200k
+// segments 1.52 -> 1.21 ms, 128 events of 72k segments 52.5 -> 50.5 ms, and the adjoint's equal row counts an
+// XCD 720 -> 575 us (near), 420 -> 319 (far), 570 -> 430 (waveforms).  Runs of 4 to 64 are within 3 %.
+constexpr int kRowRun = 16;
 
-// Processing order of the pixel rows: by tile of `tile` x `tile` cells of one event plane, in row
-// order within a tile (a stable sort on the tile id).  Consecutive workgroups of an XCD then work
-// on neighbouring pixels, whose neighbourhoods share most of their segments, so the segment
-// records and corrections a band reads stay in that XCD's L2.  The order changes which workgroup
-// computes a row and when, never what it computes (tile 1: plain row order).
-inline int64_t row_tiles(const Dev& d, int tile) {
-  const int64_t ntx = (d.gx + tile - 1) / tile, nty = (d.gy + tile - 1) / tile;
-  return d.n_cells / ((int64_t)d.gx * d.gy) * ntx * nty;
+__device__ __forceinline__ int64_t run_row() {  // of this workgroup; at or past the number of rows: none
+  const int64_t x = blockIdx.x % kXcd, j = blockIdx.x / kXcd;
+  return (j / kRowRun * kXcd + x) * kRowRun + j % kRowRun;
 }
 
-// Sort keys of the rows: the tile id, or `past` for the rows P..max_rows-1 (after every tile).
-__global__ void k_tile_keys(Dev d, int tile, const int* __restrict__ row_cell, const int* __restrict__ n_rows_dev,
-                            int64_t max_rows, uint32_t past, uint32_t* __restrict__ keys, uint32_t* __restrict__ vals,
-                            int64_t* __restrict__ n_rows_out, int* __restrict__ status) {
-  const int64_t r = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (r == 0) copy_count(n_rows_dev, n_rows_out, max_rows, status);
-  if (r >= max_rows) return;
-  const int64_t P = *n_rows_dev < max_rows ? *n_rows_dev : max_rows;
-  vals[r] = (uint32_t)r;
-  if (r >= P) {
-    keys[r] = past;
-    return;
-  }
-  const int cell = row_cell[r];
-  const int cx = cell % d.gx, cy = (cell / d.gx) % d.gy, evp = cell / (d.gx * d.gy);
-  const uint32_t ntx = (uint32_t)((d.gx + tile - 1) / tile), nty = (uint32_t)((d.gy + tile - 1) / tile);
-  keys[r] = ((uint32_t)evp * nty + (uint32_t)(cy / tile)) * ntx + (uint32_t)(cx / tile);
-}
-
-// Estimated work of every row, in processing order (work[s] for the row order[s]): one thread per
-// slot.  Rows P..max_rows-1 hold no pixel (and keep their place in the order): their hit count is
-// zeroed here for the hit scan over max_rows (the row kernel never visits them).
-// kWorkLanes lanes a row: its (2 ne + 1)^2 cell ranges are a few loads in flight per lane, not a chain.
-constexpr int kWorkLanes = 16;
-__global__ void k_row_work(Dev d, const int2* __restrict__ rng, const int* __restrict__ row_cell,
-                           const int* __restrict__ order, const int* __restrict__ n_rows_dev, int64_t max_rows,
-                           int row_cost, int* __restrict__ work, int* __restrict__ hit_cnt) {
-  const int64_t g = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  const int64_t s = g / kWorkLanes;
-  const int l = (int)(g & (kWorkLanes - 1));
-  const int64_t P = *n_rows_dev < max_rows ? *n_rows_dev : max_rows;
-  if (s >= P) {
-    if (l == 0 && s < max_rows) hit_cnt[s] = 0;
-    return;
-  }
-  const int cell = row_cell[order[s]];
-  const int px = cell % d.gx - d.halo;
-  const int py = (cell / d.gx) % d.gy - d.halo;
-  const int evp = cell / (d.gx * d.gy);
-  const int W = 2 * d.ne + 1;
-  int n = 0;
-#pragma unroll 6
-  for (int k = l; k < W * W; k += kWorkLanes) {
-    const int qx = px - (k / W - d.ne), qy = py - (k % W - d.ne);
-    const bool in = qx >= -d.halo && qx < d.nx + d.halo && qy >= -d.halo && qy < d.ny + d.halo;
-    const int2 rg = rng[in ? ((int64_t)evp * d.gy + (qy + d.halo)) * d.gx + (qx + d.halo) : 0];
-    n += in ? rg.y - rg.x : 0;
-  }
-#pragma unroll
-  for (int m = kWorkLanes / 2; m >= 1; m >>= 1) n += __shfl_xor(n, m, kWorkLanes);
-  if (l == 0) work[s] = n + row_cost;
-}
-
-// Band starts band[0..kXcd] (band[kXcd] = P) at equal shares of the total work; one workgroup of
-// kBandThreads threads.  The equal-work start of band x is the first row whose exclusive work
-// prefix reaches x/kXcd of the total (every row's work is >= 1, so the prefix is strictly
-// increasing).  Each band then holds at most `slots` rows (the workgroups per XCD of the row
-// kernel, kXcd * slots >= P): start_x is clamped to [max(start_{x-1}, P - (kXcd - x) slots),
-// start_{x-1} + slots], which keeps the starts non-decreasing and leaves room for the later bands.
-constexpr int kBandThreads = 1024;
-
-__global__ __launch_bounds__(kBandThreads) void k_bands(const int* __restrict__ work, const int* __restrict__ n_rows_dev,
-                                                      int64_t max_rows, int64_t slots, int* __restrict__ band,
-                                                      int* __restrict__ next) {
-  __shared__ int64_t part[kBandThreads];
-  __shared__ int64_t cut[kXcd + 1];
-  const int t = threadIdx.x;
-  if (t < kXcd) next[t * kNextPad] = 0;
-  const int64_t P = *n_rows_dev < max_rows ? *n_rows_dev : max_rows;
-  const int64_t per = (P + kBandThreads - 1) / kBandThreads;
-  const int64_t r0 = (int64_t)t * per < P ? (int64_t)t * per : P;
-  const int64_t r1 = r0 + per < P ? r0 + per : P;
-  int64_t s = 0;
-  for (int64_t r = r0; r < r1; ++r) s += work[r];
-  part[t] = s;
-  __syncthreads();
-  for (int off = 1; off < kBandThreads; off <<= 1) {  // inclusive Hillis-Steele scan
-    const int64_t v = t >= off ? part[t - off] : 0;
-    __syncthreads();
-    part[t] += v;
-    __syncthreads();
-  }
-  const int64_t total = part[kBandThreads - 1];
-  const int64_t ex = part[t] - s;
-  for (int x = 1; x < kXcd; ++x) {
-    const int64_t target = total * x / kXcd;
-    if (ex < target && target <= ex + s) {
-      int64_t r = r0, e = ex;
-      while (e < target) e += work[r++];
-      cut[x] = r;
-    }
-    if (target == 0 && t == 0) cut[x] = 0;
-  }
-  __syncthreads();
-  if (t == 0) {
-    int64_t prev = 0;
-    band[0] = 0;
-    for (int x = 1; x < kXcd; ++x) {
-      int64_t lo = P - (int64_t)(kXcd - x) * slots;
-      lo = lo > prev ? lo : prev;
-      const int64_t hi = prev + slots;
-      int64_t v = cut[x] < lo ? lo : cut[x];
-      v = v > hi ? hi : v;
-      band[x] = (int)v;
-      prev = v;
-    }
-    band[kXcd] = (int)P;
-  }
-}
-
-// XCD-aware mapping of workgroups onto rows: workgroups are dispatched round-robin over the XCDs, so
-// workgroup i runs on XCD x = i % kXcd.  Band x (k_bands) holds contiguous slots of the tile-major
-// processing order at equal shares of the estimated work, so a band's records and tables stay in that
-// XCD's L2.  Workgroup i takes slot i / kXcd of band x among the band's first `fixed` slots (three
-// quarters of an equal share of the rows); the later workgroups take the next slot of band x that is left
-// and, with band x used up, one of another band: the work estimate is linear in the pairs, rows are not,
-// and an XCD that is done early would stand idle (on 60 events of 5k and 72k segments a quarter of the
-// CU time did: 25.0 -> 20.0 ms).  Taking every slot that way is slower for launches of 10k light rows (the
-// counters' atomics pass to the memory side: 0.32 -> 0.50 ms).  Which workgroup computes a row
-// changes nothing in the row.  Workgroups that find no slot exit at once.  A launch whose workgroups are
-// all resident together (max_rows <= kStaticRows) needs no balancing: every slot is taken by its index.
-constexpr int kStaticRows = 1024;
-
-__device__ __forceinline__ int take_row(const int* __restrict__ band, int* __restrict__ next,
-                                        const int* __restrict__ order, int P, int64_t max_rows, int* sh) {
-  const int x = (int)(blockIdx.x % kXcd);
-  const int j = (int)(blockIdx.x / kXcd), fixed = max_rows <= kStaticRows ? P : 3 * (P / kXcd) / 4;
-  if (j < fixed && j < band[x + 1] - band[x]) return band[x] + j < P ? order[band[x] + j] : -1;
-  if (max_rows <= kStaticRows) return -1;
-  if (threadIdx.x < kWave) {
-    // lane b < kXcd: band b.  The bands with slots left, this XCD's first; a band found used up on the
-    // way is not tried again.
-    const int b = threadIdx.x < kXcd ? threadIdx.x : 0;
-    const int len = band[b + 1] - band[b], b0 = band[b] + (len < fixed ? len : fixed), n = band[b + 1] - b0;
-    const bool left =
-        threadIdx.x < kXcd && __hip_atomic_load(next + b * kNextPad, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < n;
-    uint32_t m = (uint32_t)__ballot(left);
-    int r = -1;
-    while (m != 0 && r < 0) {
-      const uint32_t from_x = m >> x << x;
-      const int y = __builtin_ctz(from_x ? from_x : m);
-      m &= ~(1u << y);
-      int i = 0;
-      if (threadIdx.x == 0) i = atomicAdd(next + y * kNextPad, 1);
-      i = __builtin_amdgcn_readfirstlane(i);
-      const int y0 = __builtin_amdgcn_readlane(b0, y), ny = __builtin_amdgcn_readlane(n, y);
-      if (i < ny && y0 + i < P) r = order[y0 + i];
-    }
-    if (threadIdx.x == 0) *sh = r;
-  }
-  __syncthreads();
-  const int r = *sh;
-  __syncthreads();
-  return r;
+inline int64_t run_grid(int64_t max_rows) {
+  return (max_rows + kXcd * kRowRun - 1) / (kXcd * kRowRun) * (kXcd * kRowRun);
 }
 
 // One workgroup per pixel row.  What bounds it (160k rows, 2e8 stripe pairs, 4 waves a row; parts by
@@ -1169,8 +1013,6 @@ template <int NB, int WAVES>
 __global__ __launch_bounds__(WAVES * kWave) void k_rows_fwd(Dev d, Tables tb, const SegRec* __restrict__ rec,
                                                             const int2* __restrict__ rng, const int* __restrict__ row_cell,
                                                             const int* __restrict__ n_rows_dev, int64_t max_rows,
-                                                            const int* __restrict__ band, int* __restrict__ next,
-                                                            const int* __restrict__ order,
                                                             const float* __restrict__ dtot,
                                                             const PairRec* __restrict__ prs, int64_t nseg, RowOut out) {
   constexpr int NT = WAVES * kWave;
@@ -1181,8 +1023,13 @@ __global__ __launch_bounds__(WAVES * kWave) void k_rows_fwd(Dev d, Tables tb, co
 
   const int P0 = *n_rows_dev;
   const int P = P0 < max_rows ? P0 : (int)max_rows;
-  const int r = take_row(band, next, order, P, max_rows, ncls);
-  if (r < 0) return;
+  const int64_t row = run_row();
+  if (row == 0 && threadIdx.x == 0) copy_count(n_rows_dev, out.n_rows, max_rows, out.status);
+  if (row >= P) {
+    if (row < max_rows && threadIdx.x == 0) out.hit_cnt[row] = 0;  // (the hit scan runs over max_rows)
+    return;
+  }
+  const int r = (int)row;
   const int nout = d.nout;
   float* acc = (float*)smem;
   // this row's neighbourhood cells: far cells first, then the 3x3 near cells, in (a, b) order

@@ -183,10 +183,6 @@ struct Ws {
   int* hit_cnt;
   int* hit_off;
   int* scan_tmp;
-  int* row_work;  // [n] estimated work of each pixel row in processing order (XCD band cuts)
-  int* band;      // [kXcd + 1] first processing slot of each XCD's band
-  int* next;      // [kXcd][kNextPad] slots taken so far of those past each band's fixed part
-  uint32_t *tk0, *tv0, *tk1, *tv1;  // [n + 1] tile sort ping-pong; the processing order lands in tv0 or tv1
   float* dtot;  // [(2 nn + 1)^2][n] boundary corrections of every (segment, row offset) pair
   size_t bytes;
 };
@@ -198,7 +194,7 @@ Ws layout(void* base, int64_t n, int64_t n_cells) {
   w.v0 = c.take<uint32_t>(n);
   w.k1 = c.take<uint32_t>(n);
   w.v1 = c.take<uint32_t>(n);
-  w.sort_scratch = c.take<char>((int64_t)radix_sort_scratch(n + 1));  // segments, then rows (<= max(n, 1))
+  w.sort_scratch = c.take<char>((int64_t)radix_sort_scratch(n));
   w.rec = c.take<SegRec>(n);
   w.prs = c.take<PairRec>(n);
   w.rng = c.take<int2>(n_cells);
@@ -209,13 +205,6 @@ Ws layout(void* base, int64_t n, int64_t n_cells) {
   w.hit_cnt = c.take<int>(n);
   w.hit_off = c.take<int>(n);
   w.scan_tmp = c.take<int>(scan_tiles(n) + 4);
-  w.row_work = c.take<int>(n);
-  w.band = c.take<int>(kXcd + 1);
-  w.next = c.take<int>(kXcd * kNextPad);
-  w.tk0 = c.take<uint32_t>(n + 1);
-  w.tv0 = c.take<uint32_t>(n + 1);
-  w.tk1 = c.take<uint32_t>(n + 1);
-  w.tv1 = c.take<uint32_t>(n + 1);
   w.dtot = nullptr;
   w.bytes = c.off + 256;
   return w;
@@ -246,53 +235,12 @@ void sorted_buffers(const Ws& w, const Dev& d, uint32_t*& keys, uint32_t*& vals)
   vals = (passes & 1) ? w.v1 : w.v0;
 }
 
-// Fixed cost of one pixel row (set-up, row sum, cumulative charge, self-trigger) in units of
-// segment-row pairs, for the work estimate the XCD bands are cut on (lsim_set_row_cost).
-int g_row_cost = 256;
-
-// Rows each XCD's band may hold: 1.5 times an equal share of max_rows (the grid of the row kernel
-// is kXcd times this, so at most a third of its workgroups find no row).
-int64_t band_slots(int64_t max_rows) { return (3 * max_rows + 2 * kXcd - 1) / (2 * kXcd); }
-
-// Side of the square cell tiles of the rows' processing order (lsim_set_row_tile).
-int g_row_tile = 16;
-
-// Bits of the tile-order sort key: every tile id and the key of the rows past P.
-int tile_key_bits(const Dev& d) { return bits_for(row_tiles(d, g_row_tile) + 1); }
-
-// The processing order of the rows (sorted by tile: k_tile_keys + radix sort); the buffer it lands
-// in depends only on the key width, like sorted_buffers.
-const int* row_order(const Ws& w, const Dev& d) {
-  return (const int*)((((tile_key_bits(d) + 7) / 8) & 1) ? w.tv1 : w.tv0);
-}
-
-// Processing order, work estimate of every row and the XCD band cuts (k_tile_keys + sort,
-// k_row_work, k_bands) before the row kernel; also zeroes the hit counts of the rows past P.
-int launch_row_bands(const Dev& d, const Ws& w, int64_t max_rows, int64_t* n_rows_out, int* status, hipStream_t st) {
-  const int bits = tile_key_bits(d);
-  const unsigned g = (unsigned)((max_rows + 255) / 256);
-  hipLaunchKernelGGL(k_tile_keys, dim3(g), dim3(256), 0, st, d, g_row_tile, w.row_cell, w.n_rows, max_rows,
-                     (uint32_t)(((uint64_t)1 << bits) - 1), w.tk0, w.tv0, n_rows_out, status);
-  hipError_t err;
-  radix_sort_pairs(w.tk0, w.tv0, w.tk1, w.tv1, max_rows, bits, w.sort_scratch, st, &err);
-  HIP_TRY(err);
-  hipLaunchKernelGGL(k_row_work, dim3((unsigned)((max_rows * kWorkLanes + 255) / 256)), dim3(256), 0, st, d, w.rng, w.row_cell, row_order(w, d), w.n_rows, max_rows,
-                     g_row_cost, w.row_work, w.hit_cnt);
-  hipLaunchKernelGGL(k_bands, dim3(1), dim3(kBandThreads), 0, st, w.row_work, w.n_rows, max_rows, band_slots(max_rows),
-                     w.band, w.next);
-  HIP_TRY(hipGetLastError());
-  return LSIM_OK;
-}
-
 template <int NB, int WAVES>
 void launch_rows_nb(const Dev& d, const Tables& tb, const Ws& w, int64_t n_seg, int64_t max_rows, const RowOut& ro,
                     hipStream_t st) {
   const size_t lds = rows_lds_bytes(WAVES, d.nout, d.L, (2 * d.ne + 1) * (2 * d.ne + 1));
-  // static rows: the longest band; else a workgroup per row and an eighth more, so that an XCD that is
-  // done early finds workgroups to go on with
-  const int64_t grid = max_rows <= kStaticRows ? kXcd * band_slots(max_rows) : max_rows + max_rows / 8;
-  hipLaunchKernelGGL((k_rows_fwd<NB, WAVES>), dim3((unsigned)grid), dim3(WAVES * kWave), lds, st, d, tb, w.rec, w.rng,
-                     w.row_cell, w.n_rows, max_rows, w.band, w.next, row_order(w, d), w.dtot, w.prs, n_seg, ro);
+  hipLaunchKernelGGL((k_rows_fwd<NB, WAVES>), dim3((unsigned)run_grid(max_rows)), dim3(WAVES * kWave), lds, st, d, tb,
+                     w.rec, w.rng, w.row_cell, w.n_rows, max_rows, w.dtot, w.prs, n_seg, ro);
 }
 
 template <int WAVES>
@@ -363,13 +311,11 @@ int lsim_set_row_waves(int waves) {
 
 int lsim_set_row_cost(int pairs) {
   if (pairs < 1 || pairs > (1 << 20)) return fail(LSIM_E_ARG, "row cost must be in [1, 2^20] pairs");
-  g_row_cost = pairs;
   return LSIM_OK;
 }
 
 int lsim_set_row_tile(int cells) {
   if (cells < 1 || cells > 4096) return fail(LSIM_E_ARG, "row tile must be in [1, 4096] cells");
-  g_row_tile = cells;
   return LSIM_OK;
 }
 
@@ -404,7 +350,7 @@ int lsim_ctx_create(lsim_ctx** out, const lsim_geometry* geo, const lsim_config*
   if (nsb < 2 || (nsb & 1)) return fail(LSIM_E_ARG, "nb_sampling_bins_per_pixel must be even and >= 2");
   if ((nb - 1) / 2 >= nsb) return fail(LSIM_E_ARG, "diffusion bins wider than a pixel are not supported");
   if (cfg->number_pix_neighbors < 0 || cfg->number_pix_neighbors > 8) return fail(LSIM_E_ARG, "number_pix_neighbors out of range");
-  if (cfg->signal_length < 1 || cfg->signal_length > 3 * kChunk - 2)
+  if (cfg->signal_length < 1 || cfg->signal_length > kMaxWindow)
     return fail(LSIM_E_ARG, "signal_length out of range (1..187)");
   if (cfg->n_ticks < 4 || cfg->n_ticks - 1 > kMaxOut) return fail(LSIM_E_ARG, "n_ticks out of range (<= 2049)");
   if (cfg->max_adc_values < 1 || cfg->max_adc_values > kMaxH) return fail(LSIM_E_ARG, "max_adc_values out of range");
@@ -560,9 +506,9 @@ static int forward_rows_impl(lsim_ctx* c, const Dev& d, const Ws& w, int64_t n_s
   ro.tape = (FeeTape*)out->tape;
   ro.hit_cnt = w.hit_cnt;
   ro.pixel_ids = out->pixel_ids;
+  ro.n_rows = out->n_rows;
+  ro.status = out->status;
   if (max_rows > 0) {
-    const int rc = launch_row_bands(d, w, max_rows, out->n_rows, out->status, st);
-    if (rc) return rc;
     hipEvent_t stop_ev;
     timer_begin(st, &stop_ev);
     switch (g_row_waves) {
@@ -808,9 +754,6 @@ int lsim_backward_query(lsim_ctx* c, int64_t n_seg, int64_t max_rows, size_t* by
   return LSIM_OK;
 }
 
-// Row count from which the adjoint's row kernels take the forward's work-balanced bands (rebuilt
-// per backward, about 0.1 ms); below it, equal row counts per XCD.
-constexpr int64_t kAdjBandRows = 32768;
 
 static int backward_impl(lsim_ctx* c, const lsim_params* p, const lsim_segments* seg, int32_t n_events, void* ws,
                          size_t ws_bytes, int64_t max_rows, const lsim_fwd_out* fwd, const float* d_adc, const float* d_z,
@@ -841,32 +784,21 @@ static int backward_impl(lsim_ctx* c, const lsim_params* p, const lsim_segments*
   uint32_t *keys, *vals;
   sorted_buffers(w, d, keys, vals);
   if (max_rows > 0) {
-    // large launches: the rows' processing order and XCD bands, rebuilt as the forward builds them
-    // (the schedule settings may have changed since; the result does not depend on them: the
-    // partials are reduced by row); the rows no workgroup takes keep zero partials
-    const bool banded = max_rows >= kAdjBandRows;
-    if (banded) {
-      const int rc2 = launch_row_bands(d, w, max_rows, nullptr, nullptr, st);
-      if (rc2) return rc2;
-    }
-    fill<double>(partial, 2 * max_rows * kNGrad, 0.0, st);
-    const int* band = banded ? w.band : nullptr;
-    const int* order = banded ? row_order(w, d) : nullptr;
     hipLaunchKernelGGL(k_fee_adjoint, dim3((unsigned)((max_rows + kFeeRows - 1) / kFeeRows)), dim3(kFeeRows * kWave), 0, st,
                        d, (const FeeTape*)fwd->tape,
                        d_adc, d_z, fwd->n_rows, max_rows, pieces, dz);
     if (n > 0)
       hipLaunchKernelGGL(k_adj_records, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, d, in, keys, vals, n, adj);
-    const dim3 grid((unsigned)(banded ? kXcd * band_slots(max_rows) : max_rows)), block(kAdjWaves * kWave);
+    const dim3 grid((unsigned)run_grid(max_rows)), block(kAdjWaves * kWave);
     double* pnear = partial + max_rows * kNGrad;
 #define LSIM_ADJ_LAUNCH(NBV)                                                                                        \
   hipLaunchKernelGGL((k_rows_adj<NBV, kAdjWaves, false>), grid, block, 0, st, d, tb, w.rec, w.prs, adj, w.rng,       \
-                     w.row_cell, w.n_rows, max_rows, band, order, pieces, partial);                               \
+                     w.row_cell, w.n_rows, max_rows, pieces, partial);                               \
   hipLaunchKernelGGL((k_rows_adj<NBV, kAdjWaves, true>), grid, block, 0, st, d, tb, w.rec, w.prs, adj, w.rng,        \
-                     w.row_cell, w.n_rows, max_rows, band, order, pieces, pnear)
+                     w.row_cell, w.n_rows, max_rows, pieces, pnear)
 #define LSIM_ADJ_DENSE(NBV)                                                                                       \
   hipLaunchKernelGGL((k_rows_adj_dense<NBV, kAdjWaves>), grid, block, 0, st, d, tb, w.rec, w.prs, adj, w.rng,       \
-                     w.row_cell, w.n_rows, max_rows, band, order, pieces, d_wfs, partial)
+                     w.row_cell, w.n_rows, max_rows, pieces, d_wfs, partial)
     if (d_wfs) {
       if (d.nb == 5) {
         LSIM_ADJ_DENSE(5);

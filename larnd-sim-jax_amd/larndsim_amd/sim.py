@@ -539,11 +539,12 @@ def set_row_waves(w: int):
 
 
 def set_row_cost(pairs: int):
+    """Accepted without effect (a setting of an earlier schedule of the rows)."""
     _lib.check(_lib.load().lsim_set_row_cost(int(pairs)))
 
 
 def set_row_tile(cells: int):
-    """Side of the square pixel-cell tiles the waveform kernel processes rows in (1: row order)."""
+    """Accepted without effect (a setting of an earlier schedule of the rows)."""
     _lib.check(_lib.load().lsim_set_row_tile(int(cells)))
 
 
@@ -572,28 +573,11 @@ def autotune_row_waves(runner: Runner, candidates=(1, 2, 4, 8), reps=3):
 
 
 def autotune_rows(runner: Runner, waves=(1, 2, 4, 8), costs=(64, 256, 1024), tiles=(8, 16, 32), reps=3):
-    """Tune the waveform kernel on the runner's workload, one knob at a time: waves per row
-    workgroup (at the default row cost and tile), then the per-row cost the XCD bands are balanced
-    with, then the side of the cell tiles the rows are processed in (tiled orders only: they time
-    within noise of the plain row order and fetch a third less from HBM).  All three only change
-    the schedule and the per-wave partial sums; the settings stay in effect.  Returns (waves, row
-    cost, tile, {setting: kernel ms})."""
+    """Tune the waveform kernel on the runner's workload: the waves per row workgroup, which change only
+    the schedule and the per-wave partial sums; the setting stays in effect.  ``costs`` and ``tiles``
+    belong to settings without effect, which are left at their defaults.  Returns (waves, row cost, tile,
+    {setting: kernel ms})."""
     set_row_cost(256)
     set_row_tile(16)
-    w, res_w = autotune_row_waves(runner, waves, reps)
-
-    def pick(setter, values):
-        best, best_ms, res = None, None, {}
-        for v in values:
-            setter(v)
-            res[v] = _kernel_ms(runner, reps)
-            if best_ms is None or res[v] < best_ms:
-                best, best_ms = v, res[v]
-        setter(best)
-        return best, res
-
-    c, res_c = pick(set_row_cost, costs)
-    t, res_t = pick(set_row_tile, tiles)
-    return w, c, t, {**{f"waves={k}": v for k, v in res_w.items()}, **{f"row_cost={k}": v for k, v in res_c.items()},
-                     **{f"row_tile={k}": v for k, v in res_t.items()}}
-
+    w, res = autotune_row_waves(runner, waves, reps)
+    return w, 256, 16, {f"waves={k}": v for k, v in res.items()}
