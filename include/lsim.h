@@ -290,6 +290,16 @@ int lsim_param_backward(lsim_ctx *c, const lsim_params *p, const lsim_segments *
                         const void *fee_tape, const float *d_adc, const float *d_z, const float *d_wfs, void *ws,
                         size_t ws_bytes, double *d_params, void *stream);
 
+/* The two kernel sums of the MMD over hit clouds x (weights px) and y (py) whose points interact within an
+ * event, grid and sorting included: out_xx[i] = sum over the x_j, out_xy[i] = sum over the y_j of x_i's event of
+ * k(x_i, .) (w, w x, w y, w z), as lsim_rbf_sums_grid gives them.  x [nx][3], px [nx], y [ny][3], py [ny]
+ * float64 (rounded to float32 for the kernel values), events int64 (of 32 bits), any order; out [nx][4]
+ * float64.  Non-finite coordinates are outside the contract.  Deterministic.  Workspace by the query. */
+int lsim_rbf_mmd_query(int64_t nx, int64_t ny, size_t *ws_bytes);
+int lsim_rbf_mmd_sums(const double *x, const double *px, const int64_t *x_event, int64_t nx, const double *y,
+                      const double *py, const int64_t *y_event, int64_t ny, float sigma, void *ws, size_t ws_bytes,
+                      double *out_xx, double *out_xy, void *stream);
+
 /* The distance beyond which lsim_rbf_sums_grid leaves pairs out (1.01 sqrt(212) sigma); callers size
  * the grid's cells from it (any cell size is correct; about a third of it culls well). */
 float lsim_rbf_cull_radius(float sigma);

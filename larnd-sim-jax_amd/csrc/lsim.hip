@@ -982,10 +982,85 @@ int lsim_rbf_sums_grid(const float* x, const int32_t* x_event, int64_t nx, const
   const dim3 g((unsigned)((nx + kWave - 1) / kWave));
   if (dims == 3)
     hipLaunchKernelGGL(k_rbf_grid<3>, g, dim3(kRbfCols), 0, (hipStream_t)stream, (const float4*)x, x_event, nx,
-                       (const float4*)y, (const float4*)c, y_key, (int32_t)ny, grid, inv, rc, out);
+                       (const float4*)y, (const float4*)c, y_key, (int32_t)ny, grid, inv, rc, (const uint32_t*)nullptr, out);
   else
     hipLaunchKernelGGL(k_rbf_grid<4>, g, dim3(kRbfCols), 0, (hipStream_t)stream, (const float4*)x, x_event, nx,
-                       (const float4*)y, (const float4*)c, y_key, (int32_t)ny, grid, inv, rc, out);
+                       (const float4*)y, (const float4*)c, y_key, (int32_t)ny, grid, inv, rc, (const uint32_t*)nullptr, out);
+  HIP_TRY(hipGetLastError());
+  return LSIM_OK;
+}
+
+namespace {
+struct RbfWs {
+  float *part, *grid;
+  uint32_t *k0, *v0, *k1, *v1;
+  void* sort;
+  float4 *pts, *cols;
+  int64_t* key;
+  int32_t* ev;
+  size_t bytes;
+};
+RbfWs rbf_layout(void* base, int64_t n) {
+  Carve c(base);
+  RbfWs w;
+  w.part = c.take<float>(kRbfBoundBlocks * 6);
+  w.grid = c.take<float>(9);
+  w.k0 = c.take<uint32_t>(n);
+  w.v0 = c.take<uint32_t>(n);
+  w.k1 = c.take<uint32_t>(n);
+  w.v1 = c.take<uint32_t>(n);
+  w.sort = c.take<char>((int64_t)radix_sort_scratch(n));
+  w.pts = c.take<float4>(n);
+  w.cols = c.take<float4>(n);
+  w.key = c.take<int64_t>(n);
+  w.ev = c.take<int32_t>(n);
+  w.bytes = c.off + 256;
+  return w;
+}
+}  // namespace
+
+int lsim_rbf_mmd_query(int64_t nx, int64_t ny, size_t* ws_bytes) {
+  if (!ws_bytes) return fail(LSIM_E_ARG, "NULL argument");
+  if (nx < 0 || ny < 0 || nx + ny >= ((int64_t)1 << 31)) return fail(LSIM_E_ARG, "bad sizes");
+  *ws_bytes = rbf_layout(nullptr, nx + ny).bytes;
+  return LSIM_OK;
+}
+
+int lsim_rbf_mmd_sums(const double* x, const double* px, const int64_t* x_event, int64_t nx, const double* y,
+                      const double* py, const int64_t* y_event, int64_t ny, float sigma, void* ws, size_t ws_bytes,
+                      double* out_xx, double* out_xy, void* stream) {
+  size_t need;
+  const int rc0 = lsim_rbf_mmd_query(nx, ny, &need);
+  if (rc0) return rc0;
+  if (!(sigma > 0.f) || !std::isfinite(sigma)) return fail(LSIM_E_ARG, "sigma must be finite and > 0");
+  if (nx == 0) return LSIM_OK;
+  if (!x || !px || !x_event || !ws || !out_xx || !out_xy || (ny > 0 && (!y || !py || !y_event)))
+    return fail(LSIM_E_ARG, "NULL argument");
+  if (need > ws_bytes) return fail(LSIM_E_SPACE, "workspace too small");
+  hipStream_t st = (hipStream_t)stream;
+  const int64_t n = nx + ny;
+  const RbfWs w = rbf_layout(ws, n);
+  const RbfClouds r{x, px, x_event, nx, y, py, y_event, ny};
+  const float inv = 1.f / (2.f * sigma * sigma), rc = lsim_rbf_cull_radius(sigma);
+  const dim3 g((unsigned)((n + 255) / 256)), gx((unsigned)((nx + kWave - 1) / kWave));
+  hipLaunchKernelGGL(k_rbf_bounds, dim3(kRbfBoundBlocks), dim3(256), 0, st, r, w.part);
+  hipLaunchKernelGGL(k_rbf_grid_of, dim3(1), dim3(kWave), 0, st, w.part, rc, w.grid);
+  uint32_t *ka = w.k0, *va = w.v0, *kb = w.k1, *vb = w.v1;
+  const int bits[3] = {kRbfCellBits, 32, 1};
+  for (int s = 0; s < 3; ++s) {
+    hipLaunchKernelGGL(k_rbf_keys, g, dim3(256), 0, st, r, w.grid, s, s ? (const uint32_t*)va : (const uint32_t*)nullptr, ka, va);
+    hipError_t err;
+    if (radix_sort_pairs(ka, va, kb, vb, n, bits[s], w.sort, st, &err)) {
+      std::swap(ka, kb);
+      std::swap(va, vb);
+    }
+    HIP_TRY(err);
+  }
+  hipLaunchKernelGGL(k_rbf_gather, g, dim3(256), 0, st, r, w.grid, va, w.pts, w.cols, w.key, w.ev);
+  hipLaunchKernelGGL(k_rbf_grid<3>, gx, dim3(kRbfCols), 0, st, w.pts, w.ev, nx, w.pts, w.cols, w.key, (int32_t)nx, w.grid,
+                     inv, rc, va, out_xx);
+  hipLaunchKernelGGL(k_rbf_grid<3>, gx, dim3(kRbfCols), 0, st, w.pts, w.ev, nx, w.pts + nx, w.cols + nx, w.key + nx,
+                     (int32_t)ny, w.grid, inv, rc, va, out_xy);
   HIP_TRY(hipGetLastError());
   return LSIM_OK;
 }

@@ -22,7 +22,7 @@ EXPORTS = (
     "lsim_backward_query", "lsim_backward", "lsim_backward_wfs", "lsim_set_row_waves", "lsim_set_row_cost",
     "lsim_set_row_tile",
     "lsim_segment_records", "lsim_timing", "lsim_timing_read", "lsim_rbf_sums", "lsim_rbf_sums_grid",
-    "lsim_rbf_cull_radius", "lsim_nearest", "lsim_chop_query", "lsim_chop_count", "lsim_chop_fill",
+    "lsim_rbf_mmd_query", "lsim_rbf_mmd_sums", "lsim_rbf_cull_radius", "lsim_nearest", "lsim_chop_query", "lsim_chop_count", "lsim_chop_fill",
     "lsim_prob_fee_query", "lsim_prob_fee", "lsim_prob_fee_backward", "lsim_sdtw_query", "lsim_sdtw",
     "lsim_param_electrons", "lsim_param_rows", "lsim_param_backward_query", "lsim_param_backward",
 )
@@ -119,6 +119,8 @@ def load(path: str = LIB_PATH):
         "lsim_timing_read": [C.POINTER(C.c_double), C.POINTER(i64)],
         "lsim_rbf_sums": [vp, i64, vp, vp, vp, vp, i64, C.c_float, vp, vp],
         "lsim_rbf_sums_grid": [vp, vp, i64, vp, vp, vp, i64, vp, i32, C.c_float, vp, vp],
+        "lsim_rbf_mmd_query": [i64, i64, C.POINTER(sz)],
+        "lsim_rbf_mmd_sums": [vp, vp, vp, i64, vp, vp, vp, i64, C.c_float, vp, sz, vp, vp, vp],
         "lsim_nearest": [vp, i64, vp, vp, vp, i64, i64, vp, vp, vp],
         "lsim_prob_fee_query": [i64, i32, i32, i32, C.POINTER(sz)],
         "lsim_prob_fee": [vp, i64, i32, i32, i32, i32, C.c_float, C.c_float, C.c_float, C.c_float, vp, sz, vp, vp, vp],

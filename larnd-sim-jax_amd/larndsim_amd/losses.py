@@ -143,6 +143,28 @@ def _block_sums(x, ex, y, ey, c, sigma, dims=3):
     return out
 
 
+def _mmd_sums_hip(x, px, ex, y, py, ey, sigma):
+    """Both kernel sums of the MMD for float64 clouds (lsim_rbf_mmd_sums, no host synchronisation): per point of
+    x, the sums of (p, p x) over x and of (py, py y) over y, within its event."""
+    import ctypes as C
+
+    from . import _lib
+
+    lib = _lib.load()
+    x, px, y, py = (t.contiguous() for t in (x, px, y, py))
+    ex, ey = ex.to(torch.int64).contiguous(), ey.to(torch.int64).contiguous()
+    N, M = x.shape[0], y.shape[0]
+    sz = C.c_size_t()
+    _lib.check(lib.lsim_rbf_mmd_query(N, M, C.byref(sz)))
+    ws = torch.empty(int(sz.value), dtype=torch.uint8, device=x.device)
+    kx, ky = torch.empty((2, N, 4), dtype=torch.float64, device=x.device)
+    st = C.c_void_p(torch.cuda.current_stream(x.device).cuda_stream)
+    ptr = lambda t: C.c_void_p(t.data_ptr())  # noqa: E731
+    _lib.check(lib.lsim_rbf_mmd_sums(ptr(x), ptr(px), ptr(ex), N, ptr(y), ptr(py), ptr(ey), M, C.c_float(float(sigma)),
+                                     ptr(ws), ws.numel(), ptr(kx), ptr(ky), st))
+    return kx, ky
+
+
 class _BlockMMDTerms(torch.autograd.Function):
     """Kernel sums of the event-blocked RBF MMD without keeping the kernel matrices.
 
@@ -153,7 +175,7 @@ class _BlockMMDTerms(torch.autograd.Function):
     K (px x), K_xy py, K_xy (py y)) kept from the forward.  Gradients flow to x and px (the
     simulated hits); the target cloud is a constant.  Kernel values are evaluated in float32
     (relative error ~1e-7 per term), sums in float64.  On the GPU the sums come from the HIP
-    kernel lsim_rbf_sums (one pass, no host synchronisation); CPU tensors use chunked torch code.
+    kernels of lsim_rbf_mmd_sums (no host synchronisation); CPU tensors use chunked torch code.
     """
 
     @staticmethod
@@ -163,8 +185,7 @@ class _BlockMMDTerms(torch.autograd.Function):
         inv = 1.0 / (2.0 * sigma * sigma)
         N = x.shape[0]
         if x.is_cuda:
-            kx = _block_sums(x, ex, x, ex, torch.cat([px[:, None], px[:, None] * x], dim=1), sigma)
-            ky = _block_sums(x, ex, y, ey, torch.cat([py[:, None], py[:, None] * y], dim=1), sigma)
+            kx, ky = _mmd_sums_hip(x, px, ex, y, py, ey, sigma)
             A = (px * kx[:, 0]).sum()
             C = (px * ky[:, 0]).sum()
             ctx.save_for_backward(x, px, kx, ky)
