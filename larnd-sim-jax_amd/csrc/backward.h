@@ -19,10 +19,9 @@
 namespace lsim {
 
 constexpr int kNGrad = 7;
-#ifndef LSIM_ADJ_WAVES
-#define LSIM_ADJ_WAVES 4
-#endif
-constexpr int kAdjWaves = LSIM_ADJ_WAVES;  // waves per pixel-row workgroup of the adjoint
+// waves per pixel-row workgroup of the adjoint; the bins' pass has few pairs a row (2 waves 414, 4 476, 1 556 us
+// for 200k segments, where the stripes' takes 403, 352 and 490)
+constexpr int kAdjWaves = 4, kAdjNearWaves = 2;
 
 __device__ __forceinline__ double readlane_d(double v, int j) {
   const int lo = __builtin_amdgcn_readlane(__double2loint(v), j);
@@ -356,11 +355,11 @@ __device__ __forceinline__ void stripe_adjoint(const Dev& d, const Tables& tb, i
 
 // The diffusion bins of x-bin i (and every later x-bin with the same LUT cell, merged into it)
 // landing on pixel offset (a, b), |a|, |b| <= 1: d loss / d (n_e, f, sigma_T, lambda) summed over
-// the y bins (only y-bin jsel when jsel >= 0).  false (nothing added) when bin i misses column a
+// the y bins.  false (nothing added) when bin i misses column a
 // or an earlier x-bin has its cell.
 template <int NB>
 __device__ __forceinline__ bool xbin_adjoint(const Dev& d, const Tables& tb, const SegRec& R, const AdjRec* __restrict__ Ap,
-                                             const PairCtx& c, int a, int b, int i, int jsel, const RowG& G, double& gN,
+                                             const PairCtx& c, int a, int b, int i, const RowG& G, double& gN,
                                              double& gF, double& gS, double& gL) {
   constexpr int SYM = (NB - 1) / 2;
   const int L = d.L, nsb = d.nsb, cm = d.cm;
@@ -389,7 +388,7 @@ __device__ __forceinline__ bool xbin_adjoint(const Dev& d, const Tables& tb, con
   const double f = c.f, ne = c.ne;
 #pragma unroll
   for (int jj = 0; jj < NB; ++jj) {
-    if (!oky[jj] || (jsel >= 0 && jj != jsel)) continue;
+    if (!oky[jj]) continue;
     const int64_t cell = ((int64_t)R.idx * cm + cx) * cm + cyv[jj];
     double y1[3], y0[3];
     g_dots<3>(G, tb.CTM + (cell - (int64_t)cm * cm) * (L + 1), tstride, c, L, y1, y0);
@@ -422,18 +421,16 @@ __device__ __forceinline__ void add_chain(const AdjRec* __restrict__ Ap, double 
   }
 }
 
-#ifndef LSIM_ADJ_BIN_ITEMS
-#define LSIM_ADJ_BIN_ITEMS 0
-#endif
-constexpr bool kAdjBinItems = LSIM_ADJ_BIN_ITEMS != 0;  // one work item per diffusion bin (else per x-bin row)
 
 // Stage 2, row-owned: one workgroup per pixel row holds the row's step function in LDS and walks
 // the segments of its neighbourhood cells (the same pairs the forward's waveform kernel visits),
 // every thread taking pairs from the flattened list; fixed-order block reduction to the row's 7
 // partial gradients.  Two passes (separate launches, separate partials): NEAR = false takes the
-// neighbour-only cells (|a| or |b| > 1; little register state, high occupancy), NEAR = true the
-// 3x3 cells with the diffusion bins.  Rows without gradient (no valid hit) exit at once.  (A
-// waveform cotangent takes k_rows_adj_dense instead.)
+// stripes of every offset but the centre (little register state, high occupancy), NEAR = true the
+// diffusion bins of the 3x3 cells.  The stripes of the 8 cells around the centre, when they were items of the
+// second pass beside the bins that mostly miss those cells, kept few lanes of a wave busy (near and far
+// 575 + 319 -> 414 + 352 us for 200k segments; a side pair's bins as one item: 878).  Rows without
+// gradient (no valid hit) exit at once.  (A waveform cotangent takes k_rows_adj_dense instead.)
 template <int NB, int WAVES, bool NEAR>
 __global__ __launch_bounds__(WAVES * kWave) __attribute__((amdgpu_waves_per_eu(4))) void k_rows_adj(Dev d, Tables tb, const SegRec* __restrict__ rec,
                                                             const PairRec* __restrict__ prs,
@@ -486,9 +483,10 @@ __global__ __launch_bounds__(WAVES * kWave) __attribute__((amdgpu_waves_per_eu(4
   const RowG G{spx, spc, sdc, qlut, np};
   list_cells<NT>(
       d, rng, row_cell[r],
-      [](int a, int b) {
-        const bool near = a >= -1 && a <= 1 && b >= -1 && b <= 1;
-        return near == NEAR ? 0 : -1;
+      [&](int a, int b) {
+        const bool centre = a == 0 && b == 0;
+        if (NEAR) return centre ? 0 : (a >= -1 && a <= 1 && b >= -1 && b <= 1 ? 1 : -1);
+        return !centre && a >= -d.nn && a <= d.nn && b >= -d.nn && b <= d.nn ? 0 : -1;
       },
       [&](int b, int e) {
         int lo = b, hi = e;  // the first dead pair of [b, e)
@@ -505,14 +503,10 @@ __global__ __launch_bounds__(WAVES * kWave) __attribute__((amdgpu_waves_per_eu(4
   for (int k = 0; k < kNGrad; ++k) g[k] = 0.0;
   const int nct = ncls[2];
   const int tot = c_cum[nct];
-  // work items: a far pair is one item (its stripe); a near pair is NX + 1 items on consecutive
-  // threads, its diffusion bins by x-bin row (NX = NB) or one by one (NX = NB * NB), and its stripe
-  constexpr int NX = kAdjBinItems ? NB * NB : NB;
-  constexpr int NI = NEAR ? NX + 1 : 1;
   int cur = 0;
   const int lane = t & (kWave - 1), wid = t / kWave;
   if (!NEAR) {
-    // far pairs: the stripe only.  Each thread fetches its next pair's record (the first 16 bytes
+    // stripes, one item a pair.  Each thread fetches its next pair's record (the first 16 bytes
     // of the pair record) and chain factors while the current pair's table loads are in flight.
     struct FarItem {
       int4 P;  // S, ne, f, flags
@@ -550,27 +544,22 @@ __global__ __launch_bounds__(WAVES * kWave) __attribute__((amdgpu_waves_per_eu(4
       x = y;
     }
   }
-  for (int it = t; NEAR && it < tot * NI; it += NT) {
-    const int i = it / NI, part = it - i * NI;
+  // diffusion bins: a pair is NB items on consecutive threads, by x-bin row; few side pairs are reached by any
+  for (int it = t; NEAR && it < tot * NB; it += NT) {
+    const int i = it / NB, part = it - i * NB;
     while (i >= c_cum[cur + 1]) ++cur;
     const int s = c_beg[cur] + (i - c_cum[cur]);
-    const int ab = c_ab[cur];
-    const int a = (ab >> 8) - 64, b = (ab & 255) - 64;
-    double gN = 0.0, gF = 0.0, gS = 0.0, gL = 0.0;
-    PairCtx pc;
+    const int a = (c_ab[cur] >> 8) - 64, b = (c_ab[cur] & 255) - 64;
+    const int uv = prs[s].flags;
+    if (!bins_reach<NB>((uv >> 8) & 255, a, d.nsb) || !bins_reach<NB>((uv >> 16) & 255, b, d.nsb)) continue;
     const SegRec R = rec[s];
     if (R.ne == 0.f) continue;
     const int S = d.nt - d.L - R.k0;
     if (pair_dead(S, G)) continue;
+    PairCtx pc;
     pair_ctx(d, S, R.ne, R.f, G, pc);
-    if (part == NX) {
-      if ((a == 0 && b == 0) || a < -d.nn || a > d.nn || b < -d.nn || b > d.nn) continue;  // no stripe there
-      stripe_adjoint(d, tb, R.uxy & 0xffff, R.uxy >> 16, pc, a, b, G, gN, gF);
-    } else if (!xbin_adjoint<NB>(d, tb, R, adj + s, pc, a, b, kAdjBinItems ? part / NB : part,
-                                 kAdjBinItems ? part % NB : -1, G, gN, gF, gS, gL)) {
-      continue;
-    }
-    add_chain(adj + s, gN, gF, gS, gL, NEAR, g);
+    double gN = 0.0, gF = 0.0, gS = 0.0, gL = 0.0;
+    if (xbin_adjoint<NB>(d, tb, R, adj + s, pc, a, b, part, G, gN, gF, gS, gL)) add_chain(adj + s, gN, gF, gS, gL, true, g);
   }
 #pragma unroll
   for (int k = 0; k < kNGrad; ++k) {

@@ -794,7 +794,7 @@ static int backward_impl(lsim_ctx* c, const lsim_params* p, const lsim_segments*
 #define LSIM_ADJ_LAUNCH(NBV)                                                                                        \
   hipLaunchKernelGGL((k_rows_adj<NBV, kAdjWaves, false>), grid, block, 0, st, d, tb, w.rec, w.prs, adj, w.rng,       \
                      w.row_cell, w.n_rows, max_rows, pieces, partial);                               \
-  hipLaunchKernelGGL((k_rows_adj<NBV, kAdjWaves, true>), grid, block, 0, st, d, tb, w.rec, w.prs, adj, w.rng,        \
+  hipLaunchKernelGGL((k_rows_adj<NBV, kAdjNearWaves, true>), grid, dim3(kAdjNearWaves * kWave), 0, st, d, tb, w.rec, w.prs, adj, w.rng,        \
                      w.row_cell, w.n_rows, max_rows, pieces, pnear)
 #define LSIM_ADJ_DENSE(NBV)                                                                                       \
   hipLaunchKernelGGL((k_rows_adj_dense<NBV, kAdjWaves>), grid, block, 0, st, d, tb, w.rec, w.prs, adj, w.rng,       \
