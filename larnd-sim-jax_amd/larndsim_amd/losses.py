@@ -150,6 +150,9 @@ def _mmd_sums_hip(x, px, ex, y, py, ey, sigma):
 
     from . import _lib
 
+    for p, w, e in ((x, px, ex), (y, py, ey)):
+        if p.dim() != 2 or p.shape[1] != 3 or w.shape != p.shape[:1] or e.shape != p.shape[:1]:
+            raise ValueError("clouds must be (N, 3) with a weight and an event per point")
     lib = _lib.load()
     x, px, y, py = (t.contiguous() for t in (x, px, y, py))
     ex, ey = ex.to(torch.int64).contiguous(), ey.to(torch.int64).contiguous()
