@@ -695,9 +695,9 @@ def main():
     ap.add_argument("--steps", type=int, default=20)
     ap.add_argument("--warmup", type=int, default=3)
     ap.add_argument("--waves", type=int, default=0, help="waves per row workgroup (0 = autotune)")
-    ap.add_argument("--row-tile", type=int, default=16, help="cell tile of the row order (with --waves)")
+    ap.add_argument("--row-tile", type=int, default=16, help="accepted without effect")
     ap.add_argument("--row-cost", type=int, default=256,
-                    help="per-row cost (pairs) of the XCD band cuts when --waves is given (else autotuned)")
+                    help="accepted without effect")
     ap.add_argument("--no-cpu", action="store_true")
     ap.add_argument("--no-bwd", action="store_true")
     ap.add_argument("--no-batched-bwd", action="store_true", help="skip the batched forward+backward of 32 events")
