@@ -155,7 +155,8 @@ inline hipError_t exclusive_scan(const T* in, T* out, int64_t n, T* tmp, TT* tot
 // Three sizes, each bound by the latency of its steps rather than by the 16 bytes an item moves per pass:
 //   n <= 4096            all passes in one workgroup with the items in LDS: one launch instead of 3 a pass
 //                        (the sorts of a 1k-segment call 124 -> 34 us);
-//   n <= 256 tiles of 8  two launches a pass, R = 1 .. 8 such that there are at most 256 tiles (many small
+//   up to 524288 (256 tiles of 8 rounds)
+//                        two launches a pass, R = 1 .. 8 such that there are at most 256 tiles (many small
 //                        tiles in flight); a tile sums the histograms of those before it as it starts
 //                        (256 KB from L2 at most), which saves the scan's one to three launches
 //                        (200k segments 190 -> 98 us, 30k 128 -> 62);
@@ -164,7 +165,6 @@ inline hipError_t exclusive_scan(const T* in, T* out, int64_t n, T* tmp, TT* tot
 constexpr int kSortThreads = 256;
 constexpr int kSortWaves = kSortThreads / kWave;
 constexpr int kSortRounds = 8;  // the most
-constexpr int kSortTile = kSortThreads * kSortRounds;
 constexpr int kRadix = 256;
 constexpr int kSortSumTiles = 256;
 constexpr int kSumBatch = 32;
