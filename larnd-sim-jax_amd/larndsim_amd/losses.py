@@ -153,8 +153,10 @@ def _mmd_sums_hip(x, px, ex, y, py, ey, sigma):
     for p, w, e in ((x, px, ex), (y, py, ey)):
         if p.dim() != 2 or p.shape[1] != 3 or w.shape != p.shape[:1] or e.shape != p.shape[:1]:
             raise ValueError("clouds must be (N, 3) with a weight and an event per point")
+        if not (p.device == w.device == e.device == x.device):
+            raise ValueError("both clouds, their weights and events must be on one device")
     lib = _lib.load()
-    x, px, y, py = (t.contiguous() for t in (x, px, y, py))
+    x, px, y, py = (t.to(torch.float64).contiguous() for t in (x, px, y, py))
     ex, ey = ex.to(torch.int64).contiguous(), ey.to(torch.int64).contiguous()
     N, M = x.shape[0], y.shape[0]
     sz = C.c_size_t()
