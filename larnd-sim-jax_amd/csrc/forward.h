@@ -6,23 +6,11 @@
 
 namespace lsim {
 
-// Window tables of the waveform adjoint are zero padded: P[p] = W[p - 2] for 2 <= p < L + 2 and 0
+// Window tables of the raw response are zero padded: P[p] = W[p - 2] for 2 <= p < L + 2 and 0
 // elsewhere, kWinPad entries per series, read without bounds tests (windows up to kMaxWindow samples).
 constexpr int kWinPad = 3 * kWave;
 constexpr int kMaxWindow = kWinPad - 5;
 constexpr int kXcd = 8;  // XCDs of an MI355X (workgroup i runs on XCD i % 8)
-
-// Raw-response windows as the stripe accumulation reads them: row (cx, cy) of `stripe_stride(L)` floats
-// holds kStripeLead zeros and then the L samples, and zeros follow up to the stride; the next row's
-// leading zeros serve as this row's tail.  The last of the leading zeros (sample -1) is kStripeMark:
-// the window's tick of the boundary correction, whose value depends on the segment and is put in
-// its place by the reader.  One more row, of zeros, follows the table.
-constexpr int kStripeLead = kWave;
-constexpr uint32_t kStripeMark = 0x7fa5c3e1u;
-__host__ __device__ inline int stripe_stride(int L) { return kStripeLead + (L > 2 * kWave ? L : 2 * kWave); }
-__host__ __device__ inline int64_t stripe_floats(int lx, int ly, int L) {
-  return ((int64_t)lx * ly + 1) * stripe_stride(L) + kWave;
-}
 
 // Per-segment record of the window paths (sorted order): window start, charge, fractional tick and
 // sub-bin position.
@@ -96,10 +84,10 @@ __global__ void k_cell_keys(Dev d, SegIn in, const uint32_t* __restrict__ vals, 
 // 2. records in cell order, cell ranges, pixel rows
 // ------------------------------------------------------------------------------------------
 
-// Boundary corrections of every (row offset, segment) pair of record R per unit charge, written where
-// the record is built: dtot[ab][i] = D.x - f D.y of the neighbour stripe (raw response, unless the
-// offset is (0, 0)) plus, for |a|, |b| <= 1, the sum over the diffusion bins landing on that row of
-// w_bin (D.x - f D.y) of the idx template (sim_jax.py:227-261), D = (C[nt-L] - C[k0],
+// Boundary corrections of every (row offset, segment) pair of record R, written where the record
+// is built: dtot[ab][i] = n_e (D.x - f D.y) of the neighbour stripe (raw response, unless the offset
+// is (0, 0)) plus, for |a|, |b| <= 1, the sum over the diffusion bins landing on that row of
+// n_bin (D.x - f D.y) of the idx template (sim_jax.py:227-261), D = (C[nt-L] - C[k0],
 // C[k0+1] - C[k0]), ab = (a + n)(2n + 1) + (b + n).  The D tables are tick-major, so all of one
 // segment's entries lie in the tick-k0 plane; the waveform kernels then read dtot[ab][cell range]
 // contiguously.
@@ -163,7 +151,7 @@ __device__ __forceinline__ void seg_corrections(const Dev& d, const float2* __re
       const int ab = ab0 + u;
       const int a = ab / W - d.ne, b = ab % W - d.ne;
       const bool on = ab < WW && (a != 0 || b != 0) && a >= -d.nn && a <= d.nn && b >= -d.nn && b <= d.nn;
-      dl[u] = on ? D[u].x - f * D[u].y : 0.f;
+      dl[u] = on ? R.ne * (D[u].x - f * D[u].y) : 0.f;
     }
 #pragma unroll
     for (int u = 0; u < kCorrBatch; ++u) {
@@ -187,7 +175,7 @@ __device__ __forceinline__ void seg_corrections(const Dev& d, const float2* __re
   for (int k = 0; k < NB; ++k) {
     const int vx = ux + k - SYM;
     const int dx = vx < 0 ? -1 : (vx >= nsb ? 1 : 0);
-    const float wxs = R.wx[k];
+    const float wxs = R.ne * R.wx[k];
     const int cx = offset_bin(vx - dx * nsb, 0, nsb);
     float2 D[NB];
     float c[NB];
@@ -334,7 +322,6 @@ struct Tables {
   const float* TMW;   // [cm][cm][nm][bin_stride(L)] the same, two zeros before each window (and after the last)
   const float* TN;    // [lx][ly][L]       raw response window (neighbours)
   const float* TNP;   // [lx][ly][kWinPad] the same, padded
-  const float* TNQ;   // the same as stripe_floats() values (kStripeMark in each row's sample -1)
   const float2* DM;   // [nt][nm][cm][cm]  (C[nt-L]-C[k], C[min(k+1,nt-1)]-C[k]) of template m (tick-major)
   const float2* DN;   // [nt][lx][ly]      same for the raw response
   const double* CTM;  // [nm][cm][cm][L+1] window prefix sums (adjoint)
@@ -576,34 +563,36 @@ __device__ __forceinline__ float lane_next0(float v) {
 }
 
 // Store of a whole window V held three samples per lane: lane l holds V[3 l - 2 + k] in vk, zero outside
-// 0 <= m < L, for 3 l < L + 2.  Output m receives (1-f) V[m] + f V[m+1]; delta is the boundary correction.
-// `interior` windows (2 <= S and S + L <= nout) need no tick checks.
-__device__ __forceinline__ void store_window(float* accw, int lane, float v0, float v1, float v2, float omf, float f,
-                                             float delta, int S, int L, int nout, bool interior) {
+// 0 <= m < L, for 3 l < L + 2 (the lanes that call it).  Output m receives so V[m] + sf V[m+1], and outputs -1 and -2
+// their boundary corrections d1 and d2.  INSIDE windows (2 <= S and S + L <= nout) need no tick checks.
+//
+// The rounding is fixed: fma(so, V[m], sf V[m+1]), then the correction, then the row's tick.  d1 and d2 come rounded
+// except that in windows that reach the row's ends a FUSED one is the multiply-add of its factors (so, sf) and delta.
+template <bool INSIDE, bool FUSED>
+__device__ __forceinline__ void store_window(float* accw, int lane, float v0, float v1, float v2, float so, float sf,
+                                             float d1, float d2, float delta, int S, int L, int nout) {
+#pragma clang fp contract(off)
   const float nx = lane_next0(v0);
   const int m = 3 * lane - 2;
-  float c0 = omf * v0 + f * v1, c1 = omf * v1 + f * v2, c2 = omf * v2 + f * nx;
-  if (interior) {
-    c0 += lane == 0 ? f * delta : 0.f;
-    c1 += lane == 0 ? omf * delta : 0.f;
-    if (m < L) {
-      float* p = accw + S + m;
-      const float a0 = p[0], a1 = p[1], a2 = p[2];
-      p[0] = a0 + c0;
-      p[1] = a1 + (m + 1 < L ? c1 : 0.f);
-      p[2] = a2 + (m + 2 < L ? c2 : 0.f);
-    }
+  float c0 = __builtin_fmaf(so, v0, sf * v1), c1 = __builtin_fmaf(so, v1, sf * v2), c2 = __builtin_fmaf(so, v2, sf * nx);
+  float* p = accw + S + m;
+  if (INSIDE) {
+    const float first = lane == 0 ? 1.f : 0.f;
+    const float a0 = p[0], a1 = p[1], a2 = p[2];
+    c0 = __builtin_fmaf(d2, first, c0);
+    c1 = __builtin_fmaf(d1, first, c1);
+    p[0] = a0 + c0;
+    p[1] = a1 + c1;
+    p[2] = a2 + c2;
   } else {
 #pragma unroll
     for (int k = 0; k < 3; ++k) {
       const int o = S + m + k;
       if (m + k < L && o >= 0 && o < nout) {
         float val = o >= 1 ? (k == 0 ? c0 : (k == 1 ? c1 : c2)) : 0.f;
-        if (o <= nout - 2) {
-          if (m + k == -1) val += omf * delta;
-          if (m + k == -2) val += f * delta;
-        }
-        accw[o] += val;
+        if (o <= nout - 2 && m + k == -1) val = FUSED ? __builtin_fmaf(so, delta, val) : val + d1;
+        if (o <= nout - 2 && m + k == -2) val = FUSED ? __builtin_fmaf(sf, delta, val) : val + d2;
+        p[k] += val;
       }
     }
   }
@@ -612,111 +601,29 @@ __device__ __forceinline__ void store_window(float* accw, int lane, float v0, fl
 // 0x00020000: word 3 of a raw (stride 0) buffer descriptor on gfx9-family GPUs.
 constexpr int kBufDesc3 = 0x00020000;
 
-// ---- neighbour stripes of one row: pairs sorted by time chunk, accumulated chunk by chunk ----
-//
-// Output tick o of the row receives, from every pair, (1-f) n_e V[o - S] + f n_e V[o - S + 1], V the raw
-// window with the unit-charge boundary correction as its sample -1.  With
-//   A0[o] = sum so V[o - S],  A1[o] = sum sf V[o - S],  so = n_e (1-f), sf = n_e f,
-// the row is A0[o] + A1[o + 1], so a lane that owns tick o needs one sample of each pair: no
-// lane shift per pair and no read-modify-write of LDS per pair, which a wave that owns the pair needs.
-// Ticks are cut into chunks of 64 (position o + kTickOff, chunk position / 64); a pair whose first
-// position S - 1 lies in chunk b reaches chunks b .. b + 2, and b + 3 when it starts late enough in b
-// (r = position % 64 >= 192 - L).  The pairs of a batch are therefore counting-sorted in LDS by
-// 2 b + (reaches b + 3): those of chunk c are one contiguous run, the last part of it (b = c) holding
-// the samples -1.
-//
-// Per (pair, chunk): one 4-byte LDS read (lane l takes word l % 4 of the 16-byte entry; each word
-// reaches its use by a quad broadcast folded into the instruction), one 256-byte window load from L2 or
-// L1, an address add and two multiply-adds.
-constexpr int kTickOff = 3 * kWave;                         // S >= 1 - L > -kTickOff
-constexpr int kRowChunks = kMaxOut / kWave + 1;             // output chunks of the longest row, and tick nout of A1
-constexpr int kStripeKeys = 2 * (kRowChunks + 3);           // 2 b + late, b < kRowChunks + 3
-constexpr int kKeyOdd = kStripeKeys;                        // non-finite factors (handled tick by tick)
-constexpr int kKeyNone = kStripeKeys + 1;                   // not listed (no charge, or past the row)
-constexpr int kStripeRounds = 6;                            // pairs per lane and batch
-static_assert((kStripeKeys & 1) == 0 && kStripeKeys / 2 + 1 <= kWave, "one lane per pair of keys");
+constexpr int kFarGroup = 8;  // pairs whose windows a wave has in flight (128 events of 72k segments: 4 56.9, 8 55.3, 16 54.6 ms)
 
-struct __align__(16) StripeEnt {
-  int addr;       // byte offset into TNQ at position 0: 4 (row stride + kStripeLead - kTickOff - S)
-  float so, sf;   // n_e (1 - f), n_e f
-  float D;        // boundary correction per unit charge (kKeyOdd: S)
-};
-
-template <int K>
-__device__ __forceinline__ int quad_word(int v) {  // word K of the lane's quad in every lane of it
-  return __builtin_amdgcn_mov_dpp(v, K * 0x55, 0xf, 0xf, true);
-}
-
-// N entries at ent (lane l's word): their shares of the lane's position (pos4 = 4 * position).  HEAD:
-// chunks that may hold a pair's sample -1.  n < N: the entries from n on repeat entry n - 1 with no
-// charge.  Four sums of each kind, so that a sum's float32 rounding is that of a chain a quarter as long (the
-// rows' error against float64 is that of per-wave partial rows: 7e-8 of their norm).
-constexpr int kStripeSums = 4;
-struct StripeSums {
-  float a0[kStripeSums] = {}, a1[kStripeSums] = {};
-};
-
-template <int N, bool HEAD>
-__device__ __forceinline__ void stripe_group(__amdgpu_buffer_rsrc_t tnq, const int* ent, int n, bool is_addr, int pos4,
-                                             StripeSums& A) {
-  int w[N];
-#pragma unroll
-  for (int g = 0; g < N; ++g) {
-    w[g] = ent[4 * (g < n ? g : n - 1)];
-    if (g >= n && !is_addr) w[g] = 0;
-  }
-  int v[N];
-#pragma unroll
-  for (int g = 0; g < N; ++g) v[g] = __builtin_amdgcn_raw_buffer_load_b32(tnq, pos4 + quad_word<0>(w[g]), 0, 0);
-#pragma unroll
-  for (int g = 0; g < N; ++g) {
-    if (HEAD) {
-      const int corr = quad_word<3>(w[g]);  // taken by every lane: a lane reads its quad, active or not
-      v[g] = v[g] == (int)kStripeMark ? corr : v[g];
-    }
-    float &a0 = A.a0[g % kStripeSums], &a1 = A.a1[g % kStripeSums];
-    a0 = __builtin_fmaf(__int_as_float(quad_word<1>(w[g])), __int_as_float(v[g]), a0);
-    a1 = __builtin_fmaf(__int_as_float(quad_word<2>(w[g])), __int_as_float(v[g]), a1);
-  }
-}
-
-template <bool HEAD>
-__device__ __forceinline__ void stripe_run(__amdgpu_buffer_rsrc_t tnq, const StripeEnt* list, int e, int e1, int lane,
-                                           int pos4, StripeSums& A) {
-  const int* ent = reinterpret_cast<const int*>(list) + (lane & 3);
-  const bool is_addr = (lane & 3) == 0;
-  for (; e1 - e >= 16; e += 16) stripe_group<16, HEAD>(tnq, ent + 4 * e, 16, is_addr, pos4, A);
-  if (e1 - e >= 8) {
-    stripe_group<8, HEAD>(tnq, ent + 4 * e, 8, is_addr, pos4, A);
-    e += 8;
-  }
-  if (e1 - e >= 4) {
-    stripe_group<4, HEAD>(tnq, ent + 4 * e, 4, is_addr, pos4, A);
-    e += 4;
-  }
-  if (e < e1) stripe_group<4, HEAD>(tnq, ent + 4 * e, e1 - e, is_addr, pos4, A);
-}
-
-// A pair with a non-finite factor at output tick o: what storing its whole padded window leaves there
+// A pair with a non-finite factor (window T) at output tick o: what storing its whole padded window leaves there
 // (a non-finite charge times the padding's zeros is NaN from S - 2 to S + 186 of an interior window).
-__device__ __forceinline__ float odd_pair(const float* __restrict__ TNQ, const StripeEnt& E, int o, int L, int nout) {
-  const int S = __float_as_int(E.D), m = o - S;
+__device__ __forceinline__ float odd_pair(const float* __restrict__ T, float so, float sf, int S, int o, int L, int nout) {
+  const int m = o - S;
   const bool interior = S >= 2 && S + L <= nout;
   if (m < -2 || m > (interior ? 3 * (kWave - 1) - 3 : L - 1)) return 0.f;
-  const float* T = TNQ + E.addr + kStripeLead;
   const float v = m >= 0 && m < L ? T[m] : 0.f, vn = m + 1 >= 0 && m + 1 < L ? T[m + 1] : 0.f;
-  float val = interior || o >= 1 ? E.so * v + E.sf * vn : 0.f;
-  if (interior ? m <= kWave - 4 : (m < 0 && o <= nout - 2)) val += 0.f * (E.so + E.sf);
+  float val = interior || o >= 1 ? so * v + sf * vn : 0.f;
+  if (interior ? m <= kWave - 4 : (m < 0 && o <= nout - 2)) val += 0.f * (so + sf);
   return val;
 }
 
 // Distinct LUT cells of a segment's diffusion bins that land on pixel offset a along one axis, with
 // the bins' weights summed per cell: bins on the same cell read the same template window and the
 // bin weights factorise (n_bin = n_e wx wy), so each distinct (cx, cy) is visited once with weight
-// W[i] W[j].  ok[i] marks the distinct entries (slot of the first bin of each cell).
+// W[i] W[j].  ok[i] marks the distinct entries (slot of the first bin of each cell).  Later bins' weights are
+// rounded and added, those of slot 0's cell by multiply-adds.
 template <int NB>
 __device__ __forceinline__ void axis_merge(int u, int a, int nsb, const float* w, float scale, bool* ok, int* cell,
                                            float* W) {
+#pragma clang fp contract(off)
   constexpr int SYM = (NB - 1) / 2;
 #pragma unroll
   for (int i = 0; i < NB; ++i) {
@@ -735,7 +642,7 @@ __device__ __forceinline__ void axis_merge(int u, int a, int nsb, const float* w
 #pragma unroll
     for (int j = 0; j < i; ++j) {
       if (!merged && ok[j] && cell[j] == cc) {
-        W[j] += wi;
+        W[j] = j == 0 ? __builtin_fmaf(scale, w[i], W[j]) : W[j] + wi;
         merged = true;
       }
     }
@@ -759,25 +666,26 @@ __device__ __forceinline__ bool bins_reach(int u, int a, int nsb) {
 // lb T_idx + lc T_{idx+1})[cx][cy][m] (sim_jax.py:186-194), three samples per lane as store_window takes
 // them, each distinct LUT cell once.  `st` holds the merged bins of the two axes, NB each: weights along
 // x (charge included) and y, byte offsets of the cells in TMW along x and y.  Lane i NB + j forms the
-// product of bin i along x and bin j along y; the wave then walks the non-zero ones, four at a time:
-// weight and offset by a lane read, nine multiply-adds, and the three templates' rows (neighbours in TMW)
-// by one 12-byte load per lane each.  TMW (1.5 MB for 100 templates of 150 samples) stays in each XCD's L2.
+// product of bin i along x and bin j along y; the wave then walks the non-zero ones in order, four at a time:
+// weight and offset by a lane read, the three templates' rows (neighbours in TMW) by one 12-byte load per lane
+// each, per sample their interpolation and one multiply-add.  TMW (1.5 MB for 100 templates of 150 samples) stays
+// in each XCD's L2.
 // lane12: 12 * lane for the lanes that hold samples, past the table for the others (they read 0).
 __host__ __device__ inline int bin_stride(int L) { return L + 2; }
 __host__ __device__ inline int64_t bin_floats(int nm, int cm, int L) { return (int64_t)nm * cm * cm * bin_stride(L) + 4; }
 constexpr int kBinItems = 16;  // items whose merged bins a wave stages at a time
 
 template <int NB>
-__device__ __forceinline__ void bins_window(__amdgpu_buffer_rsrc_t tmw, const float* st, int base, int ws4, int lane,
+__device__ __forceinline__ void bins_window(__amdgpu_buffer_rsrc_t tmw, const int* st, int base, int ws4, int lane,
                                             int lane12, float la, float lb, float lc, float& v0, float& v1, float& v2) {
   float c = 0.f;
   int off = 0;
   if (lane < NB * NB) {
     const int i = lane / NB, j = lane - i * NB;
-    c = st[i] * st[NB + j];
-    off = base + __float_as_int(st[2 * NB + i]) + __float_as_int(st[3 * NB + j]);
+    c = __int_as_float(st[i]) * __int_as_float(st[NB + j]);
+    off = base + st[2 * NB + i] + st[3 * NB + j];
   }
-  float A[3] = {0.f, 0.f, 0.f}, B[3] = {0.f, 0.f, 0.f}, C[3] = {0.f, 0.f, 0.f};
+  float V[3] = {0.f, 0.f, 0.f};
   for (uint64_t m = __ballot(c != 0.f); m != 0;) {
     constexpr int G = 4;
     float w[G];
@@ -800,27 +708,22 @@ __device__ __forceinline__ void bins_window(__amdgpu_buffer_rsrc_t tmw, const fl
     for (int g = 0; g < G; ++g) {
 #pragma unroll
       for (int k = 0; k < 3; ++k) {
-        A[k] = __builtin_fmaf(w[g], qa[g][k], A[k]);
-        B[k] = __builtin_fmaf(w[g], qb[g][k], B[k]);
-        C[k] = __builtin_fmaf(w[g], qc[g][k], C[k]);
+        const float T = __builtin_fmaf(lc, qc[g][k], __builtin_fmaf(la, qa[g][k], lb * qb[g][k]));
+        V[k] = __builtin_fmaf(w[g], T, V[k]);
       }
     }
   }
-  v0 = lb * B[0] + la * A[0] + lc * C[0];
-  v1 = lb * B[1] + la * A[1] + lc * C[1];
-  v2 = lb * B[2] + la * A[2] + lc * C[2];
+  v0 = V[0];
+  v1 = V[1];
+  v2 = V[2];
 }
 
-// Dynamic LDS of the waveform kernel: the per-wave partial rows (the stripe list lies over rows 1 and up
-// first; afterwards the rows are reused for the unreset float64 cumulative charge of the tape), then
-// the neighbourhood's cell lists (ncell begins, ncell + 1 cumulative counts, ncell offsets).
-__host__ __device__ inline int stripe_batch(int waves) { return kStripeRounds * kWave * waves; }
-__host__ __device__ inline size_t rows_list_off(int nout, int L) { return ((size_t)(nout + row_pad(L)) * 4 + 15) & ~(size_t)15; }
+// Dynamic LDS of the waveform kernel: the per-wave partial rows (reused afterwards for the unreset
+// float64 cumulative charge of the tape), then the neighbourhood's cell lists (ncell begins, ncell + 1
+// cumulative counts, ncell offsets).
 __host__ __device__ inline size_t rows_acc_bytes(int waves, int nout, int L) {
   const size_t acc = (size_t)waves * (nout + row_pad(L)) * 4, q = (size_t)nout * 8;
-  const size_t list = rows_list_off(nout, L) + (size_t)stripe_batch(waves) * sizeof(StripeEnt);
-  const size_t m = acc > q ? acc : q;
-  return ((m > list ? m : list) + 15) & ~(size_t)15;
+  return ((acc > q ? acc : q) + 15) & ~(size_t)15;
 }
 inline size_t rows_lds_bytes(int waves, int nout, int L, int ncell) {
   return rows_acc_bytes(waves, nout, L) + (size_t)(3 * ncell + 1) * 4;
@@ -1004,13 +907,20 @@ inline int64_t run_grid(int64_t max_rows) {
   return (max_rows + kXcd * kRowRun - 1) / (kXcd * kRowRun) * (kXcd * kRowRun);
 }
 
-// One workgroup per pixel row.  What bounds it (160k rows, 2e8 stripe pairs, 4 waves a row; parts by
-// leaving each out): the stripes' chunk sums 7 of 19 ms (one 4-byte-per-lane load per pair and chunk is near
-// the texture unit's 16 lanes a cycle), the bins' windows 5.5, their counting sort 2.5, the self-trigger 2;
-// occupancy is 4 workgroups a CU by LDS (40 KB).  One wave per pair with a read-modify-write of the row in
-// LDS, and the bins as unrolled scalar code, took 25 to 32 ms for the same rows.
+// One workgroup per pixel row.  Whether a charge within rounding of the threshold crosses it, and so a hit's tick,
+// hangs on the order in which the row's float32 terms are added, so the order is part of the result: wave w sums the
+// pairs of blocks w, w + WAVES, .. of 64 pairs of the far and side cells in pair order (cells in list order, a
+// cell's segments by window and input order), each block's stripes and then its diffusion bins; then the centre
+// cell's segments w, w + WAVES, .. ; then the waves' partial rows are added in order.  (Pairs sorted by time and
+// summed by 64-tick chunks, two multiply-adds a pair and chunk, took 1.20 ms for 200k segments and 50.6 for 128
+// events of 72k, where this order takes 1.32 and 55.3, but moved about one hit in 3 million to another tick.)
+//
+// What bounds it: the issue of vector instructions, 20 a stripe pair (six lane reads of the pair's values, a
+// lane shift, nine for its three samples a lane, two corrections, two addresses), and the bins' 12 multiply-adds a
+// cell; occupancy is 4 workgroups a CU by LDS (38 KB).  The same order with three 4-byte loads and as many lane
+// shifts a pair, a branch on each pair's window and the bins as unrolled scalar code took 1.60 and 67.9 ms.
 template <int NB, int WAVES>
-__global__ __launch_bounds__(WAVES * kWave) void k_rows_fwd(Dev d, Tables tb, const SegRec* __restrict__ rec,
+__global__ __launch_bounds__(WAVES * kWave) __attribute__((amdgpu_waves_per_eu(4))) void k_rows_fwd(Dev d, Tables tb, const SegRec* __restrict__ rec,
                                                             const int2* __restrict__ rng, const int* __restrict__ row_cell,
                                                             const int* __restrict__ n_rows_dev, int64_t max_rows,
                                                             const float* __restrict__ dtot,
@@ -1019,7 +929,7 @@ __global__ __launch_bounds__(WAVES * kWave) void k_rows_fwd(Dev d, Tables tb, co
   extern __shared__ __align__(16) char smem[];
   __shared__ double shd[NT / kWave];
   __shared__ int shi[2][NT / kWave];
-  __shared__ int ncls[3];  // far cells, + the centre cell, + the 8 side cells
+  __shared__ int ncls[3];  // far cells, + the 8 side cells, + the centre cell
 
   const int P0 = *n_rows_dev;
   const int P = P0 < max_rows ? P0 : (int)max_rows;
@@ -1032,7 +942,7 @@ __global__ __launch_bounds__(WAVES * kWave) void k_rows_fwd(Dev d, Tables tb, co
   const int r = (int)row;
   const int nout = d.nout;
   float* acc = (float*)smem;
-  // this row's neighbourhood cells: far cells first, then the 3x3 near cells, in (a, b) order
+  // this row's neighbourhood cells: far, then the 8 side cells, then the centre, each in (a, b) order
   const int ncell = (2 * d.ne + 1) * (2 * d.ne + 1);
   int* const c_beg = (int*)(smem + rows_acc_bytes(WAVES, nout, d.L));
   int* const c_cum = c_beg + ncell;
@@ -1050,237 +960,161 @@ __global__ __launch_bounds__(WAVES * kWave) void k_rows_fwd(Dev d, Tables tb, co
     out.pixel_ids[r] = ((int64_t)evp * d.ny + py) * d.nx + px;
   }
   if (wid == 0) list_cells_fwd(d, rng, cell, lane, c_beg, c_cum, c_ab, ncls);
-  __shared__ int s_hist[kStripeKeys + 2][WAVES];  // counts, then first places, of (key, wave)
-  __shared__ int s_start[kStripeKeys + 2];        // first place of each key
-  __shared__ float s_edge[kRowChunks + 1];        // A1 at each chunk's first tick (belongs to the tick before)
-  __shared__ int s_next;                          // next non-empty chunk to take
-  __shared__ float s_tick0[WAVES];                // what the waves' pairs leave at output tick 0
-  __shared__ float s_bins[WAVES][kBinItems][4 * NB];
-  for (int o = t; o < rstride; o += NT) acc[o] = 0.f;
-  if (t <= kRowChunks) s_edge[t] = 0.f;
+  __shared__ int s_bins[WAVES][kBinItems][4 * NB];
+  {
+    const int nz = WAVES * rstride, n4 = nz / 4;
+    for (int o = t; o < n4; o += NT) reinterpret_cast<float4*>(acc)[o] = make_float4(0.f, 0.f, 0.f, 0.f);
+    for (int o = 4 * n4 + t; o < nz; o += NT) acc[o] = 0.f;
+  }
   __syncthreads();
 
   float* accw = acc + wid * rstride;
   const int nsc = ncls[1], nct = ncls[2];  // far + side cells, all cells
-  const int nsb = d.nsb, L = d.L;
-  // Neighbour stripes of the far and side pairs, flattened over those cells, in batches of
-  // kStripeRounds * 64 pairs per wave.  Lane by lane: the pair's record and correction, its factors,
-  // window and sort key; the batch is counting-sorted (stable: by wave, round, lane) into the list, and
-  // the waves take its non-empty chunks in turn.  A side pair's correction covers its diffusion bins
-  // too (they follow below).
-  float tick0 = 0.f;
-  {
-    const int nfar = c_cum[nsc], side = 2 * d.ne + 1;
-    const int stride = stripe_stride(L), nchunk = nout / kWave + 1;
-    StripeEnt* const list = reinterpret_cast<StripeEnt*>(smem + rows_list_off(nout, L));
-    const __amdgpu_buffer_rsrc_t tnq = __builtin_amdgcn_make_buffer_rsrc(
-        (void*)tb.TNQ, 0, (int)(uint32_t)(stripe_floats(d.lx, d.ly, L) * 4), kBufDesc3);
-    for (int b0 = 0; b0 < nfar; b0 += stripe_batch(WAVES)) {
-      for (int i = t; i < (kStripeKeys + 2) * WAVES; i += NT) (&s_hist[0][0])[i] = 0;
-      __syncthreads();  // also: the last batch's list has been read
-      StripeEnt E[kStripeRounds];
-      int key[kStripeRounds], place[kStripeRounds];
-#pragma unroll
-      for (int q = 0; q < kStripeRounds; ++q) {
-        const int p0 = b0 + (q * WAVES + wid) * kWave, p = p0 + lane;
-        key[q] = kKeyNone;
-        place[q] = 0;
-        if (p0 >= nfar) continue;
-        if (p < nfar) {
-          int lo = 0, hi = nsc - 1;  // the cell holding p: last c with c_cum[c] <= p
-          while (lo < hi) {
-            const int mid = (lo + hi + 1) >> 1;
-            if (c_cum[mid] <= p) lo = mid;
-            else hi = mid - 1;
-          }
-          const int sg = c_beg[lo] + (p - c_cum[lo]);
-          const int ab = c_ab[lo];
-          const int a = (ab >> 8) - 64, b = (ab & 255) - 64;
-          const PairRec P = prs[sg];
-          const float D = dtot[(int64_t)((a + d.ne) * side + (b + d.ne)) * nseg + sg];
-          E[q].D = D;
-          const float omf = 1.f - P.f;
-          E[q].so = P.ne * omf;
-          E[q].sf = P.ne * P.f;
-          if (P.S == 1) tick0 += E[q].so * D;  // the corrections at output tick 0
-          if (P.S == 2) tick0 += E[q].sf * D;
-          if (P.S == nout) E[q].so = 0.f;  // a correction at the last tick is dropped
-          // with no neighbour stripes (nn = 0) a side pixel gets its diffusion bins only: the zero row
-          const bool on = a >= -d.nn && a <= d.nn && b >= -d.nn && b <= d.nn;
-          const int row = on ? offset_bin((P.flags >> 8) & 255, a, nsb) * d.ly + offset_bin((P.flags >> 16) & 255, b, nsb)
-                             : d.lx * d.ly;
-          E[q].addr = (int)(4u * ((uint32_t)row * (uint32_t)stride + (uint32_t)(kStripeLead - kTickOff - P.S)));
-          const int pos = P.S - 1 + kTickOff;
-          key[q] = 2 * (pos / kWave) + ((pos & (kWave - 1)) >= kTickOff - L ? 1 : 0);
-          if (P.ne == 0.f || P.S > nout) key[q] = kKeyNone;
-          if (!(fabsf(E[q].so) + fabsf(E[q].sf) < __builtin_inff())) {
-            key[q] = kKeyOdd;
-            E[q].addr = row * stride;
-            E[q].D = __int_as_float(P.S);
-          }
-        }
-        // place among the wave's pairs of the same key so far
-        uint64_t peers = ~0ull;
-#pragma unroll
-        for (int bt = 0; bt < 7; ++bt) {
-          const bool bit = (key[q] >> bt) & 1;
-          const uint64_t m = __ballot(bit);
-          peers &= bit ? m : ~m;
-        }
-        const int rank = __popcll(peers & ((1ull << lane) - 1));
-        const int before = s_hist[key[q]][wid];
-        __builtin_amdgcn_wave_barrier();  // wave-local LDS: program order
-        if (rank == 0) s_hist[key[q]][wid] = before + __popcll(peers);
-        __builtin_amdgcn_wave_barrier();
-        place[q] = before + rank;
-      }
-      __syncthreads();
-      if (wid == 0) {
-        if (lane == 0) s_next = 0;
-        // lane l: keys 2 l and 2 l + 1
-        int n[2] = {0, 0};
-#pragma unroll
-        for (int h = 0; h < 2; ++h)
-          if (2 * lane + h < kKeyNone)
-            for (int w = 0; w < WAVES; ++w) n[h] += s_hist[2 * lane + h][w];
-        int inc = n[0] + n[1];
-#pragma unroll
-        for (int dd = 1; dd < kWave; dd <<= 1) {
-          const int u = __shfl_up(inc, dd, kWave);
-          if (lane >= dd) inc += u;
-        }
-        int at = inc - n[0] - n[1];
-#pragma unroll
-        for (int h = 0; h < 2; ++h) {
-          const int k = 2 * lane + h;
-          if (k <= kKeyNone) s_start[k] = at;
-          if (k < kKeyNone)
-            for (int w = 0; w < WAVES; ++w) {
-              const int c = s_hist[k][w];
-              s_hist[k][w] = at;
-              at += c;
-            }
-        }
-      }
-      __syncthreads();
-#pragma unroll
-      for (int q = 0; q < kStripeRounds; ++q)
-        if (key[q] < kKeyNone) list[s_hist[key[q]][wid] + place[q]] = E[q];
-      __syncthreads();
-      // lane k: does output chunk k hold anything?  The waves take the non-empty ones as they come free
-      // (whichever wave takes a chunk adds the same pairs in the same order).
-      const int kk = lane < nchunk ? lane : 0;
-      uint64_t todo = __ballot(lane < nchunk && s_start[2 * kk + 8] > s_start[2 * kk + 1]);
-      for (int turn = 0;;) {
-        int mine = 0;
-        if (lane == 0) mine = atomicAdd(&s_next, 1);
-        mine = __builtin_amdgcn_readfirstlane(mine);
-        for (; turn < mine && todo != 0; ++turn) todo &= todo - 1;
-        if (todo == 0) break;
-        const int k = __builtin_ctzll(todo);
-        const int e0 = __builtin_amdgcn_readfirstlane(s_start[2 * k + 1]);  // chunk k + 3: keys 2 k + 1 .. 2 k + 7
-        const int e1 = __builtin_amdgcn_readfirstlane(s_start[2 * k + 6]);
-        const int e2 = __builtin_amdgcn_readfirstlane(s_start[2 * k + 8]);
-        const int pos4 = 4 * (k * kWave + kTickOff + lane);
-        StripeSums A;
-        stripe_run<false>(tnq, list, e0, e1, lane, pos4, A);
-        stripe_run<true>(tnq, list, e1, e2, lane, pos4, A);
-        const float a0 = (A.a0[0] + A.a0[1]) + (A.a0[2] + A.a0[3]), a1 = (A.a1[0] + A.a1[1]) + (A.a1[2] + A.a1[3]);
-        const int o = k * kWave + lane;
-        if (lane == 0) s_edge[k] += a1;
-        const float v = a0 + lane_next0(a1);
-        if (o < nout) acc[o] += v;
-      }
-      // pairs with non-finite factors, tick by tick (each tick has one owner in this loop)
-      const int x0 = s_start[kKeyOdd], x1 = s_start[kKeyNone];
-      if (x0 < x1) {
-        __syncthreads();
-        for (int x = x0; x < x1; ++x)
-          for (int o = t; o < nout; o += NT) {
-            const float v = odd_pair(tb.TNQ, list[x], o, L, nout);
-            if (o == 0) tick0 += v;
-            else acc[o] += v;
-          }
+  const int nsb = d.nsb, L = d.L, cm = d.cm, side = 2 * d.ne + 1, ws4 = 4 * bin_stride(L);
+  const bool holds = 3 * lane < L + 2;  // does the lane hold samples of a window
+  const int lane12 = holds ? 12 * lane : 0x7ffffff0;
+  const __amdgpu_buffer_rsrc_t tnp =
+      __builtin_amdgcn_make_buffer_rsrc((void*)tb.TNP, 0, d.lx * d.ly * kWinPad * 4, kBufDesc3);
+  const __amdgpu_buffer_rsrc_t tmw = __builtin_amdgcn_make_buffer_rsrc(
+      (void*)tb.TMW, 0, (int)(uint32_t)(bin_floats(d.nm, cm, L) * 4), kBufDesc3);
+  // The wave's blocks of 64 pairs: of the far and side cells' pairs, flattened, blocks wid, wid + WAVES, ..;
+  // then of the centre cell's segments wid, wid + WAVES, .. .
+  const int nfar = c_cum[nsc], nall = c_cum[nct];
+  const int nfb = (nfar - wid * kWave + WAVES * kWave - 1) / (WAVES * kWave);
+  const int ncb = (nall - nfar - wid + WAVES * kWave - 1) / (WAVES * kWave);
+  struct Pair {
+    PairRec P;
+    float D;      // boundary correction
+    int sg, ab;   // segment (-1: none), row offset
+  };
+  auto fetch = [&](int i, Pair& B) {
+    B = Pair{PairRec{0, 0.f, 0.f, 0}, 0.f, -1, 0};
+    int lo = nsc;
+    const int p = i < nfb ? (i * WAVES + wid) * kWave + lane : nfar + wid + WAVES * (kWave * (i - nfb) + lane);
+    if (i >= nfb + ncb || p >= (i < nfb ? nfar : nall)) return;
+    if (i < nfb) {
+      int hi = nsc - 1;  // the cell holding p: last c with c_cum[c] <= p
+      lo = 0;
+      while (lo < hi) {
+        const int mid = (lo + hi + 1) >> 1;
+        if (c_cum[mid] <= p) lo = mid;
+        else hi = mid - 1;
       }
     }
-    tick0 = wave_sum(tick0);
-    if (lane == 0) s_tick0[wid] = tick0;
-    __syncthreads();
-    // chunk edges, tick 0 and the other waves' rows
-    if (t >= 1 && t < nchunk && t * kWave - 1 < nout) acc[t * kWave - 1] += s_edge[t];
-    if (t == 0) {
-      float v = 0.f;
-      for (int w = 0; w < WAVES; ++w) v += s_tick0[w];
-      acc[0] = v;
-    }
-    for (int o = rstride + t; o < WAVES * rstride; o += NT) acc[o] = 0.f;
-    __syncthreads();
-  }
-  // Diffusion bins that land on this pixel: from every segment of the centre cell, and from those of the
-  // side cells near their pixel's edge.  Each wave takes every WAVES-th pair (the centre cell's pairs are most
-  // of the work), 64 at a time.  Lane by lane: does any bin land here, and the bins merged per LUT cell
-  // along each axis, staged in LDS for the wave, which then computes and stores one pair's window after
-  // the other.
-  {
-    const int p0 = c_cum[ncls[0]], p1 = c_cum[nct];
-    const int cm = d.cm, ws4 = 4 * bin_stride(L);
-    const float* dtc = dtot + (int64_t)(d.ne * (2 * d.ne + 1) + d.ne) * nseg;
-    const int lane12 = 3 * lane < L + 2 ? 12 * lane : 0x7ffffff0;
-    const __amdgpu_buffer_rsrc_t tmw = __builtin_amdgcn_make_buffer_rsrc(
-        (void*)tb.TMW, 0, (int)(uint32_t)(bin_floats(d.nm, cm, L) * 4), kBufDesc3);
-    for (int b0 = p0; b0 < p1; b0 += WAVES * kWave) {
-      const int p = b0 + lane * WAVES + wid;
-      bool on = false;
-      PairRec P;
-      int base = 0, cxs[NB], cys[NB];
-      float la = 0.f, lb = 0.f, lc = 0.f, delta = 0.f, WX[NB], WY[NB];
-      if (p < p1) {
-        int lo = ncls[0];  // at most 9 cells
-        while (c_cum[lo + 1] <= p) ++lo;
-        const int sg = c_beg[lo] + (p - c_cum[lo]);
-        const int ab = c_ab[lo];
-        const int a = (ab >> 8) - 64, b = (ab & 255) - 64;
-        P = prs[sg];
-        const int ux = (P.flags >> 8) & 255, uy = (P.flags >> 16) & 255;
-        on = P.ne != 0.f && bins_reach<NB>(ux, a, nsb) && bins_reach<NB>(uy, b, nsb);
-        if (on) {
-          const SegRec& R = rec[sg];
-          la = R.la;
-          lb = R.lb;
-          lc = R.lc;
-          base = (R.idx - 1) * ws4;
-          if (lo >= nsc) delta = P.ne * dtc[sg];  // (a side pair's correction went with its stripe)
-          bool ok[NB];
-          axis_merge<NB>(ux, a, nsb, R.wx, P.ne, ok, cxs, WX);
-          axis_merge<NB>(uy, b, nsb, R.wy, 1.f, ok, cys, WY);
-        }
+    B.sg = c_beg[lo] + (p - c_cum[lo]);
+    B.ab = c_ab[lo];
+    B.P = prs[B.sg];
+    B.D = dtot[(int64_t)(((B.ab >> 8) - 64 + d.ne) * side + ((B.ab & 255) - 64 + d.ne)) * nseg + B.sg];
+  };
+  Pair nxt;
+  fetch(0, nxt);
+  for (int i = 0; i < nfb + ncb; ++i) {
+    const Pair B = nxt;
+    fetch(i + 1, nxt);  // (its loads arrive while this block is worked on)
+    const PairRec P = B.P;
+    const int a = (B.ab >> 8) - 64, b = (B.ab & 255) - 64;
+    const int ux = (P.flags >> 8) & 255, uy = (P.flags >> 16) & 255;
+    const float omf = 1.f - P.f;
+    const float d1 = omf * B.D, d2 = P.f * B.D;
+    if (i < nfb) {
+      // stripes (with none, nn = 0, a side pixel gets the correction and its diffusion bins only)
+      const bool on = a >= -d.nn && a <= d.nn && b >= -d.nn && b <= d.nn;
+      const float st = on ? 1.f : 0.f;
+      float so = st * (P.ne * omf), sf = st * (P.ne * P.f);
+      const int row = on ? offset_bin(ux, a, nsb) * d.ly + offset_bin(uy, b, nsb) : 0;
+      const bool odd = B.sg >= 0 && !(fabsf(so) + fabsf(sf) < __builtin_inff());
+      int S = P.S, off = row * (kWinPad * 4);
+      float e1 = d1, e2 = d2;
+      if (B.sg < 0 || odd || P.ne == 0.f) {  // no pair: a window inside the row that adds nothing
+        S = 2;
+        off = 0;
+        so = sf = e1 = e2 = 0.f;
       }
-      for (uint64_t m = __ballot(on); m != 0;) {
-        const int rank = __popcll(m & ((1ull << lane) - 1));
-        if (((m >> lane) & 1) && rank < kBinItems) {
-          float* st = s_bins[wid][rank];
+      const int n = min(nfar - (i * WAVES + wid) * kWave, kWave);
+      const uint64_t edge = __ballot(S < 2 || S + L > nout);
+      if (holds) {
+        auto from = [](float v, int j) { return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), j)); };
+        for (int j = 0; j < n; j += kFarGroup) {
+          typedef float f32x3 __attribute__((ext_vector_type(3)));
+          f32x3 v[kFarGroup];
 #pragma unroll
-          for (int k = 0; k < NB; ++k) {
-            st[k] = WX[k];
-            st[NB + k] = WY[k];
-            st[2 * NB + k] = __int_as_float(cxs[k] * cm * d.nm * ws4);
-            st[3 * NB + k] = __int_as_float(cys[k] * d.nm * ws4);
+          for (int g = 0; g < kFarGroup; ++g)
+            v[g] = __builtin_bit_cast(
+                f32x3, __builtin_amdgcn_raw_buffer_load_b96(tnp, lane12, __builtin_amdgcn_readlane(off, j + g), 0));
+          if (((edge >> j) & ((1 << kFarGroup) - 1)) == 0) {
+#pragma unroll
+            for (int g = 0; g < kFarGroup; ++g)
+              store_window<true, false>(accw, lane, v[g][0], v[g][1], v[g][2], from(so, j + g), from(sf, j + g),
+                                        from(e1, j + g), from(e2, j + g), 0.f, __builtin_amdgcn_readlane(S, j + g), L, nout);
+            continue;
+          }
+#pragma unroll
+          for (int g = 0; g < kFarGroup; ++g) {
+            const float p = from(so, j + g), q = from(sf, j + g), c1 = from(e1, j + g), c2 = from(e2, j + g);
+            const int at = __builtin_amdgcn_readlane(S, j + g);
+            if ((edge >> (j + g)) & 1) store_window<false, false>(accw, lane, v[g][0], v[g][1], v[g][2], p, q, c1, c2, 0.f, at, L, nout);
+            else store_window<true, false>(accw, lane, v[g][0], v[g][1], v[g][2], p, q, c1, c2, 0.f, at, L, nout);
           }
         }
-        __builtin_amdgcn_wave_barrier();  // wave-local LDS: program order
-        for (int k = 0; k < kBinItems && m != 0; ++k) {
-          const int j = __builtin_ctzll(m);
-          m &= m - 1;
-          auto get = [&](float v) { return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), j)); };
-          const int S = __builtin_amdgcn_readlane(P.S, j);
-          const float f = get(P.f);
-          float v0, v1, v2;
-          bins_window<NB>(tmw, s_bins[wid][k], __builtin_amdgcn_readlane(base, j), ws4, lane, lane12, get(la), get(lb),
-                          get(lc), v0, v1, v2);
-          store_window(accw, lane, v0, v1, v2, 1.f - f, f, get(delta), S, L, nout, S >= 2 && S + L <= nout);
-        }
-        __builtin_amdgcn_wave_barrier();  // the stage is rewritten
       }
+      for (uint64_t m = __ballot(odd); m != 0; m &= m - 1) {
+        const int j = __builtin_ctzll(m);
+        const float* T = tb.TNP + (int64_t)__builtin_amdgcn_readlane(row, j) * kWinPad + 2;
+        const float q = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(st * (P.ne * omf)), j));
+        const float r = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(st * (P.ne * P.f)), j));
+        for (int o = lane; o < nout; o += kWave)
+          accw[o] += odd_pair(T, q, r, __builtin_amdgcn_readlane(P.S, j), o, L, nout);
+      }
+    }
+    // Diffusion bins that land on this pixel: of every segment of the centre cell, and of those of the side
+    // cells near their pixel's edge.  Lane by lane: does any bin land here, and the bins merged per LUT cell
+    // along each axis, staged in LDS for the wave, which then computes and stores one pair's window after
+    // the other.
+    const bool bins = B.sg >= 0 && a >= -1 && a <= 1 && b >= -1 && b <= 1 && P.ne != 0.f && bins_reach<NB>(ux, a, nsb) &&
+                      bins_reach<NB>(uy, b, nsb);
+    uint64_t m = __ballot(bins);
+    if (m == 0) continue;
+    bool ok[NB];
+    int base = 0, cxs[NB], cys[NB];
+    float la = 0.f, lb = 0.f, lc = 0.f, WX[NB], WY[NB];
+    if (bins) {
+      const SegRec& R = rec[B.sg];
+      la = R.la;
+      lb = R.lb;
+      lc = R.lc;
+      base = (R.idx - 1) * ws4;
+      axis_merge<NB>(ux, a, nsb, R.wx, P.ne, ok, cxs, WX);
+      axis_merge<NB>(uy, b, nsb, R.wy, 1.f, ok, cys, WY);
+    }
+    const float delta = i < nfb ? 0.f : B.D;  // (a side pair's correction went with its stripe)
+    while (m != 0) {
+      const int rank = __popcll(m & ((1ull << lane) - 1));
+      if (((m >> lane) & 1) && rank < kBinItems) {
+        int* stg = s_bins[wid][rank];
+#pragma unroll
+        for (int k = 0; k < NB; ++k) {
+          stg[k] = __float_as_int(WX[k]);
+          stg[NB + k] = __float_as_int(WY[k]);
+          stg[2 * NB + k] = cxs[k] * cm * d.nm * ws4;
+          stg[3 * NB + k] = cys[k] * d.nm * ws4;
+        }
+      }
+      __builtin_amdgcn_wave_barrier();  // wave-local LDS: program order
+      for (int k = 0; k < kBinItems && m != 0; ++k) {
+        const int j = __builtin_ctzll(m);
+        m &= m - 1;
+        auto get = [&](float v) { return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), j)); };
+        float v0, v1, v2;
+        bins_window<NB>(tmw, s_bins[wid][k], __builtin_amdgcn_readlane(base, j), ws4, lane, lane12, get(la), get(lb),
+                        get(lc), v0, v1, v2);
+        const float dl = get(delta), f = get(P.f);
+        const int S = __builtin_amdgcn_readlane(P.S, j);
+        if (holds) {
+          if (S >= 2 && S + L <= nout) store_window<true, true>(accw, lane, v0, v1, v2, 1.f - f, f, (1.f - f) * dl, f * dl, dl, S, L, nout);
+          else store_window<false, true>(accw, lane, v0, v1, v2, 1.f - f, f, (1.f - f) * dl, f * dl, dl, S, L, nout);
+        }
+      }
+      __builtin_amdgcn_wave_barrier();  // the stage is rewritten
     }
   }
   __syncthreads();
@@ -1515,20 +1349,6 @@ __global__ __launch_bounds__(256) void k_lut_tables(Dev d, const float* __restri
       c += (double)win[j];
       CT[sbase * (L + 1) + j + 1] = c;
     }
-  }
-}
-
-// The raw-response windows TN as TNQ (stripe_floats values).
-__global__ void k_lut_tnq(Dev d, const float* __restrict__ TN, float* __restrict__ TNQ) {
-  const int stride = stripe_stride(d.L);
-  const int64_t ns = (int64_t)d.lx * d.ly, total = stripe_floats(d.lx, d.ly, d.L);
-  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < total; i += (int64_t)gridDim.x * blockDim.x) {
-    const int64_t row = i / stride;
-    const int m = (int)(i - row * stride) - kStripeLead;
-    float v = 0.f;
-    if (row <= ns && m == -1) v = __uint_as_float(kStripeMark);
-    if (row < ns && m >= 0 && m < d.L) v = TN[row * d.L + m];
-    TNQ[i] = v;
   }
 }
 

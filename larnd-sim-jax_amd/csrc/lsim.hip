@@ -61,7 +61,6 @@ struct lsim_ctx {
   float* TM = nullptr;
   float* TN = nullptr;
   float* TNP = nullptr;
-  float* TNQ = nullptr;
   float* TMW = nullptr;
   float2* DM = nullptr;
   float2* DN = nullptr;
@@ -279,14 +278,13 @@ void free_tables(lsim_ctx* c) {
   (void)hipFree(c->TM);
   (void)hipFree(c->TN);
   (void)hipFree(c->TNP);
-  (void)hipFree(c->TNQ);
   (void)hipFree(c->TMW);
   (void)hipFree(c->DM);
   (void)hipFree(c->DN);
   (void)hipFree(c->DNS);
   (void)hipFree(c->CTM);
   (void)hipFree(c->CTN);
-  c->TM = c->TN = c->TNP = c->TNQ = c->TMW = nullptr;
+  c->TM = c->TN = c->TNP = c->TMW = nullptr;
   c->TM3 = nullptr;
   c->DM = c->DN = c->DNS = nullptr;
   c->CTM = c->CTN = nullptr;
@@ -401,7 +399,6 @@ int lsim_lut_set(lsim_ctx* c, const float* raw, int32_t nx, int32_t ny, int32_t 
         {(void**)&c->TM3, ms * kWinPad * sizeof(float3)}, {(void**)&c->TM, ms * L * sizeof(float)},
         {(void**)&c->TN, ns * L * sizeof(float)},         {(void**)&c->TNP, ns * kWinPad * sizeof(float)},
         {(void**)&c->TMW, (size_t)bin_floats(k.n_templates, c->cm, L) * sizeof(float)},
-        {(void**)&c->TNQ, (size_t)stripe_floats(nx, ny, L) * sizeof(float)},
         {(void**)&c->DM, ms * nt * sizeof(float2)},       {(void**)&c->DN, ns * nt * sizeof(float2)},
         {(void**)&c->DNS, nds * nt * sizeof(float2)},
         {(void**)&c->CTM, ms * (L + 1) * sizeof(double)}, {(void**)&c->CTN, ns * (L + 1) * sizeof(double)}};
@@ -418,7 +415,6 @@ int lsim_lut_set(lsim_ctx* c, const float* raw, int32_t nx, int32_t ny, int32_t 
   hipLaunchKernelGGL(k_lut_tables, dim3((unsigned)ns), dim3(256), 0, st, d, raw, 0, c->TN, c->TNP, c->DN, c->CTN);
   hipLaunchKernelGGL(k_lut_tm3, dim3(1024), dim3(256), 0, st, d, c->TM, c->TM3);
   hipLaunchKernelGGL(k_lut_tmw, dim3(1024), dim3(256), 0, st, d, c->TM, c->TMW, bin_floats(k.n_templates, c->cm, L));
-  hipLaunchKernelGGL(k_lut_tnq, dim3(1024), dim3(256), 0, st, d, c->TN, c->TNQ);
   hipLaunchKernelGGL(k_lut_dns, dim3(4096), dim3(256), 0, st, d, c->DN, c->DNS);
   const hipError_t e = hipGetLastError();
   if (e != hipSuccess) {
@@ -498,7 +494,7 @@ int lsim_forward_prepare(lsim_ctx* c, const lsim_params* p, const lsim_segments*
 
 static int forward_rows_impl(lsim_ctx* c, const Dev& d, const Ws& w, int64_t n_seg, int64_t max_rows,
                              const lsim_fwd_out* out, hipStream_t st) {
-  Tables tb{c->TM3, c->TM, c->TMW, c->TN, c->TNP, c->TNQ, c->DM, c->DN, c->CTM, c->CTN};
+  Tables tb{c->TM3, c->TM, c->TMW, c->TN, c->TNP, c->DM, c->DN, c->CTM, c->CTN};
   RowOut ro;
   ro.wfs = out->wfs;
   ro.adc = out->adc;
@@ -779,7 +775,7 @@ static int backward_impl(lsim_ctx* c, const lsim_params* p, const lsim_segments*
   double* dz = cv.take<double>(max_rows);
   double* partial = cv.take<double>(2 * max_rows * kNGrad);  // far pass rows, then near pass rows
   AdjRec* adj = cv.take<AdjRec>(n);
-  Tables tb{c->TM3, c->TM, c->TMW, c->TN, c->TNP, c->TNQ, c->DM, c->DN, c->CTM, c->CTN};
+  Tables tb{c->TM3, c->TM, c->TMW, c->TN, c->TNP, c->DM, c->DN, c->CTM, c->CTN};
   SegIn in = make_segin(seg);
   uint32_t *keys, *vals;
   sorted_buffers(w, d, keys, vals);
