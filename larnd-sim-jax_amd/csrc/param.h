@@ -252,8 +252,10 @@ __device__ __forceinline__ double lane_next_d(double v) {  // lane i receives la
 // other vector instructions a pair, 84 % of the cycles (erf, two erfc and two exponentials, each with its own
 // quotient, took 760; 50k-segment event, 4.1 M pairs, 81 pixels an electron: the whole call 5.59 -> 3.62 ms).
 // Two pairs at a time did not pay: their lane reads run out of scalar registers.
-// Lanes whose exponential leaves (or nears) the float64 range take emg_cdf_half itself, so that what
-// overflows there overflows here, to the same infinities and NaNs.
+// Lanes whose exponential leaves (or nears) the float64 range take emg_cdf_half itself (undoubled, as then are the
+// pair's other lanes), and a tail whose normaliser F_1 - F_{T-1} is not a number of ordinary size is taken by
+// quotients, so that what overflows there overflows here, to the same zeros, infinities and NaNs.  (The reciprocal of
+// an infinite normaliser by Newton steps is NaN, which makes NaN of the samples whose quotient is 0.)
 __device__ __forceinline__ double pair_sample(const PairCur& mine, int l, double gj, double dt, int T, bool diffusion) {
   if (!diffusion) {
     const double a = readlane_d(mine.a, l), loc = readlane_d(mine.loc, l);
@@ -280,14 +282,17 @@ __device__ __forceinline__ double pair_sample(const PairCur& mine, int l, double
   if (__builtin_amdgcn_ballot_w64(general)) {  // (wave uniform: the lane reads need every lane's registers)
     const double loc = readlane_d(mine.loc, l), sig = readlane_d(mine.sig, l);
     const double lb = 1.0 / readlane_d(mine.sb, l), lc = 1.0 / readlane_d(mine.sc, l);
-    const double Gb = 2.0 * emg_cdf_half(gj, loc, sig, lb), Gc = 2.0 * emg_cdf_half(gj, loc, sig, lc);
-    Fb = general ? Gb : Fb;
-    Fc = general ? Gc : Fc;
+    const double Gb = emg_cdf_half(gj, loc, sig, lb), Gc = emg_cdf_half(gj, loc, sig, lc);
+    Fb = general ? Gb : 0.5 * Fb;
+    Fc = general ? Gc : 0.5 * Fc;
   }
   const double db = readlane_d(Fb, 1) - readlane_d(Fb, T - 1), dc = readlane_d(Fc, 1) - readlane_d(Fc, T - 1);
-  double ib = rcp_nr(db), ic = rcp_nr(dc);
-  if (__builtin_amdgcn_readfirstlane(!(fmin(db, dc) > 1e-280))) ib = 1.0 / db, ic = 1.0 / dc;
-  return (Fb - lane_next_d(Fb)) * ib * readlane_d(mine.qb, l) + (Fc - lane_next_d(Fc)) * ic * readlane_d(mine.qc, l);
+  const double nb = Fb - lane_next_d(Fb), nc = Fc - lane_next_d(Fc);
+  const double qb = readlane_d(mine.qb, l), qc = readlane_d(mine.qc, l);
+  const bool usual = fmin(db, dc) > 1e-280 && db < 1e280 && dc < 1e280;
+  if (!__builtin_amdgcn_readfirstlane(usual)) return nb / db * qb + nc / dc * qc;
+  const double ib = rcp_nr(db), ic = rcp_nr(dc);
+  return nb * ib * qb + nc * ic * qc;
 }
 
 // One workgroup per row (sorted unique pixel id upix[r]): the pairs order[offs[r] .. offs[r+1]) in
