@@ -595,9 +595,13 @@ __global__ __launch_bounds__(WAVES * kWave) __attribute__((amdgpu_waves_per_eu(4
 //     the sums of G with T_m and with the differences dm = T_{m-1} - T_m, dp = T_{m+1} - T_m from the
 //     interleaved template windows of TM3: V = (la + lb + lc) T_m + la dm + lc dp for n_e, f, sigma_T, and
 //     dV/dlambda = da dm + dc dp for lambda (the three Lagrange derivatives sum to zero).
+// A window's products are formed and added in float64; only those with the templates' differences, which enter with
+// small weights (and alone in lambda's derivative), three at a time in float32 first.  Sums of twelve products in
+// float32 were less exact than a lane's three of a whole wave per window, and 436 us where these take 506 (50k-segment
+// step with a waveform loss; by threes throughout 480).
 // A whole wave per window spent its time on what it did once a window or cell in every lane (25 float64
-// instructions a cell, 7 a stripe, 16-byte reads of the stage) and on 4-byte loads: 796 -> 570 us for the
-// 50k-segment step with a waveform loss; one group of four windows in flight is enough (two 588, four 686 us).
+// instructions a cell, 7 a stripe, 16-byte reads of the stage) and on 4-byte loads: 796 us; several groups of four
+// windows in flight did not help.
 
 constexpr int kGOff = 192;                       // LDS index of output tick 0
 constexpr int kGLen = kMaxOut + 2 * kGOff + 64;  // ticks -kGOff .. kMaxOut + kGOff + 63
@@ -617,7 +621,6 @@ struct DenseCell {
   double w, dw;
   int cell, pad;
 };
-constexpr int kDensePairs = 1;  // groups of four pairs in flight
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 // G at a correction tick (those are kept for 0 <= o <= nout - 2); Gw holds 0 at tick 0 (a window
@@ -630,7 +633,7 @@ __device__ __forceinline__ double g_corr(const float* Gw, float G0, int o, int n
 __device__ __forceinline__ bool window_live(int S, int L, int nout) { return S >= 2 - L && S <= nout; }
 
 template <int NB, int WAVES>
-__global__ __launch_bounds__(WAVES * kWave) void k_rows_adj_dense(Dev d, Tables tb, const SegRec* __restrict__ rec,
+__global__ __launch_bounds__(WAVES * kWave) __attribute__((amdgpu_waves_per_eu(4))) void k_rows_adj_dense(Dev d, Tables tb, const SegRec* __restrict__ rec,
                                                                   const PairRec* __restrict__ prs,
                                                                   const AdjRec* __restrict__ adj,
                                                                   const int2* __restrict__ rng,
@@ -765,38 +768,31 @@ __global__ __launch_bounds__(WAVES * kWave) void k_rows_adj_dense(Dev d, Tables 
     stage[wid][lane] = z;
     __builtin_amdgcn_wave_barrier();
     const int n = __builtin_amdgcn_readfirstlane(nstripe - b0 < kWave ? nstripe - b0 : kWave);
-    for (int i = 0; i < n; i += 4 * kDensePairs) {
+    for (int i = 0; i < n; i += 4) {
       // four pairs at a time, 16 lanes each (entries past n are padding: factors 0, a window at S = 2)
-      f32x4 x[kDensePairs][3];
-      int S[kDensePairs];
+      const DenseStripe& q = stage[wid][i + grp];
+      f32x4 x[3];
 #pragma unroll
-      for (int h = 0; h < kDensePairs; ++h) {
-        const DenseStripe& q = stage[wid][i + 4 * h + grp];
-        S[h] = q.S;
-        const int off = q.off + sub * 16;
+      for (int c = 0; c < 3; ++c)
+        x[c] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(tnp, q.off + sub * 16, c * 4 * kWave, 0));
+      double u1 = 0.0, u0 = 0.0;
+      const float* gp = Gw + kGOff + q.S - 2 + 4 * sub;
 #pragma unroll
-        for (int c = 0; c < 3; ++c)
-          x[h][c] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(tnp, off, c * 4 * kWave, 0));
-      }
+      for (int c = 0; c < 3; ++c) {
+        double g0 = (double)gp[kWave * c - 1];
 #pragma unroll
-      for (int h = 0; h < kDensePairs; ++h) {
-        const DenseStripe& q = stage[wid][i + 4 * h + grp];
-        float u1 = 0.f, u0 = 0.f;
-#pragma unroll
-        for (int c = 0; c < 3; ++c) {
-          const float* gp = Gw + kGOff + S[h] - 2 + 4 * sub + kWave * c;
-#pragma unroll
-          for (int k = 0; k < 4; ++k) {
-            u1 = __builtin_fmaf(gp[k], x[h][c][k], u1);
-            u0 = __builtin_fmaf(gp[k - 1], x[h][c][k], u0);
-          }
+        for (int k = 0; k < 4; ++k) {
+          const double g1 = (double)gp[kWave * c + k], xk = (double)x[c][k];
+          u1 = __builtin_fma(g1, xk, u1);
+          u0 = __builtin_fma(g0, xk, u0);
+          g0 = g1;
         }
-        const double aa = (double)(q.c1 * u1 + q.c0 * u0), bb = (double)(q.ne * (u0 - u1));
-        g[0] += q.fN[0] * aa;
-        g[1] += q.fN[1] * aa;
-        g[2] += q.fN[2] * aa + q.fF * bb;
-        g[3] += q.fN[3] * aa;
       }
+      const double aa = (double)q.c1 * u1 + (double)q.c0 * u0, bb = (double)q.ne * (u0 - u1);
+      g[0] += q.fN[0] * aa;
+      g[1] += q.fN[1] * aa;
+      g[2] += q.fN[2] * aa + q.fF * bb;
+      g[3] += q.fN[3] * aa;
     }
     __builtin_amdgcn_wave_barrier();  // the stage is rewritten by the next block
   }
@@ -870,8 +866,8 @@ __global__ __launch_bounds__(WAVES * kWave) void k_rows_adj_dense(Dev d, Tables 
       for (int c = 0; c < 3; ++c)
 #pragma unroll
         for (int k = 0; k < 5; ++k) gv[c][k] = Gw[kGOff + S - 3 + 4 * sub + kWave * c + k];
-      const float la = R.la, lc = R.lc, ls = R.la + R.lb + R.lc;
-      const float da = (float)A->dl[0], dc = (float)A->dl[2];
+      const double la = (double)R.la, lc = (double)R.lc, ls = la + (double)R.lb + lc;
+      const double da = A->dl[0], dc = A->dl[2];
       double U1 = 0.0, U0 = 0.0, D1 = 0.0, D0 = 0.0, L1 = 0.0, L0 = 0.0;
       for (int k4 = 0; k4 < nc; k4 += 4) {
         const DenseCell q = cells[k4 + grp];
@@ -882,29 +878,36 @@ __global__ __launch_bounds__(WAVES * kWave) void k_rows_adj_dense(Dev d, Tables 
 #pragma unroll
           for (int k = 0; k < 3; ++k) v[c][k] = T[c * (3 * kWave / 4) + k];
         // sums of G and of G one tick on with T_m and its differences from T_{m-1}, T_{m+1}
-        float y1 = 0.f, y0 = 0.f, p1 = 0.f, p0 = 0.f, n1 = 0.f, n0 = 0.f;
+        double y1 = 0.0, y0 = 0.0, p1 = 0.0, p0 = 0.0, n1 = 0.0, n0 = 0.0;
 #pragma unroll
-        for (int c = 0; c < 3; ++c) {
+        for (int k = 0; k < 4; ++k) {
+          float a1 = 0.f, a0 = 0.f, b1 = 0.f, b0 = 0.f;
 #pragma unroll
-          for (int k = 0; k < 4; ++k) {
+          for (int c = 0; c < 3; ++c) {
             const float tm = v[c][(3 * k) / 4][(3 * k) % 4], tc = v[c][(3 * k + 1) / 4][(3 * k + 1) % 4],
                         tp = v[c][(3 * k + 2) / 4][(3 * k + 2) % 4];
             const float dm = tm - tc, dp = tp - tc;
-            y1 = __builtin_fmaf(gv[c][k + 1], tc, y1);
-            y0 = __builtin_fmaf(gv[c][k], tc, y0);
-            p1 = __builtin_fmaf(gv[c][k + 1], dm, p1);
-            p0 = __builtin_fmaf(gv[c][k], dm, p0);
-            n1 = __builtin_fmaf(gv[c][k + 1], dp, n1);
-            n0 = __builtin_fmaf(gv[c][k], dp, n0);
+            float g1 = gv[c][k + 1], g0 = gv[c][k];
+            asm volatile("" : "+v"(g1), "+v"(g0));  // converted here: kept in float64 over the loop they take 30 registers
+            y1 = __builtin_fma((double)g1, (double)tc, y1);
+            y0 = __builtin_fma((double)g0, (double)tc, y0);
+            a1 = __builtin_fmaf(g1, dm, a1);
+            a0 = __builtin_fmaf(g0, dm, a0);
+            b1 = __builtin_fmaf(g1, dp, b1);
+            b0 = __builtin_fmaf(g0, dp, b0);
           }
+          p1 += (double)a1;
+          p0 += (double)a0;
+          n1 += (double)b1;
+          n0 += (double)b0;
         }
-        const double u1 = (double)(ls * y1 + la * p1 + lc * n1), u0 = (double)(ls * y0 + la * p0 + lc * n0);
+        const double u1 = ls * y1 + la * p1 + lc * n1, u0 = ls * y0 + la * p0 + lc * n0;
         U1 += q.w * u1;
         U0 += q.w * u0;
         D1 += q.dw * u1;
         D0 += q.dw * u0;
-        L1 += q.w * (double)(da * p1 + dc * n1);
-        L0 += q.w * (double)(da * p0 + dc * n0);
+        L1 += q.w * (da * p1 + dc * n1);
+        L0 += q.w * (da * p0 + dc * n0);
       }
       __builtin_amdgcn_wave_barrier();  // the slots are rewritten by the next item
       gN += (1.0 - f) * U1 + f * U0;
