@@ -509,7 +509,7 @@ __global__ __launch_bounds__(WAVES * kWave) __attribute__((amdgpu_waves_per_eu(4
     // stripes, one item a pair.  Each thread fetches its next pair's record (the first 16 bytes
     // of the pair record) and chain factors while the current pair's table loads are in flight.
     struct FarItem {
-      int4 P;  // S, ne, f, flags
+      int4 P;  // S, ne, f, uv
       double fN0, fN1, fN2, fN3, fF;
       int ab;
     };
@@ -534,7 +534,7 @@ __global__ __launch_bounds__(WAVES * kWave) __attribute__((amdgpu_waves_per_eu(4
         PairCtx pc;
         pair_ctx(d, x.P.x, ne, __int_as_float(x.P.z), G, pc);
         double gN = 0.0, gF = 0.0;
-        stripe_adjoint(d, tb, (x.P.w >> 8) & 255, (x.P.w >> 16) & 255, pc, (x.ab >> 8) - 64, (x.ab & 255) - 64, G, gN,
+        stripe_adjoint(d, tb, x.P.w & 0xffff, (int)((uint32_t)x.P.w >> 16), pc, (x.ab >> 8) - 64, (x.ab & 255) - 64, G, gN,
                        gF);
         g[0] += gN * x.fN0;
         g[1] += gN * x.fN1;
@@ -550,8 +550,8 @@ __global__ __launch_bounds__(WAVES * kWave) __attribute__((amdgpu_waves_per_eu(4
     while (i >= c_cum[cur + 1]) ++cur;
     const int s = c_beg[cur] + (i - c_cum[cur]);
     const int a = (c_ab[cur] >> 8) - 64, b = (c_ab[cur] & 255) - 64;
-    const int uv = prs[s].flags;
-    if (!bins_reach<NB>((uv >> 8) & 255, a, d.nsb) || !bins_reach<NB>((uv >> 16) & 255, b, d.nsb)) continue;
+    const int uv = prs[s].uv;
+    if (!bins_reach<NB>(uv & 0xffff, a, d.nsb) || !bins_reach<NB>((int)((uint32_t)uv >> 16), b, d.nsb)) continue;
     const SegRec R = rec[s];
     if (R.ne == 0.f) continue;
     const int S = d.nt - d.L - R.k0;
@@ -737,7 +737,7 @@ __global__ __launch_bounds__(WAVES * kWave) __attribute__((amdgpu_waves_per_eu(4
       if (R.ne != 0.f) {
         const int S = R.S;
         const double f = (double)R.f, ne = (double)R.ne;
-        const int ux = (R.flags >> 8) & 255, uy = (R.flags >> 16) & 255;
+        const int ux = R.u(), uy = R.v();
         const int sidx = offset_bin(ux, a, nsb) * d.ly + offset_bin(uy, b, nsb);
         const float2 D = tb.DN[(int64_t)(d.nt - L - S) * lxly + sidx];  // tick-major, k0 = nt - L - S
         const double corr = (double)D.x - f * (double)D.y, dy = (double)D.y;

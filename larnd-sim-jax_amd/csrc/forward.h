@@ -17,7 +17,9 @@ constexpr int kXcd = 8;  // XCDs of an MI355X (workgroup i runs on XCD i % 8)
 struct __align__(16) PairRec {
   int S;          // first output tick of the (1-f) window: nt - L - k0
   float ne, f;
-  int flags;      // bit 0: 2 <= S and S + L <= nout (interior window); bits 8-15: u; bits 16-23: v
+  int uv;         // u | v << 16, sixteen bits each as in SegRec
+  __device__ __forceinline__ int u() const { return uv & 0xffff; }
+  __device__ __forceinline__ int v() const { return (int)((uint32_t)uv >> 16); }
 };
 static_assert(sizeof(PairRec) == 16, "PairRec layout");
 
@@ -236,7 +238,7 @@ __device__ __forceinline__ void record(const Dev& d, const SegIn& in, int64_t sr
   P.S = d.nt - d.L - ph.k0;
   P.ne = r.ne;
   P.f = r.f;
-  P.flags = ((P.S >= 2 && P.S + d.L <= d.nout) ? 1 : 0) | (ux << 8) | (uy << 16);
+  P.uv = r.uxy;
   prs[i] = P;
 }
 
@@ -1013,7 +1015,7 @@ __global__ __launch_bounds__(WAVES * kWave) __attribute__((amdgpu_waves_per_eu(4
     fetch(i + 1, nxt);  // (its loads arrive while this block is worked on)
     const PairRec P = B.P;
     const int a = (B.ab >> 8) - 64, b = (B.ab & 255) - 64;
-    const int ux = (P.flags >> 8) & 255, uy = (P.flags >> 16) & 255;
+    const int ux = P.u(), uy = P.v();
     const float omf = 1.f - P.f;
     const float d1 = omf * B.D, d2 = P.f * B.D;
     if (i < nfb) {
