@@ -696,8 +696,7 @@ def main():
     ap.add_argument("--warmup", type=int, default=3)
     ap.add_argument("--waves", type=int, default=0, help="waves per row workgroup (0 = autotune)")
     ap.add_argument("--row-tile", type=int, default=16, help="accepted without effect")
-    ap.add_argument("--row-cost", type=int, default=256,
-                    help="accepted without effect")
+    ap.add_argument("--row-cost", type=int, default=256, help="accepted without effect")
     ap.add_argument("--no-cpu", action="store_true")
     ap.add_argument("--no-bwd", action="store_true")
     ap.add_argument("--no-batched-bwd", action="store_true", help="skip the batched forward+backward of 32 events")
@@ -793,8 +792,6 @@ def main():
         brun = S.Runner(simr, params, torch.from_numpy(bt).to(dev), bf, n_events=128, want_wfs=True)
         if a.waves:
             S.set_row_waves(a.waves)
-            S.set_row_cost(a.row_cost)
-            S.set_row_tile(a.row_tile)
         for i in range(a.steps):
             brun.forward()
             torch.cuda.synchronize()
@@ -813,13 +810,10 @@ def main():
         log(f"[bench] N={NB} rows={PB}")
         if a.waves:
             S.set_row_waves(a.waves)
-            S.set_row_cost(a.row_cost)
-            S.set_row_tile(a.row_tile)
-            waves, row_cost, row_tile, tune = a.waves, a.row_cost, a.row_tile, {}
+            waves, tune = a.waves, {}
         else:
-            waves, row_cost, row_tile, tune = S.autotune_rows(brun)
-        log(f"[bench] waves per row workgroup: {waves}, row cost {row_cost} pairs, row tile {row_tile} "
-            f"(tuning ms: {tune})")
+            waves, tune = S.autotune_row_waves(brun)
+        log(f"[bench] waves per row workgroup: {waves} (tuning ms: {tune})")
         g = torch.cuda.CUDAGraph()
         s = torch.cuda.Stream()
         s.wait_stream(torch.cuda.current_stream())
@@ -856,12 +850,9 @@ def main():
     extra = {}
     if a.single_only and a.waves:
         S.set_row_waves(a.waves)
-        S.set_row_cost(a.row_cost)
-        S.set_row_tile(a.row_tile)
     if a.headline_only:
         print(json.dumps({"metric": "segments/s", "value": seg_s, "ms_per_step": ms_step, "kernel_ms": k_avg,
-                          "achieved_gbs": achieved, "config": {"segments": NB, "pixel_rows": PB, "row_waves": waves,
-                                                                "row_cost": row_cost, "row_tile": row_tile}}),
+                          "achieved_gbs": achieved, "config": {"segments": NB, "pixel_rows": PB, "row_waves": waves}}),
               flush=True)
         return
     # ---- the 200k-segment event alone ----
@@ -1176,8 +1167,8 @@ def main():
         "config": {"workload": "batched forward: 128 events with log-uniform 2k-400k segments (seed 3), one "
                                "hipGraph replay per step, module0 geometry, 45x45x1950 LUT, 4 neighbour pixels, "
                                "5x5 diffusion bins, noise off",
-                   "segments": NB, "events": 128, "pixel_rows": PB, "row_waves": waves, "row_cost": row_cost,
-                   "row_tile": row_tile, "tuning_ms": tune},
+                   "segments": NB, "events": 128, "pixel_rows": PB, "row_waves": waves,
+                   "tuning_ms": tune},
         "roofline": {"bound": "hbm", "kernel": "k_rows_fwd", "achieved": achieved, "peak": HBM_PEAK_GBS,
                      "unit": "GB/s", "frac": achieved / HBM_PEAK_GBS, "traffic": traffic,
                      "traffic_stamp": stamp, "algorithmic_bytes": bytes_fwd, "kernel_ms": k_avg,

@@ -574,9 +574,9 @@ def autotune_row_waves(runner: Runner, candidates=(1, 2, 4, 8), reps=3):
 
 def autotune_rows(runner: Runner, waves=(1, 2, 4, 8), costs=(64, 256, 1024), tiles=(8, 16, 32), reps=3):
     """Tune the waveform kernel on the runner's workload: the waves per row workgroup, which change only
-    the schedule and the per-wave partial sums; the setting stays in effect.  ``costs`` and ``tiles``
-    belong to settings without effect, which are left at their defaults.  Returns (waves, row cost, tile,
-    {setting: kernel ms})."""
+    the schedule and the per-wave partial sums; the setting stays in effect.  ``costs`` and ``tiles`` are
+    accepted without effect (no such setting is tuned any more), and the second and third value returned
+    are the constants 256 and 16.  Returns (waves, 256, 16, {setting: kernel ms})."""
     set_row_cost(256)
     set_row_tile(16)
     w, res = autotune_row_waves(runner, waves, reps)
