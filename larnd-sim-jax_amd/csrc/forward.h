@@ -603,7 +603,9 @@ __device__ __forceinline__ void store_window(float* accw, int lane, float v0, fl
 // 0x00020000: word 3 of a raw (stride 0) buffer descriptor on gfx9-family GPUs.
 constexpr int kBufDesc3 = 0x00020000;
 
-constexpr int kFarGroup = 8;  // pairs whose windows a wave has in flight (128 events of 72k segments: 4 56.9, 8 55.3, 16 54.6 ms)
+// pairs whose windows a wave has in flight (128 events of 72k segments: 4 56.9, 8 55.3, 16 54.6 ms; 200k segments 8
+// and 16 alike, and a row's last block is padded to a whole group)
+constexpr int kFarGroup = 8;
 
 // A pair with a non-finite factor (window T) at output tick o: what storing its whole padded window leaves there
 // (a non-finite charge times the padding's zeros is NaN from S - 2 to S + 186 of an interior window).
@@ -897,7 +899,8 @@ __device__ __forceinline__ void list_cells_fwd(const Dev& d, const int2* __restr
 // and of the empty parts of an event.  One contiguous band an XCD, cut at equal shares of the estimated work
 // in an order by cell tiles, with the last quarter of the rows handed out by counters, balanced worse: 200k
 // segments 1.52 -> 1.21 ms, 128 events of 72k segments 52.5 -> 50.5 ms, and the adjoint's equal row counts an
-// XCD 720 -> 575 us (near), 420 -> 319 (far), 570 -> 430 (waveforms).  Runs of 4 to 64 are within 3 %.
+// XCD 720 -> 575 us (near), 420 -> 319 (far), 570 -> 430 (waveforms).  Runs of 4 to 64 are within 3 %.  (Each
+// pair of figures on the row kernels of the time; they take 1.32 and 55.3 ms, 414, 352 and 506 us as they are now.)
 constexpr int kRowRun = 16;
 
 __device__ __forceinline__ int64_t run_row() {  // of this workgroup; at or past the number of rows: none
